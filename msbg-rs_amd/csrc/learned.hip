@@ -19,6 +19,7 @@
 // chain of 14 tap pairs (K = 16 input channels x 2 taps), the input planes
 // staged in LDS.  The weight gradient is a second GEMM with K running over
 // cells.
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -253,80 +254,227 @@ __global__ void prep_wb_kernel(const float *__restrict__ params, u4v *wb, u4v *w
     wbf[i] = vb;
 }
 
+// ---------------------------------------------------------------------------
+// Weight gradients: dW[t][c][o] = sum over the cells p of X[p + off + d_t][c]
+// G[p][o], a GEMM with K running over cells (16x16x32 BF16 MFMA, N = o).  Both
+// operands need 8 cells of one channel per lane, and the tensors are
+// channels-last, so a work-group stages a slab of z-planes of one tile in LDS
+// channel-major (two x-neighbours packed per 32-bit word on the way in); K
+// then runs along x in groups of 8 cells, one aligned 16-byte LDS read per
+// operand.  The reads of single 2-byte values from global memory that this
+// replaces bound the layer: 64 tiles took 499 us for a 16-channel layer and
+// 288 us for the 2-channel one, plus 267 us a layer for one thread's serial
+// sum over 1,024 partials.  Now 256 partials a layer at most (a work-group
+// walks further tiles with its sums in registers), added by 8 waves per 64
+// parameters in a fixed order.
+// ---------------------------------------------------------------------------
+constexpr int kWgTiles = 64;  // tile groups: 64 x 4 slabs = one 16-channel work-group per CU
+constexpr int kWg16Slabs = 4, kWg16Waves = 9;          // 4 output planes each; one wave per (dy, dz)
+constexpr int kWg2Planes = 3, kWg2Slabs = 6, kWg2Waves = 10;  // 3 of 18 output planes each
+constexpr int kLP2 = 27 * 2 * 16 + 16;                 // partial of the 2-channel layer: W[27][2][16], bias[16]
+// LDS, in 32-bit words (2 cells): X[16][6][18][24], G[16][4][16][16]; the
+// channel strides are odd multiples of 16 bytes, so the 16 channels a wave
+// reads side by side fall on different banks.
+constexpr int kX16C = 6 * 18 * 12 + 4, kG16C = 4 * 16 * 8 + 4;
+constexpr int kWg16Lds = 16 * (kX16C + kG16C) * 4;
+// 2-channel layer: V[c][dx][5][20][24] with V[c][dx][..][x] = X[..][x + dx][c], G[16][3][18][24]
+constexpr int kV2C = 5 * 20 * 12 + 4, kG2C = 3 * 18 * 12 + 4;
+constexpr int kWg2Lds = (6 * kV2C + 16 * kG2C) * 4;
+
 struct WgArgs {
     const uint16_t *X;
     const int32_t *idx;
-    int sin, sout, off;
+    int sin, off;
     const uint16_t *G;  // [tile][sout^3][16]
-    int chunks;         // waves per tile
-    int gpc;            // 16-cell groups per wave
-    int n_tiles;
-    float *part;        // [wave][kLP]
+    int n_tiles, groups;  // work-group (group g, slab) takes tiles g, g + groups, ...
+    float *part;        // [work-group][kLP] (16 channels), [2 work-group][kLP2] (2 channels)
 };
 
-// Weight / bias gradient partials of one layer: wave (tile, chunk) sums over
-// its cells dW[t][c][o] += X[p + off + d_t][c] G[p][o] (MFMA 16x16x16 with
-// M = c, N = o, K = 16 cells: A[m][k] from lane m + 16 (k / 4), B[k][n] from
-// lane n + 16 (k / 4), D[m][n] in element m % 4 of lane n + 16 (m / 4)) and
-// db[o] += G[p][o].
-template <int CIN>
-__global__ __launch_bounds__(256) void wgrad_kernel(WgArgs a) {
-    const int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    const int tile = wave / a.chunks, chunk = wave - tile * a.chunks;
-    if (tile >= a.n_tiles) return;
-    const int ncell = a.sout * a.sout * a.sout;
-    const int groups = (ncell + 15) / 16;
-    const int m = lane & 15, kg = lane >> 4;
-    const int64_t xbase = (int64_t)(a.idx ? a.idx[tile] : tile) * a.sin * a.sin * a.sin;
-    f4 acc[27];
-    for (int t = 0; t < 27; ++t) acc[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-    float bsum = 0.0f;
-    const int g0 = chunk * a.gpc, g1 = min(groups, g0 + a.gpc);
-    for (int g = g0; g < g1; ++g) {
-        s4 bv;
-        int cx[4], cy[4], cz[4];
-        bool cvalid[4];
-        for (int i = 0; i < 4; ++i) {
-            const int c = g * 16 + 4 * kg + i;
-            cvalid[i] = c < ncell;
-            const int cc = cvalid[i] ? c : 0;
-            cx[i] = cc % a.sout;
-            cy[i] = (cc / a.sout) % a.sout;
-            cz[i] = cc / (a.sout * a.sout);
-            const uint16_t gv = cvalid[i] ? a.G[((int64_t)tile * ncell + c) * 16 + m] : (uint16_t)0;
-            bv[i] = (short)gv;
-            bsum += from_bf16(gv);
-        }
-        for (int t = 0; t < 27; ++t) {
-            s4 av = {0, 0, 0, 0};
-            if (m < CIN) {
-                for (int i = 0; i < 4; ++i) {
-                    const int ix = cx[i] + a.off + t % 3, iy = cy[i] + a.off + (t / 3) % 3,
-                              iz = cz[i] + a.off + t / 9;
-                    if (cvalid[i] && (unsigned)ix < (unsigned)a.sin && (unsigned)iy < (unsigned)a.sin &&
-                        (unsigned)iz < (unsigned)a.sin)
-                        av[i] = (short)a.X[(xbase + ((int64_t)iz * a.sin + iy) * a.sin + ix) * CIN + m];
-                }
-            }
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc[t], 0, 0, 0);
-        }
+// Channel pairs of two x-neighbours (8 channels each) as 8 words, one per
+// channel: low half the left cell.
+__device__ __forceinline__ void pack_cells(const u4v &l, const u4v &r, uint32_t *w) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        w[2 * i] = (l[i] & 0xffffu) | (r[i] << 16);
+        w[2 * i + 1] = (l[i] >> 16) | (r[i] & 0xffff0000u);
     }
-    float *P = a.part + (int64_t)wave * kLP;
-    for (int t = 0; t < 27; ++t)
-        for (int j = 0; j < 4; ++j) P[(t * 16 + 4 * kg + j) * 16 + m] = acc[t][j];
-    bsum += __shfl_xor(bsum, 16);
-    bsum += __shfl_xor(bsum, 32);
-    if (kg == 0) P[kTap + m] = bsum;
 }
 
-// grad[k] = sum over the n partials in order (deterministic).
-__global__ void reduce_partials_kernel(const float *__restrict__ part, int n, float *grad) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= kLP) return;
-    float s = 0.0f;
-    for (int w = 0; w < n; ++w) s += part[(int64_t)w * kLP + k];
-    grad[k] = s;
+__device__ __forceinline__ f4 mfma32(const u4v &a, const u4v &b, const f4 &c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, b), c, 0, 0, 0);
+}
+
+// 16 -> 16 channels, 16^3 output cells.  Wave v takes the taps (dx, dy = v %
+// 3, dz = v / 3), dx = 0..2: one 20-byte window of cells x .. x + 9 per group
+// gives the three A operands (words 0..3, the words shifted by one cell,
+// words 1..4), so the 27 taps cost 9 window reads.  Lane (m, kg) of a step
+// holds channel m (A: input, B: output) of the 8 cells of group 4 step + kg:
+// plane group >> 5, row (group >> 1) & 15, x = 8 (group & 1).
+__global__ __launch_bounds__(kWg16Waves * 64) void wgrad16_kernel(WgArgs a) {
+    extern __shared__ u4v lds[];
+    uint32_t *Xs = reinterpret_cast<uint32_t *>(lds), *Gs = Xs + 16 * kX16C;
+    constexpr int NT = kWg16Waves * 64;
+    const int slab = blockIdx.x % kWg16Slabs, group = blockIdx.x / kWg16Slabs;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int m = lane & 15, kg = lane >> 4, dy = wave % 3, dz = wave / 3;
+    const u4v ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+    f4 acc[3], bsum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) acc[d] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int tile = group; tile < a.n_tiles; tile += a.groups) {
+        const int sin = a.sin;
+        const int64_t tin = (int64_t)(a.idx ? a.idx[tile] : tile) * sin * sin * sin;
+        const u4v *X = reinterpret_cast<const u4v *>(a.X) + tin * 2;
+        const u4v *G = reinterpret_cast<const u4v *>(a.G) + ((int64_t)tile * 4096 + slab * 1024) * 2;
+        if (tile != group) __syncthreads();  // the last tile's reads are done
+        // X planes 4 slab + off .. + 5, rows and columns off .. off + 17, zero outside the input
+        for (int i = threadIdx.x; i < 6 * 18 * 9 * 2; i += NT) {
+            const int half = i & 1, c = i >> 1, p = c % 9, r = c / 9, y = r % 18, z = r / 18;
+            const int iz = 4 * slab + a.off + z, iy = a.off + y, ix = a.off + 2 * p;
+            const bool row = (unsigned)iz < (unsigned)sin && (unsigned)iy < (unsigned)sin;
+            const int64_t g = ((int64_t)iz * sin + iy) * sin + ix;
+            u4v l = {0u, 0u, 0u, 0u}, q = {0u, 0u, 0u, 0u};
+            if (row && (unsigned)ix < (unsigned)sin) l = X[g * 2 + half];
+            if (row && (unsigned)(ix + 1) < (unsigned)sin) q = X[g * 2 + 2 + half];
+            uint32_t w[8];
+            pack_cells(l, q, w);
+            uint32_t *d = Xs + half * 8 * kX16C + r * 12 + p;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) d[j * kX16C] = w[j];
+        }
+        for (int i = threadIdx.x; i < 512 * 2; i += NT) {  // 512 cell pairs of the slab's 4 planes
+            const int half = i & 1, p = i >> 1;
+            uint32_t w[8];
+            pack_cells(G[p * 4 + half], G[p * 4 + 2 + half], w);
+            uint32_t *d = Gs + half * 8 * kG16C + p;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) d[j * kG16C] = w[j];
+        }
+        __syncthreads();
+        const uint32_t *xr = Xs + m * kX16C + (dz * 18 + dy) * 12, *gr = Gs + m * kG16C;
+#pragma unroll 4
+        for (int st = 0; st < 32; ++st) {
+            const int g = 4 * st + kg, z = g >> 5, y = (g >> 1) & 15, xh = (g & 1) * 4;
+            const uint32_t *xp = xr + (z * 18 + y) * 12 + xh;
+            const u4v w = *reinterpret_cast<const u4v *>(xp), b = *reinterpret_cast<const u4v *>(gr + g * 4);
+            const uint32_t w4 = xp[4];
+            const u4v s1 = {__builtin_amdgcn_alignbit(w[1], w[0], 16), __builtin_amdgcn_alignbit(w[2], w[1], 16),
+                            __builtin_amdgcn_alignbit(w[3], w[2], 16), __builtin_amdgcn_alignbit(w4, w[3], 16)};
+            const u4v s2 = {w[1], w[2], w[3], w4};
+            acc[0] = mfma32(w, b, acc[0]);
+            acc[1] = mfma32(s1, b, acc[1]);
+            acc[2] = mfma32(s2, b, acc[2]);
+            if (wave == 0) bsum = mfma32(ones, b, bsum);  // every row: the sum of G over the cells
+        }
+    }
+    float *P = a.part + (int64_t)blockIdx.x * kLP;
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) P[((9 * dz + 3 * dy + d) * 16 + 4 * kg + j) * 16 + m] = acc[d][j];
+    if (wave == 0 && kg == 0) P[kTap + m] = bsum[0];
+}
+
+// 2 -> 16 channels, 18^3 output cells.  The 16 rows of an MFMA hold two (dy,
+// dz) pairs x 3 dx x 2 channels: 5 MFMAs (waves) cover the 27 taps, each lane
+// reading its own dx-shifted copy, and two sets of waves halve the steps.  A
+// row of 18 cells is three groups of 8; the cells past its end are zero in
+// both operands.
+__global__ __launch_bounds__(kWg2Waves * 64) void wgrad2_kernel(WgArgs a) {
+    extern __shared__ u4v lds[];
+    uint32_t *Vs = reinterpret_cast<uint32_t *>(lds), *Gs = Vs + 6 * kV2C;
+    constexpr int NT = kWg2Waves * 64, NG = kWg2Planes * 18 * 3, NS = (NG + 7) / 8;  // NS steps of 4 groups per wave set
+    const int slab = blockIdx.x % kWg2Slabs, group = blockIdx.x / kWg2Slabs;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, set = wave / 5, j5 = wave % 5;
+    const int m = lane & 15, kg = lane >> 4;
+    // row m: channel m & 1, dx (m >> 1) & 3 (3: unused), pair 2 j5 + (m >> 3) (9: unused)
+    const int pair = 2 * j5 + (m >> 3), dx = (m >> 1) & 3;
+    const int pr = pair < 9 ? pair : 0, vr = (m & 1) * 3 + (dx < 3 ? dx : 0);
+    const u4v ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+    f4 acc = {0.0f, 0.0f, 0.0f, 0.0f}, bsum = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int tile = group; tile < a.n_tiles; tile += a.groups) {
+        const int64_t tin = (int64_t)(a.idx ? a.idx[tile] : tile) * 8000;
+        const uint32_t *X = reinterpret_cast<const uint32_t *>(a.X) + tin + slab * kWg2Planes * 400;
+        const u4v *G = reinterpret_cast<const u4v *>(a.G) + ((int64_t)tile * 5832 + slab * kWg2Planes * 324) * 2;
+        if (tile != group) __syncthreads();
+        for (int i = threadIdx.x; i < 5 * 20 * 12; i += NT) {  // a pair of x positions: both channels, three dx
+            const int p = i % 12, r = i / 12;
+            uint32_t c[4];  // input cells 2 p .. 2 p + 3 of the row (positions 18 .. 23 of every copy are zero)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) c[j] = p < 9 && 2 * p + j < 20 ? X[r * 20 + 2 * p + j] : 0u;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                Vs[d * kV2C + i] = (c[d] & 0xffffu) | (c[d + 1] << 16);
+                Vs[(3 + d) * kV2C + i] = (c[d] >> 16) | (c[d + 1] & 0xffff0000u);
+            }
+        }
+        for (int i = threadIdx.x; i < kWg2Planes * 18 * 12 * 2; i += NT) {
+            const int half = i & 1, c = i >> 1, p = c % 12, r = c / 12;
+            u4v l = {0u, 0u, 0u, 0u}, q = {0u, 0u, 0u, 0u};
+            if (p < 9) {
+                l = G[(r * 18 + 2 * p) * 2 + half];
+                q = G[(r * 18 + 2 * p + 1) * 2 + half];
+            }
+            uint32_t w[8];
+            pack_cells(l, q, w);
+            uint32_t *d = Gs + half * 8 * kG2C + c;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) d[j * kG2C] = w[j];
+        }
+        __syncthreads();
+        const uint32_t *xr = Vs + vr * kV2C + ((pr / 3) * 20 + pr % 3) * 12, *gr = Gs + m * kG2C;
+#pragma unroll 3
+        for (int st = 0; st < NS; ++st) {
+            const int g = 8 * st + 4 * set + kg;
+            const bool in = g < NG;
+            const int gg = in ? g : 0, z = gg / 54, y = (gg / 3) % 18, xh = (gg % 3) * 4;
+            u4v w = *reinterpret_cast<const u4v *>(xr + (z * 20 + y) * 12 + xh);
+            u4v b = *reinterpret_cast<const u4v *>(gr + gg * 4);
+            if (!in) w = b = u4v{0u, 0u, 0u, 0u};
+            acc = mfma32(w, b, acc);
+            if (j5 == 0) bsum = mfma32(ones, b, bsum);
+        }
+    }
+    float *P = a.part + ((int64_t)blockIdx.x * 2 + set) * kLP2;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {  // row 4 kg + j of the result
+        const int row = 4 * kg + j, q = 2 * j5 + (row >> 3), d = (row >> 1) & 3;
+        if (q < 9 && d < 3) P[((9 * (q / 3) + 3 * (q % 3) + d) * 2 + (row & 1)) * 16 + m] = acc[j];
+    }
+    if (j5 == 0 && kg == 0) P[27 * 2 * 16 + m] = bsum[0];
+}
+
+// grad[l][k] = the sum of layer l's partials: blockIdx.y = l, 64 parameters
+// per work-group, wave w adding the partials w, w + 8, ..., then the 8 waves
+// in order (deterministic).  Layer 0's partials hold its two input channels
+// only; the rest of its gradient is zero.
+struct WgSum {
+    const float *part[4];
+    int n[4];
+    float *grad;
+};
+__global__ __launch_bounds__(512) void reduce_partials_kernel(WgSum a) {
+    __shared__ float s[8][64];
+    const int l = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int k = blockIdx.x * 64 + lane;
+    const int c = (k >> 4) & 15;
+    const int row = l ? kLP : kLP2;
+    const int at = l || k >= kTap ? k - (kLP - row) : ((k >> 8) * 2 + c) * 16 + (k & 15);
+    const bool in = k < kLP && (l || k >= kTap || c < 2);
+    float v = 0.0f;
+    if (in) {
+        const float *p = a.part[l] + at;
+#pragma unroll 8
+        for (int w = wave; w < a.n[l]; w += 8) v += p[(int64_t)w * row];
+    }
+    s[wave][lane] = v;
+    __syncthreads();
+    if (wave == 0 && k < kLP) {
+        float t = s[0][lane];
+#pragma unroll
+        for (int w = 1; w < 8; ++w) t += s[w][lane];
+        a.grad[(int64_t)l * kLP + k] = t;
+    }
 }
 
 // Loss (y - target)^2 / (2 n 4096): G4 = (y - target) / (n 4096) in channel 0,
@@ -351,13 +499,22 @@ __global__ __launch_bounds__(256) void loss_kernel(const float *__restrict__ y, 
     if (threadIdx.x == 0) part[blockIdx.x] = ((s[0] + s[1]) + s[2]) + s[3];
 }
 
-__global__ void loss_reduce_kernel(const double *__restrict__ part, int n, double scale, double *loss_out,
-                                   float *loss_f) {
-    if (threadIdx.x != 0) return;
+// Sum of the n work-group partials: thread t takes t, t + 256, ..., then a fixed tree.
+__global__ __launch_bounds__(256) void loss_reduce_kernel(const double *__restrict__ part, int n, double scale,
+                                                          double *loss_out, float *loss_f) {
+    __shared__ double s_a[256];
     double s = 0.0;
-    for (int i = 0; i < n; ++i) s += part[i];
-    *loss_out = s * scale;
-    if (loss_f) *loss_f = (float)(s * scale);
+#pragma unroll 4
+    for (int i = threadIdx.x; i < n; i += 256) s += part[i];
+    s_a[threadIdx.x] = s;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if (threadIdx.x < o) s_a[threadIdx.x] += s_a[threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x != 0) return;
+    *loss_out = s_a[0] * scale;
+    if (loss_f) *loss_f = (float)(s_a[0] * scale);
 }
 
 __global__ void adam_kernel(float *p, float *m, float *v, const float *__restrict__ g, int n, float lr, float b1,
@@ -577,7 +734,8 @@ int ensure_ws(msbg_learned *n, int64_t tiles, bool train) {
         MSBG_HIP(hipMalloc(&n->G2, a16));
         MSBG_HIP(hipMalloc(&n->G3, a16));
         MSBG_HIP(hipMalloc(&n->G4, a16));
-        MSBG_HIP(hipMalloc(&n->wpart, (size_t)tiles * 23 * kLP * 4));
+        const size_t wgs = std::min<int64_t>(tiles, kWgTiles);
+        MSBG_HIP(hipMalloc(&n->wpart, wgs * (3 * kWg16Slabs * kLP + 2 * kWg2Slabs * kLP2) * 4));
         MSBG_HIP(hipMalloc(&n->loss_part, (size_t)tiles * 16 * sizeof(double)));
         n->cap_train = tiles;
     }
@@ -614,23 +772,30 @@ void forward(msbg_learned *net, hipStream_t s, const uint16_t *x0, const int32_t
     conv<16, 16, true>(s, net->A3, nullptr, 16, -1, W + 3 * kWB, P + 3 * kLP + kTap, 0, nullptr, net->Y, n);
 }
 
-template <int CIN>
-void wgrad(msbg_learned *net, hipStream_t s, const uint16_t *X, const int32_t *idx, int sin, int sout, int off,
-           const uint16_t *G, int n, float *grad) {
+// Partials of one layer's weight gradient in net->wpart: layers 1..3 one of
+// kLP floats per work-group, then layer 0 two of kLP2.
+WgArgs wgrad_args(msbg_learned *net, int l, const uint16_t *X, const int32_t *idx, int sin, int off,
+                  const uint16_t *G, int n) {
     WgArgs a;
     a.X = X;
     a.idx = idx;
     a.sin = sin;
-    a.sout = sout;
     a.off = off;
     a.G = G;
-    a.gpc = 16;
-    a.chunks = ((sout * sout * sout + 15) / 16 + a.gpc - 1) / a.gpc;
     a.n_tiles = n;
-    a.part = net->wpart;
-    const int64_t waves = (int64_t)a.chunks * n;
-    wgrad_kernel<CIN><<<(int)((waves + 3) / 4), 256, 0, s>>>(a);
-    reduce_partials_kernel<<<(kLP + 255) / 256, 256, 0, s>>>(net->wpart, (int)waves, grad);
+    a.groups = std::min(n, kWgTiles);
+    a.part = net->wpart + (int64_t)(l ? l - 1 : 3) * a.groups * kWg16Slabs * kLP;
+    return a;
+}
+
+const float *wgrad(msbg_learned *net, hipStream_t s, int l, const uint16_t *X, const int32_t *idx, int sin, int off,
+                   const uint16_t *G, int n) {
+    const WgArgs a = wgrad_args(net, l, X, idx, sin, off, G, n);
+    if (l)
+        wgrad16_kernel<<<a.groups * kWg16Slabs, kWg16Waves * 64, kWg16Lds, s>>>(a);
+    else
+        wgrad2_kernel<<<a.groups * kWg2Slabs, kWg2Waves * 64, kWg2Lds, s>>>(a);
+    return a.part;
 }
 
 // Loss and gradients of n tiles into net->d_grad; loss into net->d_loss (and loss_f if given).
@@ -640,16 +805,21 @@ void loss_grad(msbg_learned *net, hipStream_t s, const uint16_t *x0, const float
     const double inv = 1.0 / ((double)n * 4096.0);
     const int nb = n * 16;
     loss_kernel<<<nb, 256, 0, s>>>(net->Y, target, idx, n, (float)inv, net->G4, net->loss_part);
-    loss_reduce_kernel<<<1, 64, 0, s>>>(net->loss_part, nb, 0.5 * inv, net->d_loss, loss_f);
+    loss_reduce_kernel<<<1, 256, 0, s>>>(net->loss_part, nb, 0.5 * inv, net->d_loss, loss_f);
     const u4v *Wf = net->d_wbf;
-    float *g = net->d_grad;
-    wgrad<16>(net, s, net->A3, nullptr, 16, 16, -1, net->G4, n, g + 3 * kLP);
+    const int groups = std::min(n, kWgTiles);
+    WgSum sum;
+    sum.n[0] = groups * kWg2Slabs * 2;
+    sum.n[1] = sum.n[2] = sum.n[3] = groups * kWg16Slabs;
+    sum.grad = net->d_grad;
+    sum.part[3] = wgrad(net, s, 3, net->A3, nullptr, 16, -1, net->G4, n);
     conv<16, 16, false>(s, net->G4, nullptr, 16, -1, Wf + 3 * kWB, nullptr, 0, net->A3, net->G3, n);
-    wgrad<16>(net, s, net->A2, nullptr, 16, 16, -1, net->G3, n, g + 2 * kLP);
+    sum.part[2] = wgrad(net, s, 2, net->A2, nullptr, 16, -1, net->G3, n);
     conv<16, 16, false>(s, net->G3, nullptr, 16, -1, Wf + 2 * kWB, nullptr, 0, net->A2, net->G2, n);
-    wgrad<16>(net, s, net->A1, nullptr, 18, 16, 0, net->G2, n, g + 1 * kLP);
+    sum.part[1] = wgrad(net, s, 1, net->A1, nullptr, 18, 0, net->G2, n);
     conv<16, 18, false>(s, net->G2, nullptr, 16, -2, Wf + 1 * kWB, nullptr, 0, net->A1, net->G1, n);
-    wgrad<2>(net, s, x0, idx, 20, 18, 0, net->G1, n, g + 0 * kLP);
+    sum.part[0] = wgrad(net, s, 0, x0, idx, 20, 0, net->G1, n);
+    reduce_partials_kernel<<<dim3((kLP + 63) / 64, 4), 512, 0, s>>>(sum);
 }
 
 void prep(msbg_learned *net, hipStream_t s) {
@@ -743,6 +913,10 @@ int msbg_learned_new(msbg_learned **out) {
     if (e == hipSuccess)
         e = hipFuncSetAttribute((const void *)conv2_kernel<16, 20, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (kZS + 2) * 20 * 20 * 16 * 2);
+    if (e == hipSuccess)
+        e = hipFuncSetAttribute((const void *)wgrad16_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kWg16Lds);
+    if (e == hipSuccess)
+        e = hipFuncSetAttribute((const void *)wgrad2_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kWg2Lds);
     if (e != hipSuccess) {
         msbg_learned_free(n);
         return hip_fail(e, "msbg_learned_new");

@@ -165,3 +165,24 @@ def test_trained_corrector_gain_on_unseen_shell(pkg, hip):
             assert res[learned]["converged"]
         assert res[True]["accepted"] > 0
         assert res[True]["sweeps"] < res[False]["sweeps"], (storage, res)
+
+
+@pytest.mark.parametrize("n", [1, 33, 50, 64])
+def test_gradient_of_a_repeated_batch(pkg, hip, n):
+    """A batch given twice has the gradient of the batch (below, at and past
+    the 64 tile groups of the weight-gradient kernels; the loss factor 1 / n
+    halves exactly).  The two differ by the order of FP32 sums of products of
+    one sign pattern: at most ~1e5 terms a weight, whose rounding walk is below
+    sqrt(1e5) 2^-24 = 2e-5 of their root sum of squares, taken norm-wise with
+    the cancellation of a trained-from-noise gradient (factor 5)."""
+    rng = np.random.default_rng(n)
+    x = bf16_bits(rng.normal(size=(n, 20, 20, 20, 2)).astype(np.float32))
+    tgt = rng.normal(size=(n, 4096)).astype(np.float32)
+    from msbg_rs_amd.learned import init_params
+    net = net_for(pkg, hip, init_params(n))
+    l1, g1 = net.loss_grad(hip.to_device(x), hip.to_device(tgt), n)
+    l2, g2 = net.loss_grad(hip.to_device(np.concatenate([x, x])), hip.to_device(np.concatenate([tgt, tgt])), 2 * n)
+    assert l2 == pytest.approx(l1, rel=1e-12)
+    for l in range(4):
+        a, b = g1[l * 6928:(l + 1) * 6928], g2[l * 6928:(l + 1) * 6928]
+        assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(a), (l, np.linalg.norm(a - b) / np.linalg.norm(a))
