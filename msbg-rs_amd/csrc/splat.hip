@@ -1,19 +1,19 @@
 // Density min-splat: particles::splat (particles/splat.rs:92-319) for
 // D = Density (u16, channel.rs:303-375) into a u16 slab over a grid layout.
 //
-// A block's particle bucket is cut into work items of at most
-// kItemParticles particles, and each item's (16 + 2m)^3 window
-// (m = ceil(r_scan)) into kZSlabs z-slabs, one work-group each: the
-// work-group stages its slab in LDS as u32 cells initialised to 65535, walks
-// the item's particles in chunks (positions and footprint ranges staged in
-// LDS, keeping the particles whose footprint reaches the slab), lowers every
-// (particle, footprint row) pair's cells with an LDS atomic min of the
-// quantised distance, then commits its slab to the blocks it covers with
-// dst = min(dst, staging).  Buckets run in 8 colour passes (block-coordinate
-// parity), so same-colour windows never overlap (16 + 2m <= 32); the slabs of
-// one item are disjoint, and only the items of one split block (a dense
-// point-cloud instance) commit to the same cells, with an atomic min.  min is
-// associative and commutative, so the result does not depend on any order.
+// A block's particle bucket is cut into work items, one work-group each: it
+// stages the item's (16 + 2m)^3 window (m = ceil(r_scan)) in LDS as the bits
+// of the smallest squared distance so far, walks the item's particles in
+// chunks (positions and footprint ranges staged in LDS), lowers every
+// (particle, footprint row) pair's cells with an LDS atomic min, then
+// quantises the window once and commits it to the blocks it covers with an
+// atomic min.  Non-negative floats order as their bits do, and the quantised
+// distance never decreases with the distance, so the smallest distance gives
+// the smallest code.  min is associative and commutative, so neither the cut
+// nor the order of the items changes the result, and all of them run in one
+// launch: the 8 colour passes (block parity) that kept windows apart before
+// left ~120 work-groups a pass (512^3, 64 instances of 8,171 points: 8 x 165
+// us; one launch: see density_splat_kernel).
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -30,50 +30,48 @@ struct SplatParams {
     float r, dsq_max, inv;
 };
 
-constexpr int kMaxMargin = 6;   // window edge W <= 28
-constexpr int kZSlabs = 8;      // work-groups per window
-constexpr int kSlabPlanes = 4;  // ceil(28 / 8)
-constexpr int kChunk = 256;     // particles staged per pass (one per thread)
+constexpr int kMaxMargin = 6;   // window edge W <= 28: 88 KB of LDS
+constexpr int kSplatThreads = 512;
+constexpr int kChunk = 256;     // particles staged per pass
 
-// A work item of one colour pass: particles p0 .. p1 - 1 (bucketed order) of
-// occupied block blocks[k]; `shared` when the block's particles are split
-// over several items, whose windows then commit with an atomic min.
+// A work item: particles p0 .. p1 - 1 (bucketed order) of occupied block blocks[k].
 struct DItem {
-    int32_t k, p0, p1, shared;
+    int32_t k, p0, p1;
 };
-constexpr int kItemParticles = 1024;  // particles per item: a dense block (one point-cloud instance) is split
+// Particles per item: enough items to fill the chip four groups deep, but
+// between a row of LDS atomics that outweighs the window's fill and commit,
+// and a size past which splitting a dense block gains nothing.
+constexpr int kItemMin = 128, kItemMax = 1024, kItemsWanted = 1024;
 
-// dst = min(dst, v) on a 16-bit cell, atomically (compare-and-swap on its 32-bit word).
-__device__ __forceinline__ void atomic_min_u16(uint16_t *p, uint32_t v) {
-    uint32_t *w = reinterpret_cast<uint32_t *>(reinterpret_cast<uintptr_t>(p) & ~(uintptr_t)3);
-    const int sh = (reinterpret_cast<uintptr_t>(p) & 2) ? 16 : 0;
+// Lowers the two 16-bit cells of a word to lo / hi, atomically.
+__device__ __forceinline__ void atomic_min_2xu16(uint32_t *w, uint32_t lo, uint32_t hi) {
     uint32_t old = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    while (((old >> sh) & 0xffffu) > v) {
-        const uint32_t want = (old & ~(0xffffu << sh)) | (v << sh);
+    for (;;) {
+        const uint32_t want = min(old & 0xffffu, lo) | min(old >> 16, hi) << 16;
+        if (want == old) return;
         const uint32_t seen = atomicCAS(w, old, want);
-        if (seen == old) break;
+        if (seen == old) return;
         old = seen;
     }
 }
 
-__global__ __launch_bounds__(256) void density_splat_kernel(SplatParams P, const int32_t *__restrict__ b2s,
-                                                            uint16_t *slab, const float *__restrict__ pos,
-                                                            const int32_t *__restrict__ blocks,
-                                                            const DItem *__restrict__ items) {
-    __shared__ uint32_t st[28 * 28 * kSlabPlanes];
+// LDS atomics bound it: ~270 cells a particle at r_scan = 4.
+__global__ __launch_bounds__(kSplatThreads) void density_splat_kernel(SplatParams P, const int32_t *__restrict__ b2s,
+                                                                      uint16_t *slab, const float *__restrict__ pos,
+                                                                      const int32_t *__restrict__ blocks,
+                                                                      const DItem *__restrict__ items) {
+    extern __shared__ uint32_t st[];      // W^3 squared distances (float bits)
     __shared__ int rslot[27];
     __shared__ float s_p[kChunk][3];      // particle position - 0.5
-    __shared__ int16_t s_r[kChunk][6];    // footprint: ix1, ix2, iy1, iy2, iz1, iz2 (window coordinates, slab-clipped in z)
-    __shared__ int s_n;
-    const DItem item = items[blockIdx.x / kZSlabs];
-    const int zs = blockIdx.x % kZSlabs;
+    __shared__ int8_t s_r[kChunk][8];     // footprint: ix1, ix2, iy1, iy2, iz1, iz2 (window coordinates)
+    __shared__ int s_ext[2];              // largest footprint extent of the chunk in y, in z
+    const DItem item = items[blockIdx.x];
     const int bid = blocks[item.k];
     const int bx = bid % P.nx, by = (bid / P.nx) % P.ny, bz = bid / (P.nx * P.ny);
     const int W = P.W, m = P.m;
-    const int z0 = zs * W / kZSlabs, z1 = (zs + 1) * W / kZSlabs;  // window planes [z0, z1) of this work-group
-    const int cells = W * W * (z1 - z0);
-    if (cells <= 0) return;
-    for (int i = threadIdx.x; i < cells; i += blockDim.x) st[i] = 0xffffu;
+    const int cells = W * W * W;
+    constexpr uint32_t kFar = 0x7f800000u;  // +inf
+    for (int i = threadIdx.x; i < cells; i += kSplatThreads) st[i] = kFar;
     const int b0x = bx * 16, b0y = by * 16, b0z = bz * 16, hi = 16 + m - 1;
     if (threadIdx.x < 27) {
         // region (rx, ry, rz): skipped when any voxel lies outside the domain
@@ -91,64 +89,70 @@ __global__ __launch_bounds__(256) void density_splat_kernel(SplatParams P, const
     }
     // stage (splat.rs:179-225): footprint ceil(p - r - 0.5) .. floor(p + r - 0.5),
     // clipped to the window; d2 = dx*dx + (dz*dz + dy*dy)
-    const int p0 = item.p0, p1 = item.p1;
-    const int side = 2 * m + 1;
-    for (int c0 = p0; c0 < p1; c0 += kChunk) {
-        if (threadIdx.x == 0) s_n = 0;
-        __syncthreads();
-        const int j = c0 + (int)threadIdx.x;
-        if (j < p1) {
+    for (int c0 = item.p0; c0 < item.p1; c0 += kChunk) {
+        if (threadIdx.x < 2) s_ext[threadIdx.x] = 0;
+        __syncthreads();  // the last chunk's rows are done
+        const int q = threadIdx.x, j = c0 + q;
+        if (q < kChunk && j < item.p1) {
             const float px = pos[3 * j], py = pos[3 * j + 1], pz = pos[3 * j + 2];
-            const int iz1 = max(min(max((int)ceilf((pz - P.r) - 0.5f), b0z - m), b0z + hi) - (b0z - m), z0);
-            const int iz2 = min(min(max((int)floorf((pz + P.r) - 0.5f), b0z - m), b0z + hi) - (b0z - m), z1 - 1);
-            if (iz1 <= iz2) {
-                const int q = atomicAdd(&s_n, 1);
-                s_p[q][0] = px - 0.5f;
-                s_p[q][1] = py - 0.5f;
-                s_p[q][2] = pz - 0.5f;
-                s_r[q][0] = (int16_t)(min(max((int)ceilf((px - P.r) - 0.5f), b0x - m), b0x + hi) - (b0x - m));
-                s_r[q][1] = (int16_t)(min(max((int)floorf((px + P.r) - 0.5f), b0x - m), b0x + hi) - (b0x - m));
-                s_r[q][2] = (int16_t)(min(max((int)ceilf((py - P.r) - 0.5f), b0y - m), b0y + hi) - (b0y - m));
-                s_r[q][3] = (int16_t)(min(max((int)floorf((py + P.r) - 0.5f), b0y - m), b0y + hi) - (b0y - m));
-                s_r[q][4] = (int16_t)iz1;
-                s_r[q][5] = (int16_t)iz2;
-            }
+            auto lo_of = [&](float p, int b0) { return min(max((int)ceilf((p - P.r) - 0.5f), b0 - m), b0 + hi) - (b0 - m); };
+            auto hi_of = [&](float p, int b0) { return min(max((int)floorf((p + P.r) - 0.5f), b0 - m), b0 + hi) - (b0 - m); };
+            const int y1 = lo_of(py, b0y), y2 = hi_of(py, b0y), z1 = lo_of(pz, b0z), z2 = hi_of(pz, b0z);
+            s_p[q][0] = px - 0.5f;
+            s_p[q][1] = py - 0.5f;
+            s_p[q][2] = pz - 0.5f;
+            s_r[q][0] = (int8_t)lo_of(px, b0x);
+            s_r[q][1] = (int8_t)hi_of(px, b0x);
+            s_r[q][2] = (int8_t)y1;
+            s_r[q][3] = (int8_t)y2;
+            s_r[q][4] = (int8_t)z1;
+            s_r[q][5] = (int8_t)z2;
+            atomicMax(&s_ext[0], y2 - y1 + 1);
+            atomicMax(&s_ext[1], z2 - z1 + 1);
         }
         __syncthreads();
-        const int n = s_n, rows = kSlabPlanes * side;
-        for (int i = threadIdx.x; i < n * rows; i += blockDim.x) {
-            const int q = i / rows, rr = i - q * rows;
-            const int cz = s_r[q][4] + rr / side, cy = s_r[q][2] + rr % side;
-            if (cz > s_r[q][5] || cy > s_r[q][3]) continue;
+        const int n = min(kChunk, item.p1 - c0), ey = s_ext[0], rows = ey * s_ext[1];
+        for (int i = threadIdx.x; i < n * rows; i += kSplatThreads) {
+            const int p = i / rows, rr = i - p * rows;
+            const int cz = s_r[p][4] + rr / ey, cy = s_r[p][2] + rr % ey;
+            if (cz > s_r[p][5] || cy > s_r[p][3]) continue;
             // window cell (cx, cy, cz) is grid voxel (b0 - m) + c
-            const float dz = (float)(b0z - m + cz) - s_p[q][2], dy = (float)(b0y - m + cy) - s_p[q][1];
+            const float dz = (float)(b0z - m + cz) - s_p[p][2], dy = (float)(b0y - m + cy) - s_p[p][1];
             const float dyz = dz * dz + dy * dy;
-            uint32_t *row = st + ((cz - z0) * W + cy) * W;
-            const int cx2 = s_r[q][1];
-            for (int cx = s_r[q][0]; cx <= cx2; ++cx) {
-                const float dx = (float)(b0x - m + cx) - s_p[q][0];
+            if (dyz > P.dsq_max) continue;  // dx * dx >= 0: no cell of the row is in reach
+            uint32_t *row = st + (cz * W + cy) * W;
+            const int cx2 = s_r[p][1];
+            const float x0 = s_p[p][0];
+            for (int cx = s_r[p][0]; cx <= cx2; ++cx) {
+                const float dx = (float)(b0x - m + cx) - x0;
                 const float d2 = dx * dx + dyz;
-                if (d2 <= P.dsq_max) atomicMin(row + cx, (uint32_t)(int)roundf((d2 * P.inv) * 65535.0f));
+                if (d2 <= P.dsq_max) atomicMin(row + cx, __float_as_uint(d2));
             }
         }
-        __syncthreads();
     }
-    __syncthreads();  // the staging and the region table are complete even for an empty bucket
-    // commit (splat.rs:227-313): each touched window cell, dst = min(dst, staged)
-    for (int c = threadIdx.x; c < cells; c += blockDim.x) {
-        const uint32_t v = st[c];
-        if (v == 0xffffu) continue;
-        const int cx = c % W, cy = (c / W) % W, cz = z0 + c / (W * W);
-        const int rx = cx < m ? 0 : (cx < m + 16 ? 1 : 2), ry = cy < m ? 0 : (cy < m + 16 ? 1 : 2),
+    __syncthreads();  // the staging and the region table are complete
+    // commit (splat.rs:227-313): a word of two x-neighbours at a time (blocks
+    // and window regions start at even grid x, so both lie in one block and
+    // region; with an odd margin the first and last word's outer cell is not
+    // the window's), dst = min(dst, code)
+    const int odd = m & 1, words = (W + 2 * odd) / 2;
+    auto code = [&](int cx, int row) -> uint32_t {
+        if (cx < 0 || cx >= W) return 0xffffu;
+        const uint32_t v = st[row + cx];
+        return v == kFar ? 0xffffu : (uint32_t)(int)roundf((__uint_as_float(v) * P.inv) * 65535.0f);
+    };
+    for (int i = threadIdx.x; i < W * W * words; i += kSplatThreads) {
+        const int wd = i % words, r = i / words, cy = r % W, cz = r / W, cx = 2 * wd - odd;
+        const uint32_t lo = code(cx, r * W), hi16 = code(cx + 1, r * W);
+        if ((lo & hi16) == 0xffffu) continue;
+        const int cr = cx < 0 ? 0 : cx;
+        const int rx = cr < m ? 0 : (cr < m + 16 ? 1 : 2), ry = cy < m ? 0 : (cy < m + 16 ? 1 : 2),
                   rz = cz < m ? 0 : (cz < m + 16 ? 1 : 2);
         const int slot = rslot[rx + 3 * ry + 9 * rz];
         if (slot < 0) continue;
         const int gx = b0x + cx - m, gy = b0y + cy - m, gz = b0z + cz - m;
         uint16_t *d = slab + ((int64_t)slot << 12) + ((gx & 15) | ((gy & 15) << 4) | ((gz & 15) << 8));
-        if (item.shared)
-            atomic_min_u16(d, v);
-        else if (v < *d)
-            *d = (uint16_t)v;
+        atomic_min_2xu16(reinterpret_cast<uint32_t *>(d), lo, hi16);
     }
 }
 
@@ -234,38 +238,27 @@ int msbg_density_splat(msbg_grid *g, uint16_t *d_slab16, int64_t slab_slots, con
     P.r = r_scan;
     P.dsq_max = r_scan * r_scan;
     P.inv = 1.0f / P.dsq_max;
-    // colour lists of work items (the 8 parity buckets of splat.rs:114-123),
-    // each block's particles cut into items of at most kItemParticles
-    std::vector<int32_t> hb((size_t)nb), hs((size_t)nb + 1);
-    MSBG_HIP(hipMemcpyAsync(hb.data(), d_blocks, sizeof(int32_t) * nb, hipMemcpyDeviceToHost, s));
+    // work items: each block's particles, cut
+    int64_t cut = kItemMin;
+    while (cut < kItemMax && cut * kItemsWanted < n) cut *= 2;
+    std::vector<int32_t> hs((size_t)nb + 1);
     MSBG_HIP(hipMemcpyAsync(hs.data(), d_starts, sizeof(int32_t) * (nb + 1), hipMemcpyDeviceToHost, s));
     MSBG_HIP(hipStreamSynchronize(s));
     std::vector<DItem> order;
-    int64_t cnt[8] = {0};
-    for (int c = 0; c < 8; ++c)
-        for (int64_t i = 0; i < nb; ++i) {
-            const int64_t b = hb[i];
-            const int64_t bx = b % g->nx, by = (b / g->nx) % g->ny, bz = b / (g->nx * g->ny);
-            if ((int)((bx & 1) | ((by & 1) << 1) | ((bz & 1) << 2)) != c) continue;
-            const int32_t p0 = hs[i], p1 = hs[i + 1];
-            const int32_t shared = p1 - p0 > kItemParticles ? 1 : 0;
-            for (int32_t q = p0; q < p1; q += kItemParticles) {
-                order.push_back(DItem{(int32_t)i, q, std::min(p1, q + kItemParticles), shared});
-                ++cnt[c];
-            }
-        }
-    MSBG_CHECK((int64_t)order.size() * kZSlabs < ((int64_t)1 << 31), MSBG_EINVAL,
-               "density splat: too many work items");
+    order.reserve((size_t)(nb + n / cut));
+    for (int64_t i = 0; i < nb; ++i)
+        for (int32_t q = hs[i]; q < hs[i + 1]; q += (int32_t)cut)
+            order.push_back(DItem{(int32_t)i, q, (int32_t)std::min<int64_t>(hs[i + 1], q + cut)});
     DItem *d_items = (DItem *)workspace(23, sizeof(DItem) * std::max<size_t>(order.size(), 1), &rc);
     if (rc) return rc;
     MSBG_HIP(hipMemcpyAsync(d_items, order.data(), sizeof(DItem) * order.size(), hipMemcpyHostToDevice, s));
-    int64_t off = 0;
-    for (int c = 0; c < 8; ++c) {
-        if (cnt[c])
-            density_splat_kernel<<<(int)(cnt[c] * kZSlabs), 256, 0, s>>>(P, g->d_b2s, d_slab16, d_sorted, d_blocks,
-                                                                       d_items + off);
-        off += cnt[c];
-    }
+    const size_t lds = sizeof(uint32_t) * P.W * P.W * P.W;
+    if (lds > 65536)
+        MSBG_HIP(hipFuncSetAttribute((const void *)density_splat_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int)lds));
+    if (!order.empty())
+        density_splat_kernel<<<(unsigned)order.size(), kSplatThreads, lds, s>>>(P, g->d_b2s, d_slab16, d_sorted,
+                                                                              d_blocks, d_items);
     MSBG_HIP(hipGetLastError());
     MSBG_HIP(hipStreamSynchronize(s));
     return MSBG_OK;
