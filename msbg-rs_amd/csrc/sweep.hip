@@ -64,16 +64,62 @@ __device__ __forceinline__ float4 load4(const uint8_t *p) {
     return make_float4(deq((uint8_t)(u & 0xffu)), deq((uint8_t)((u >> 8) & 0xffu)), deq((uint8_t)((u >> 16) & 0xffu)),
                        deq((uint8_t)(u >> 24)));
 }
+// Access of a slab cell whose value another work-group of the same launch may
+// write (the one-launch sweeps): agent-scope relaxed atomics, which the 8 XCDs'
+// L2s keep coherent, at the speed of plain accesses (measured: 12.4 TB/s over
+// 32 MB either way).  COH = false: plain accesses.
+template <typename T>
+__device__ __forceinline__ T ld_agent(const void *p) {
+    return __hip_atomic_load((const __attribute__((address_space(1))) T *)p, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+}
+template <bool COH, typename T>
+__device__ __forceinline__ T ld_cell(const T *p) {
+    if constexpr (!COH)
+        return ld_global<T>(p);
+    else if constexpr (sizeof(T) == 4)
+        return __builtin_bit_cast(T, ld_agent<uint32_t>(p));
+    else
+        return ld_agent<T>(p);
+}
+template <bool COH>
+__device__ __forceinline__ float4 ld_quad(const float *p) {
+    if constexpr (!COH) return load4(p);
+    const uint64_t a = ld_agent<uint64_t>(p), b = ld_agent<uint64_t>(p + 2);
+    return make_float4(__uint_as_float((uint32_t)a), __uint_as_float((uint32_t)(a >> 32)),
+                       __uint_as_float((uint32_t)b), __uint_as_float((uint32_t)(b >> 32)));
+}
+template <bool COH>
+__device__ __forceinline__ float4 ld_quad(const uint16_t *p) {
+    if constexpr (!COH) return load4(p);
+    const uint64_t u = ld_agent<uint64_t>(p);
+    return make_float4(deq((uint16_t)u), deq((uint16_t)(u >> 16)), deq((uint16_t)(u >> 32)), deq((uint16_t)(u >> 48)));
+}
+template <bool COH>
+__device__ __forceinline__ float4 ld_quad(const uint8_t *p) {
+    if constexpr (!COH) return load4(p);
+    const uint32_t u = ld_agent<uint32_t>(p);
+    return make_float4(deq((uint8_t)u), deq((uint8_t)(u >> 8)), deq((uint8_t)(u >> 16)), deq((uint8_t)(u >> 24)));
+}
 // The stochastic-rounding stream of a Density8 sweep: seed and a device
 // counter of the sweeps done (read once per work-group).
 struct SrCtx {
     uint32_t seed;
     const uint32_t *ctr;
 };
-__device__ __forceinline__ void store_back(float *p, float v) { *p = v; }
-__device__ __forceinline__ void store_back(uint16_t *p, float v) {
-    const float r = fminf(fmaxf(roundf(v * 65535.0f), 0.0f), 65535.0f);
-    *p = (uint16_t)(int)r;
+__device__ __forceinline__ float quant(float v, float *) { return v; }
+__device__ __forceinline__ uint16_t quant(float v, uint16_t *) {
+    return (uint16_t)(int)fminf(fmaxf(roundf(v * 65535.0f), 0.0f), 65535.0f);
+}
+template <bool COH, typename T>
+__device__ __forceinline__ void st_cell(T *p, T v) {
+    if constexpr (!COH)
+        *p = v;
+    else if constexpr (sizeof(T) == 4)
+        __hip_atomic_store(reinterpret_cast<uint32_t *>(p), __builtin_bit_cast(uint32_t, v), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    else
+        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---------------------------------------------------------------------------
@@ -279,138 +325,119 @@ __device__ __forceinline__ int tile_at(int hx, int hy, int hz) {
 
 // Pitched per-cell fill: the path for a block whose rows cross the domain's
 // x end (partial last block, halo.rs:130-144).
-template <int HALO, bool MULTI, typename TS>
+template <int HALO, bool MULTI, int NTHR, typename TS, bool COH>
 __device__ void fill_tile_pitched_generic(float *tile, const TS *fs, const GridView &g, const GridView &c,
                                           const int *s_nb, const int *s_nbc, int bx0, int by0, int bz0,
-                                          float empty_f32) {
+                                          float empty_f32, int t) {
     constexpr int B = 16, HSX = B + 2 * HALO, NT = HSX * HSX * HSX;
     const int x0 = bx0 * B, y0 = by0 * B, z0 = bz0 * B;
-    for (int i = threadIdx.x; i < NT; i += blockDim.x) {
+    for (int i = t; i < NT; i += NTHR) {
         const int hx = i % HSX, hy = (i / HSX) % HSX, hz = i / (HSX * HSX);
         int rx, ry, rz;
         float v = empty_f32;
         if (resolve_axis(x0 + hx - HALO, g.sx - 1, MSBG_BC_NEUMANN, rx) &&
             resolve_axis(y0 + hy - HALO, g.sy - 1, MSBG_BC_NEUMANN, ry) &&
             resolve_axis(z0 + hz - HALO, g.sz - 1, MSBG_BC_NEUMANN, rz))
-            v = deq(*cell_ptr<HALO, MULTI, TS>(fs, c, s_nb, s_nbc, bx0, by0, bz0, rx, ry, rz));
+            v = deq(ld_cell<COH>(cell_ptr<HALO, MULTI, TS>(fs, c, s_nb, s_nbc, bx0, by0, bz0, rx, ry, rz)));
         tile[tile_at<HALO>(hx, hy, hz)] = v;
     }
 }
 
-// Row-wise pitched fill for blocks whose rows lie inside the domain in x.  A
-// tile row (hy, hz) is resolved once: its 16 interior cells are one block row
-// (four float4 loads, or two float2 loads duplicated for a coarse
-// neighbour), its 2H x-halo cells are loaded one by one.  SKIP leaves out
-// the tile cells the stencil never reads: kSkipCross (7-point: the corner
-// rows and the x-halo of every row outside the block in y or z) or
-// kSkipBiLap (25-tap: a row outside the block in y or z at distance 2 takes
-// no x-halo, at distance 1 only the inner x-halo cell; of the corner rows only
-// the four at distance 1 in both y and z, without x-halo).  An x-halo cell
+// Row-wise pitched fill for blocks whose rows lie inside the domain in x (and
+// domains of at least kRowsMinDomain cells an axis, where a halo cell mirrors
+// once).  A tile row (hy, hz) is resolved by one lane: it puts the row's address into the unused words at the
+// start of the row's pitch and loads the row's 2H x-halo cells; after the
+// barrier, which also lets the other lanes see the addresses, lane 4 r + q
+// loads quad q of row r (16 bytes; of a coarse neighbour the aligned half of
+// the 8-cell row that holds the quad's two cells).  Resolving every quad and
+// halo cell on its own took ~1,200 instructions a lane, more than the stencil
+// (512^3 band, curvature + bi-Laplacian: 215 us; 205 us with this fill, 191 us
+// with the lane order of update_block16, 187 us with its constant offsets).
+// SKIP leaves out the tile cells the stencil never reads: kSkipCross
+// (7-point: the corner rows and the x-halo of every row outside the block in y
+// or z) or kSkipBiLap (25-tap: a row outside the block in y or z at distance 2
+// takes no x-halo, at distance 1 only the inner x-halo cell; of the corner rows
+// only the four at distance 1 in both y and z, without x-halo).  An x-halo cell
 // of a row outside the block lives in a diagonal neighbour block, so each
 // skipped one saves a line fetched for a single value.
+// `publish` is a barrier (of the one-launch sweeps: after the waits for the
+// neighbours); no cell is read before it.
 constexpr int kSkipNone = 0, kSkipCross = 1, kSkipBiLap = 2;
+constexpr int kRowsMinDomain = 9;  // cells reach 17 past a block's start: 2 * 9 - 1 - 17 = 0
 
-template <int HALO, bool MULTI, int NTHR, typename TS, int SKIP>
+template <int HALO, bool MULTI, int NTHR, typename TS, int SKIP, bool COH, class Publish>
 __device__ __forceinline__ void fill_tile_rows(float *tile, const TS *fs, const GridView &g, const GridView &c,
-                                               const int *s_nb, const int *s_nbc, int bx0, int by0, int bz0,
-                                               float empty_f32) {
-    constexpr int B = 16, L = 4, HSX = B + 2 * HALO, n = 2 * HALO + 1;
-    constexpr int NR = HSX * HSX, NQ = 4 * NR, NH = 2 * HALO * NR;
-    constexpr int QI = (NQ + NTHR - 1) / NTHR, HI = (NH + NTHR - 1) / NTHR;
-    const int x0 = bx0 * B, y0 = by0 * B, z0 = bz0 * B;
-    const int t = threadIdx.x;
-    const TS *qp[QI];
-    uint32_t qcoarse = 0, qwrite = 0;
+                                               const int *s_nb, const int *s_nbc, int bx0, int by0, int bz0, int t,
+                                               Publish publish) {
+    constexpr int B = 16, HSX = B + 2 * HALO, n = 2 * HALO + 1, NR = HSX * HSX;
+    constexpr int QI = (4 * NR + NTHR - 1) / NTHR;
+    static_assert(NR <= NTHR, "a lane per row");
+    static_assert(4 - HALO >= 2, "two free words at the start of a row");
+    auto mirror = [](int v, int s) { return min(max(v, -1 - v), 2 * s - 1 - v); };
+    const TS *hp[2 * HALO];
 #pragma unroll
-    for (int k = 0; k < QI; ++k) {  // interior quads: item = row * 4 + q
-        const int it = t + k * NTHR;
-        qp[k] = nullptr;
-        if (it >= NQ) continue;
-        const int r = it >> 2, q = it & 3;
-        const int hy = r % HSX, hz = r / HSX;
-        const bool yh = hy < HALO || hy >= HALO + B, zh = hz < HALO || hz >= HALO + B;
-        if (SKIP == kSkipCross && yh && zh) continue;
-        if (SKIP == kSkipBiLap && yh && zh && (out_dist<HALO>(hy) != 1 || out_dist<HALO>(hz) != 1)) continue;
-        qwrite |= 1u << k;
-        int ry, rz;
-        if (!resolve_axis(y0 + hy - HALO, g.sy - 1, MSBG_BC_NEUMANN, ry) ||
-            !resolve_axis(z0 + hz - HALO, g.sz - 1, MSBG_BC_NEUMANN, rz))
-            continue;
-        const int nb = HALO + n * ((ry >> L) - by0 + HALO) + n * n * ((rz >> L) - bz0 + HALO);
-        if (MULTI && s_nbc[nb] >= 0) {
-            // the aligned half of the 8-cell coarse row that holds this
-            // quad's two coarse cells (its elements 2 (q & 1), + 1)
-            qcoarse |= 1u << k;
-            qp[k] = reinterpret_cast<const TS *>(c.slab + (int64_t)s_nbc[nb] * 512 + (((ry >> 1) & 7) << 3) +
-                                                 (((rz >> 1) & 7) << 6) + 4 * (q >> 1));
+    for (int j = 0; j < 2 * HALO; ++j) hp[j] = nullptr;
+    if (t < NR) {
+        const int hz = t / HSX, hy = t - hz * HSX;
+        const int oy = out_dist<HALO>(hy), oz = out_dist<HALO>(hz);
+        const bool out = oy | oz, corner = oy && oz;
+        const bool row = SKIP == kSkipNone || !corner || (SKIP == kSkipBiLap && oy == 1 && oz == 1);
+        const int gy = mirror(by0 * B + hy - HALO, g.sy), gz = mirror(bz0 * B + hz - HALO, g.sz);
+        const int nyz = n * ((gy >> 4) - by0 + HALO) + n * n * ((gz >> 4) - bz0 + HALO);
+        const int cell = (gy & 15) << 4 | (gz & 15) << 8, ccell = ((gy >> 1) & 7) << 3 | ((gz >> 1) & 7) << 6;
+        const TS *rp = nullptr;
+        uint64_t coarse = 0;
+        if (MULTI && s_nbc[HALO + nyz] >= 0) {
+            rp = reinterpret_cast<const TS *>(c.slab + (int64_t)s_nbc[HALO + nyz] * 512 + ccell);
+            coarse = 1;  // rows are 32-byte aligned at least
         } else {
-            qp[k] = fs + (int64_t)s_nb[nb] * 4096 + ((ry & 15) << 4) + ((rz & 15) << 8) + 4 * q;
+            rp = fs + (int64_t)s_nb[HALO + nyz] * 4096 + cell;
         }
-    }
-    const TS *hp[HI];
-    uint32_t hwrite = 0;
+        *reinterpret_cast<uint64_t *>(tile + t * kPitch) = row ? (uint64_t)rp | coarse : 0ull;
 #pragma unroll
-    for (int k = 0; k < HI; ++k) {  // x-halo cells: item = row * 2H + j; j < H left
-        const int it = t + k * NTHR;
-        hp[k] = nullptr;
-        if (it >= NH) continue;
-        const int r = it / (2 * HALO), j = it % (2 * HALO);
-        const int hy = r % HSX, hz = r / HSX;
-        const bool yh = hy < HALO || hy >= HALO + B, zh = hz < HALO || hz >= HALO + B;
-        if (SKIP == kSkipCross && (yh || zh)) continue;
-        if (SKIP == kSkipBiLap && (yh || zh)) {
-            // only rows at distance 1 outside (not corners) take the inner x-halo cell
+        for (int j = 0; j < 2 * HALO; ++j) {  // x-halo cells, j < H left
             const bool inner = j == HALO - 1 || j == HALO;
-            if ((yh && zh) || !inner || out_dist<HALO>(yh ? hy : hz) != 1) continue;
-        }
-        hwrite |= 1u << k;
-        const int gx = j < HALO ? x0 - HALO + j : x0 + B + (j - HALO);
-        int rx, ry, rz;
-        if (resolve_axis(gx, g.sx - 1, MSBG_BC_NEUMANN, rx) &&
-            resolve_axis(y0 + hy - HALO, g.sy - 1, MSBG_BC_NEUMANN, ry) &&
-            resolve_axis(z0 + hz - HALO, g.sz - 1, MSBG_BC_NEUMANN, rz))
-            hp[k] = cell_ptr<HALO, MULTI, TS>(fs, c, s_nb, s_nbc, bx0, by0, bz0, rx, ry, rz);
-    }
-    float4 qv[QI];
-    float hv[HI];
-    if constexpr (MULTI) {
-        // One aligned 16-byte load per item, fine or coarse, none behind a
-        // branch, so a lane's loads are all in flight together; an item with
-        // no source reads the slab's first cells and takes the empty value.
-        float4 raw[QI];
-#pragma unroll
-        for (int k = 0; k < QI; ++k) raw[k] = load4(qp[k] ? qp[k] : fs);
-#pragma unroll
-        for (int k = 0; k < HI; ++k) hv[k] = hp[k] ? deq(ld_global<TS>(hp[k])) : empty_f32;
-#pragma unroll
-        for (int k = 0; k < QI; ++k) {
-            const int q = (t + k * NTHR) & 3;
-            if (!qp[k])
-                qv[k] = make_float4(empty_f32, empty_f32, empty_f32, empty_f32);
-            else if ((qcoarse >> k) & 1u)
-                qv[k] = (q & 1) ? make_float4(raw[k].z, raw[k].z, raw[k].w, raw[k].w)
-                                : make_float4(raw[k].x, raw[k].x, raw[k].y, raw[k].y);
+            const bool need = SKIP == kSkipNone    ? true
+                              : SKIP == kSkipCross ? !out
+                                                   : !out || (inner && !corner && oy + oz == 1);
+            if (!need) continue;
+            const int gx = mirror(bx0 * B + (j < HALO ? j - HALO : B + j - HALO), g.sx);  // uniform
+            const int nb = (gx >> 4) - bx0 + HALO + nyz;
+            if (MULTI && s_nbc[nb] >= 0)
+                hp[j] = reinterpret_cast<const TS *>(c.slab + (int64_t)s_nbc[nb] * 512 + ((gx >> 1) & 7) + ccell);
             else
-                qv[k] = raw[k];
+                hp[j] = fs + (int64_t)s_nb[nb] * 4096 + (gx & 15) + cell;
         }
-    } else {
-#pragma unroll
-        for (int k = 0; k < QI; ++k)
-            qv[k] = qp[k] ? load4(qp[k]) : make_float4(empty_f32, empty_f32, empty_f32, empty_f32);
-#pragma unroll
-        for (int k = 0; k < HI; ++k) hv[k] = hp[k] ? deq(ld_global<TS>(hp[k])) : empty_f32;
     }
+    publish();
+    uint64_t qe[QI];
+#pragma unroll
+    for (int k = 0; k < QI; ++k) {
+        const int it = t + k * NTHR;
+        qe[k] = it < 4 * NR ? *reinterpret_cast<const uint64_t *>(tile + (it >> 2) * kPitch) : 0ull;
+    }
+    float hv[2 * HALO];
+#pragma unroll
+    for (int j = 0; j < 2 * HALO; ++j) hv[j] = hp[j] ? deq(ld_cell<COH>(hp[j])) : 0.0f;
+    const int q = t & 3;  // NTHR is a multiple of 4
+    float4 qv[QI];
+#pragma unroll
+    for (int k = 0; k < QI; ++k) {
+        qv[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (!qe[k]) continue;
+        const TS *p = reinterpret_cast<const TS *>(qe[k] & ~1ull);
+        qv[k] = ld_quad<COH>(p + (MULTI && (qe[k] & 1) ? 4 * (q >> 1) : 4 * q));
+    }
+#pragma unroll
+    for (int j = 0; j < 2 * HALO; ++j)
+        if (hp[j]) tile[t * kPitch + (j < HALO ? 4 - HALO + j : 20 + (j - HALO))] = hv[j];
 #pragma unroll
     for (int k = 0; k < QI; ++k)
-        if ((qwrite >> k) & 1u) {
-            const int it = t + k * NTHR, r = it >> 2, q = it & 3;
-            *reinterpret_cast<float4 *>(tile + r * kPitch + 4 + 4 * q) = qv[k];
-        }
-#pragma unroll
-    for (int k = 0; k < HI; ++k)
-        if ((hwrite >> k) & 1u) {
-            const int it = t + k * NTHR, r = it / (2 * HALO), j = it % (2 * HALO);
-            tile[r * kPitch + (j < HALO ? 4 - HALO + j : 20 + (j - HALO))] = hv[k];
+        if (qe[k]) {
+            if (MULTI && (qe[k] & 1))
+                qv[k] = (q & 1) ? make_float4(qv[k].z, qv[k].z, qv[k].w, qv[k].w)
+                                : make_float4(qv[k].x, qv[k].x, qv[k].y, qv[k].y);
+            *reinterpret_cast<float4 *>(tile + ((t + k * NTHR) >> 2) * kPitch + 4 + 4 * q) = qv[k];
         }
 }
 
@@ -434,61 +461,60 @@ constexpr int sweep_tile_floats() {
 // z-halves; each lane walks 8 cells up its z column keeping the planes it
 // still needs in registers (5 / 9 / 13 LDS reads per cell for the 7 / 19 /
 // 25-tap stencils once the window is primed).
-template <int STENCIL, bool MULTI, typename TS>
-__device__ __forceinline__ void sweep_block16(GridView g, GridView c, TS *__restrict__ fslab,
-                                              const float *__restrict__ cslab, int64_t bid, const int32_t *row,
-                                              float dt, int clamp01, float empty_f32, float *tile, int *s_nb,
-                                              int *s_nbc, SrCtx sr) {
-    static_assert(!MULTI || sizeof(TS) == sizeof(float), "cross-level sweeps are FP32 only");
-    c.slab = const_cast<float *>(cslab);
+// The tile of block (bx0, by0, bz0), by the NTHR lanes t of the work-group.
+template <int STENCIL, bool MULTI, typename TS, int NTHR, bool COH, class Publish>
+__device__ __forceinline__ void fill_block16(const GridView &g, const GridView &c, const TS *fslab,
+                                             int bx0, int by0, int bz0, float empty_f32, float *tile, const int *s_nb,
+                                             const int *s_nbc, int t, Publish publish) {
     constexpr int HALO = STENCIL == MSBG_BILAPLACIAN ? 2 : 1;
-    constexpr int HSX = 16 + 2 * HALO, NN = 2 * HALO + 1, NB = NN * NN * NN, CENTER = (NB - 1) / 2;
-    constexpr int CPT = 16 * 256 / kSweepThreads;  // cells per lane along z
-    const int slot = row[CENTER];
-    if (slot < 2) return;  // dummy or absent: solver.rs:201-204 (uniform per workgroup)
-    if (threadIdx.x < NB) {
-        const int code = row[threadIdx.x];
-        s_nb[threadIdx.x] = code >= 0 ? code : 0;
-        if (MULTI) s_nbc[threadIdx.x] = code >= 0 ? -1 : -code - 1;
-    }
-    const int bx0 = (int)(bid % g.nx), by0 = (int)((bid / g.nx) % g.ny), bz0 = (int)(bid / ((int64_t)g.nx * g.ny));
-    __syncthreads();
-    if (bx0 * 16 + 16 <= g.sx)
-        fill_tile_rows<HALO, MULTI, kSweepThreads, TS,
+    if (bx0 * 16 + 16 <= g.sx && min(g.sx, min(g.sy, g.sz)) >= kRowsMinDomain) {
+        fill_tile_rows<HALO, MULTI, NTHR, TS,
                        STENCIL == MSBG_LAPLACIAN ? kSkipCross
-                                                 : (STENCIL == MSBG_BILAPLACIAN ? kSkipBiLap : kSkipNone)>(
-            tile, fslab, g, c, s_nb, s_nbc, bx0, by0, bz0, empty_f32);
-    else
-        fill_tile_pitched_generic<HALO, MULTI, TS>(tile, fslab, g, c, s_nb, s_nbc, bx0, by0, bz0, empty_f32);
-    __syncthreads();
+                                                 : (STENCIL == MSBG_BILAPLACIAN ? kSkipBiLap : kSkipNone),
+                       COH>(tile, fslab, g, c, s_nb, s_nbc, bx0, by0, bz0, t, publish);
+    } else {
+        publish();
+        fill_tile_pitched_generic<HALO, MULTI, NTHR, TS, COH>(tile, fslab, g, c, s_nb, s_nbc, bx0, by0, bz0,
+                                                              empty_f32, t);
+    }
+}
 
-    const int x = threadIdx.x & 15, y = (threadIdx.x >> 4) & 15, zs = (threadIdx.x >> 8) * CPT;
-    TS *out = fslab + (int64_t)slot * 4096 + y * 16 + x;
+// The update of the block in `slot` from its tile, in place.  sr_key: the
+// sweep's stochastic-rounding key (Density8).
+template <int STENCIL, typename TS, int NTHR, bool COH>
+__device__ __forceinline__ void update_block16(TS *fslab, int slot, int64_t bid, float dt, int clamp01,
+                                               const float *tile, uint32_t sr_key, int t) {
+    constexpr int HALO = STENCIL == MSBG_BILAPLACIAN ? 2 : 1;
+    constexpr int HSX = 16 + 2 * HALO;
+    constexpr int CPT = 16 * 256 / NTHR;  // cells per lane along z
+    // Rows y and y + 2 side by side in a half wave: their tile rows start 2
+    // kPitch = 48 words apart, 16 banks, so a tap's 32 reads fall on 32 banks
+    // (rows y and y + 1, 24 words apart, collided on a quarter of them).
+    const int x = t & 15, y = ((t >> 4) & 12) | ((t >> 5) & 1) | ((t >> 3) & 2), zs = (t >> 8) * CPT;
+    TS *out = fslab + (int64_t)slot * 4096 + zs * 256 + y * 16 + x;
     const bool cl = clamp01 != 0;
-    uint32_t sr_key = 0;
-    if constexpr (std::is_same<TS, uint8_t>::value) sr_key = sr_sweep_key(sr.seed, *sr.ctr);
-    // StoreBack of cell (x, y, z)
+    // StoreBack of cell (x, y, zs + z)
     auto put = [&](int z, float v) {
         if constexpr (std::is_same<TS, uint8_t>::value)
-            out[z * 256] = sr_quant8(v, sr_uniform(sr_key, (uint32_t)bid, (uint32_t)(z * 256 + y * 16 + x)));
+            st_cell<COH>(out + z * 256,
+                         sr_quant8(v, sr_uniform(sr_key, (uint32_t)bid, (uint32_t)((zs + z) * 256 + y * 16 + x))));
         else
-            store_back(out + z * 256, v);
+            st_cell<COH>(out + z * 256, quant(v, (TS *)nullptr));
     };
-    // T(dx, dy, z): tile value at block cell (x+dx, y+dy, z).  The lane's
-    // base is the low corner (x - H, y - H, zs - H) of its stencils, so every
-    // read is the base plus a constant (z is zs plus a constant at each call).
+    // T(dx, dy, z): tile value at block cell (x + dx, y + dy, zs + z).  The
+    // lane's base is the low corner (x - H, y - H, zs - H) of its stencils, so
+    // every read is the base plus a constant (z is one at each call).
     const float *tb = tile + tile_at<HALO>(x, y, zs);
     auto T = [&](int dx, int dy, int z) -> float {
-        return tb[((z - zs + HALO) * HSX + (dy + HALO)) * kPitch + (dx + HALO)];
+        return tb[((z + HALO) * HSX + (dy + HALO)) * kPitch + (dx + HALO)];
     };
     auto cross = [&](int z) -> Cross { return Cross{T(0, 0, z), T(-1, 0, z), T(1, 0, z), T(0, -1, z), T(0, 1, z)}; };
 
     if (STENCIL == MSBG_LAPLACIAN) {
         // kernel_laplacian -- math/laplacian.rs:44-61
-        float cm = T(0, 0, zs - 1), c0 = T(0, 0, zs);
+        float cm = T(0, 0, -1), c0 = T(0, 0, 0);
 #pragma unroll
-        for (int k = 0; k < CPT; ++k) {
-            const int z = zs + k;
+        for (int z = 0; z < CPT; ++z) {
             const float cp = T(0, 0, z + 1);
             const float cc = c0, lx = T(-1, 0, z), rx = T(1, 0, z), dyu = T(0, -1, z), dyd = T(0, 1, z), dzb = cm,
                         dzf = cp;
@@ -503,10 +529,9 @@ __device__ __forceinline__ void sweep_block16(GridView g, GridView c, TS *__rest
         }
     } else if (STENCIL == MSBG_MEAN_CURVATURE) {
         // kernel_meancurv -- math/meancurv.rs:49-100
-        Cross pm = cross(zs - 1), p0 = cross(zs);
+        Cross pm = cross(-1), p0 = cross(0);
 #pragma unroll
-        for (int k = 0; k < CPT; ++k) {
-            const int z = zs + k;
+        for (int z = 0; z < CPT; ++z) {
             const Cross pp = cross(z + 1);
             const float f0 = p0.c, f1 = p0.xm, f2 = p0.xp, f3 = p0.ym, f4 = p0.yp, f5 = pm.c, f6 = pp.c;
             const float fx = (f2 - f1) * 0.5f, fy = (f4 - f3) * 0.5f, fz = (f6 - f5) * 0.5f;
@@ -531,11 +556,10 @@ __device__ __forceinline__ void sweep_block16(GridView g, GridView c, TS *__rest
         }
     } else {
         // kernel_bilaplacian -- math/bilaplacian.rs:47-88
-        float cm2 = T(0, 0, zs - 2);
-        Cross pm = cross(zs - 1), p0 = cross(zs), pp = cross(zs + 1);
+        float cm2 = T(0, 0, -2);
+        Cross pm = cross(-1), p0 = cross(0), pp = cross(1);
 #pragma unroll
-        for (int k = 0; k < CPT; ++k) {
-            const int z = zs + k;
+        for (int z = 0; z < CPT; ++z) {
             const Cross pp2 = cross(z + 2);
             const float f0 = p0.c, f1 = p0.xm, f2 = p0.xp, f3 = p0.ym, f4 = p0.yp, f5 = pm.c, f6 = pp.c;
             const float s1 = f1 + f2 + f3 + f4 + f5 + f6;
@@ -555,6 +579,33 @@ __device__ __forceinline__ void sweep_block16(GridView g, GridView c, TS *__rest
             pp = pp2;
         }
     }
+}
+
+// Both, by a whole work-group of kSweepThreads (one block of a colour pass).
+template <int STENCIL, bool MULTI, typename TS>
+__device__ __forceinline__ void sweep_block16(GridView g, GridView c, TS *__restrict__ fslab,
+                                              const float *__restrict__ cslab, int64_t bid, const int32_t *row,
+                                              float dt, int clamp01, float empty_f32, float *tile, int *s_nb,
+                                              int *s_nbc, SrCtx sr) {
+    static_assert(!MULTI || sizeof(TS) == sizeof(float), "cross-level sweeps are FP32 only");
+    c.slab = const_cast<float *>(cslab);
+    constexpr int HALO = STENCIL == MSBG_BILAPLACIAN ? 2 : 1;
+    constexpr int NN = 2 * HALO + 1, NB = NN * NN * NN, CENTER = (NB - 1) / 2;
+    const int slot = row[CENTER];
+    if (slot < 2) return;  // dummy or absent: solver.rs:201-204 (uniform per workgroup)
+    if (threadIdx.x < NB) {
+        const int code = row[threadIdx.x];
+        s_nb[threadIdx.x] = code >= 0 ? code : 0;
+        if (MULTI) s_nbc[threadIdx.x] = code >= 0 ? -1 : -code - 1;
+    }
+    const int bx0 = (int)(bid % g.nx), by0 = (int)((bid / g.nx) % g.ny), bz0 = (int)(bid / ((int64_t)g.nx * g.ny));
+    __syncthreads();
+    fill_block16<STENCIL, MULTI, TS, kSweepThreads, false>(g, c, fslab, bx0, by0, bz0, empty_f32, tile, s_nb, s_nbc,
+                                                           (int)threadIdx.x, [] { __syncthreads(); });
+    __syncthreads();
+    uint32_t sr_key = 0;
+    if constexpr (std::is_same<TS, uint8_t>::value) sr_key = sr_sweep_key(sr.seed, *sr.ctr);
+    update_block16<STENCIL, TS, kSweepThreads, false>(fslab, slot, bid, dt, clamp01, tile, sr_key, (int)threadIdx.x);
 }
 
 // One colour pass: workgroup k updates block bids[k] in place, its halo
@@ -577,6 +628,127 @@ __global__ __launch_bounds__(kSweepThreads) void sweep_kernel(GridView g, GridVi
 // Advances a Density8 plan's sweep counter (after the 8 colour passes).
 __global__ void sr_advance_kernel(uint32_t *ctr) {
     if (threadIdx.x == 0) *ctr += 1u;
+}
+
+// ---------------------------------------------------------------------------
+// Whole sweeps of a small band in one launch.  A colour pass over few blocks
+// is a chain of latencies (launch, topology row, tile loads, update), and the
+// next colour's launch waits for its last work-group: 6.1 us a colour on a
+// 128^3 shell (8 x 35 blocks).  Here a work-group takes the next block of the
+// plan's colour-major list (a ticket), reads its topology, waits until the
+// neighbours that precede the block have been updated, updates it (1,024 lanes)
+// and marks it done: 4.4 us a colour.
+//
+// Order.  Block b of sweep S (counted over the plan's life) follows its
+// neighbours of lower colour in sweep S and all other neighbours and itself in
+// sweep S - 1: with done[k] = sweeps block k has finished, it waits for
+// done >= S + 1 and done >= S.  Those are the values the colour passes give it
+// (blocks of one colour are never neighbours), so the results are the same bits.
+//
+// Every wait ends: the list has a block after all blocks it waits for in the
+// same sweep, sweeps follow each other, and tickets are handed out in that
+// order to work-groups that are already running.  The group with the lowest
+// unfinished ticket therefore waits only for finished blocks, whatever the
+// hardware's dispatch order and however many groups are resident.
+//
+// Visibility.  The 8 XCDs' L2s keep agent-scope atomics coherent, so cells are
+// read and written as such (ld_cell, st_cell); a group's stores have completed
+// (s_waitcnt) before its flag is stored, and a reader's loads are issued after
+// its waits.
+// ---------------------------------------------------------------------------
+struct FlowArgs {
+    const int32_t *dep;  // [n][27] list index of each neighbour in the plan, -1 none; [13] is the block itself
+    uint32_t *done;      // [n]
+    unsigned long long *ticket;  // over the plan's life
+    uint32_t n;          // blocks
+};
+constexpr int kFlowThreads = 1024;
+
+template <int STENCIL, bool MULTI, typename TS>
+__global__ __launch_bounds__(kFlowThreads) void sweep_flow_kernel(GridView g, GridView c, TS *fslab,
+                                                                  const int64_t *bids, const int32_t *topo,
+                                                                  FlowArgs f, float dt, int clamp01, float empty_f32,
+                                                                  SrCtx sr) {
+    constexpr int HALO = STENCIL == MSBG_BILAPLACIAN ? 2 : 1;
+    constexpr int NN = 2 * HALO + 1, NT = NN * NN * NN, CENTER = (NT - 1) / 2;
+    __shared__ __attribute__((aligned(16))) float tile[sweep_tile_floats<STENCIL>()];
+    __shared__ int s_nb[NT];
+    __shared__ int s_nbc[MULTI ? NT : 1];
+    __shared__ unsigned long long s_ticket;
+    const int t = (int)threadIdx.x;
+    if (t == 0) s_ticket = atomicAdd(f.ticket, 1ull);
+    __syncthreads();
+    const unsigned long long q = s_ticket;
+    uint32_t sweep, k;
+    if (q >> 32) {  // (a 64-bit division costs ~150 instructions)
+        sweep = (uint32_t)(q / f.n);
+        k = (uint32_t)(q % f.n);
+    } else {
+        sweep = (uint32_t)q / f.n;
+        k = (uint32_t)q - sweep * f.n;
+    }
+    // What is one value per group is kept in scalar registers, so the branches
+    // (and the barriers inside them) are taken by whole waves.
+    sweep = (uint32_t)__builtin_amdgcn_readfirstlane((int)sweep);
+    k = (uint32_t)__builtin_amdgcn_readfirstlane((int)k);
+    const uint32_t bid = (uint32_t)__builtin_amdgcn_readfirstlane((int)bids[k]);  // < 2^31 blocks
+    const int32_t *row = topo + (int64_t)k * NT;
+    const int slot = __builtin_amdgcn_readfirstlane(row[CENTER]);
+    const int yz = (int)(bid / (uint32_t)g.nx), bx = (int)(bid - (uint32_t)yz * (uint32_t)g.nx), bz = yz / g.ny,
+              by = yz - bz * g.ny;
+    int dep = -1;
+    uint32_t need = 0;
+    if (t < NT) {
+        const int code = row[t];
+        s_nb[t] = code >= 0 ? code : 0;
+        if constexpr (MULTI) s_nbc[t] = code >= 0 ? -1 : -code - 1;
+    }
+    if (t < 27) {
+        dep = f.dep[(int64_t)k * 27 + t];
+        const int own = (bx & 1) | (by & 1) << 1 | (bz & 1) << 2;
+        const int other = ((bx + t % 3 - 1) & 1) | ((by + (t / 3) % 3 - 1) & 1) << 1 | ((bz + t / 9 - 1) & 1) << 2;
+        need = sweep + (other < own ? 1u : 0u);
+    }
+    __syncthreads();
+    // each lane waits for one neighbour, then the whole group is let through
+    auto wait = [&] {
+        if (dep >= 0)
+            while ((int32_t)(__hip_atomic_load(f.done + dep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - need) < 0)
+                __builtin_amdgcn_s_sleep(1);
+        __syncthreads();
+    };
+    const bool live = slot >= 2;  // else dummy or absent: solver.rs:201-204
+    if (live)
+        fill_block16<STENCIL, MULTI, TS, kFlowThreads, true>(g, c, fslab, bx, by, bz, empty_f32, tile, s_nb, s_nbc, t,
+                                                             wait);
+    else
+        wait();
+    __syncthreads();
+    if (live) {
+        uint32_t sr_key = 0;
+        if constexpr (std::is_same<TS, uint8_t>::value) sr_key = sr_sweep_key(sr.seed, *sr.ctr);  // one sweep a launch
+        update_block16<STENCIL, TS, kFlowThreads, true>(fslab, slot, bid, dt, clamp01, tile, sr_key, t);
+    }
+    __builtin_amdgcn_s_waitcnt(0);  // this lane's stores have completed
+    __syncthreads();
+    if (t == 0) __hip_atomic_store(f.done + k, sweep + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Plan index of each block id, and from it each planned block's 27 neighbours.
+__global__ void flow_index_kernel(const int64_t *__restrict__ bids, int64_t n, int32_t *index) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) index[bids[i]] = (int32_t)i;
+}
+__global__ void flow_dep_kernel(const int64_t *__restrict__ bids, int64_t n, int nx, int ny, int nz,
+                                const int32_t *__restrict__ index, int32_t *__restrict__ dep) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n * 27) return;
+    const int64_t bid = bids[i / 27];
+    const int t = (int)(i % 27);
+    const int x = (int)(bid % nx) + t % 3 - 1, y = (int)((bid / nx) % ny) + (t / 3) % 3 - 1,
+              z = (int)(bid / ((int64_t)nx * ny)) + t / 9 - 1;
+    dep[i] = x >= 0 && x < nx && y >= 0 && y < ny && z >= 0 && z < nz ? index[x + (int64_t)nx * (y + (int64_t)ny * z)]
+                                                                      : -1;
 }
 
 // ---------------------------------------------------------------------------
@@ -800,6 +972,9 @@ struct msbg_sweep_plan {
     uint8_t *slab8 = nullptr;    // Density8 (u8) storage over g's layout, or null
     uint32_t sr_seed = 0;        // Density8: stochastic-rounding seed
     uint32_t *d_sr_ctr = nullptr;  // Density8: sweeps done by this plan (device)
+    // One-launch sweeps (sweep_flow_kernel): n = 0 when the plan has none
+    // (all-level plans, large bands, repeated block ids).
+    msbg::FlowArgs flow{nullptr, nullptr, nullptr, 0};
     // All-level plans (msbg_sweep_plan_new_levels): g / coarse are levels 0
     // and 1, d_bids / d_topo / counts the level-0 blocks; the coarse blocks
     // are d_cbids (colour-major, then level, then Morton order) with 27-entry
@@ -886,8 +1061,56 @@ int build_topology(const msbg_grid *g, const msbg_grid *coarse, const uint8_t *d
     return MSBG_OK;
 }
 
+// Bands of at most this many blocks sweep in one launch: a curvature and a
+// bi-Laplacian sweep of 280 / 608 / 1,112 / 1,976 / 4,688 blocks take 69 / 93 /
+// 104 / 125 / 199 us that way and 98 / 104 / 107 / 119 / 182 us as colour passes,
+// where each colour has enough blocks to fill the chip and a waiting group
+// would only hold a CU's lanes.
+constexpr int64_t kFlowMost = 1024;
+
+// The neighbour table and counters of a plan's one-launch sweeps (`order`:
+// its blocks, colour-major).
+int build_flow(msbg_sweep_plan *p, const std::vector<int64_t> &order) {
+    const msbg_grid *g = p->g;
+    const int64_t n = p->n;
+    if (n > kFlowMost) return MSBG_OK;
+    int64_t off = 0;
+    for (int c = 0; c < 8; ++c) {  // a repeated id has no place in the order: such plans keep the colour passes
+        for (int64_t i = 1; i < p->counts[c]; ++i)
+            if (order[(size_t)(off + i)] == order[(size_t)(off + i - 1)]) return MSBG_OK;
+        off += p->counts[c];
+    }
+    // one allocation: ticket, done, dep; the plan index of each block id is scratch
+    const size_t at_done = sizeof(unsigned long long), at_dep = at_done + sizeof(uint32_t) * (size_t)n;
+    char *mem = nullptr;
+    MSBG_HIP(hipMalloc(&mem, at_dep + sizeof(int32_t) * 27 * (size_t)n));
+    int rc = MSBG_OK;
+    int32_t *index = (int32_t *)workspace(21, sizeof(int32_t) * (size_t)g->n_blocks, &rc);
+    if (rc) {
+        (void)hipFree(mem);
+        return rc;
+    }
+    hipError_t e = hipMemsetAsync(mem, 0, at_dep, stream());
+    if (e == hipSuccess) e = hipMemsetAsync(index, 0xff, sizeof(int32_t) * (size_t)g->n_blocks, stream());
+    if (e == hipSuccess) {
+        flow_index_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream()>>>(p->d_bids, n, index);
+        flow_dep_kernel<<<(unsigned)((n * 27 + 255) / 256), 256, 0, stream()>>>(
+            p->d_bids, n, (int)g->nx, (int)g->ny, (int)g->nz, index, (int32_t *)(mem + at_dep));
+        e = hipGetLastError();
+    }
+    if (e != hipSuccess) {
+        (void)hipFree(mem);
+        return hip_fail(e, "sweep plan neighbours");
+    }
+    p->flow.ticket = (unsigned long long *)mem;
+    p->flow.done = (uint32_t *)(mem + at_done);
+    p->flow.dep = (const int32_t *)(mem + at_dep);
+    p->flow.n = (uint32_t)n;
+    return MSBG_OK;
+}
+
 int plan_new(msbg_grid *g, const msbg_grid *coarse, const uint8_t *d_levels, const int64_t *active, int64_t n,
-             msbg_sweep_plan **out) {
+             msbg_sweep_plan **out, bool flow = true) {
     MSBG_CHECK(out, MSBG_EINVAL, "null out");
     *out = nullptr;
     MSBG_CHECK(g && g->L == 4, MSBG_EINVAL, "sweeps run on 16^3-block grids");
@@ -919,6 +1142,7 @@ int plan_new(msbg_grid *g, const msbg_grid *coarse, const uint8_t *d_levels, con
         }
         rc = build_topology(g, coarse, d_levels, p->d_bids, n, 1, p->d_topo[1]);
         if (rc == MSBG_OK) rc = build_topology(g, coarse, d_levels, p->d_bids, n, 2, p->d_topo[2]);
+        if (rc == MSBG_OK && flow) rc = build_flow(p, order);
         if (rc == MSBG_OK) {
             e = hipStreamSynchronize(stream());
             if (e != hipSuccess) rc = hip_fail(e, "sweep plan topology");
@@ -995,6 +1219,50 @@ int launch_sweep(msbg_sweep_plan *p, hipStream_t s, int stencil, float dt, int c
     return MSBG_OK;
 }
 
+template <int STENCIL, bool MULTI, typename TS>
+int launch_flow_st(msbg_sweep_plan *p, hipStream_t s, TS *fslab, float dt, int clamp01, unsigned sweeps) {
+    constexpr int halo = STENCIL == MSBG_BILAPLACIAN ? 2 : 1;
+    GridView g = p->g->view(), c = MULTI ? p->coarse->view() : g;
+    const float empty_f32 = MULTI || sizeof(TS) != sizeof(float) ? 0.0f : p->g->empty_value;
+    const SrCtx sr{p->sr_seed, p->d_sr_ctr};
+    sweep_flow_kernel<STENCIL, MULTI, TS><<<p->flow.n * sweeps, kFlowThreads, 0, s>>>(
+        g, c, fslab, p->d_bids, p->d_topo[halo], p->flow, dt, clamp01, empty_f32, sr);
+    MSBG_HIP(hipGetLastError());
+    return MSBG_OK;
+}
+
+template <bool MULTI, typename TS>
+int launch_flow(msbg_sweep_plan *p, hipStream_t s, TS *fslab, int stencil, float dt, int clamp01, unsigned sweeps) {
+    if (stencil == MSBG_LAPLACIAN) return launch_flow_st<MSBG_LAPLACIAN, MULTI, TS>(p, s, fslab, dt, clamp01, sweeps);
+    if (stencil == MSBG_MEAN_CURVATURE)
+        return launch_flow_st<MSBG_MEAN_CURVATURE, MULTI, TS>(p, s, fslab, dt, clamp01, sweeps);
+    return launch_flow_st<MSBG_BILAPLACIAN, MULTI, TS>(p, s, fslab, dt, clamp01, sweeps);
+}
+
+// `iterations` sweeps as one launch (Density8: one a sweep, whose number keys
+// its rounding), or several when their blocks would exceed 2^24.
+int launch_flow_sweeps(msbg_sweep_plan *p, hipStream_t s, int stencil, float dt, int iterations, int clamp01) {
+    const int most = p->slab8 ? 1 : (int)(((int64_t)1 << 24) / p->flow.n);
+    for (int it = 0; it < iterations; it += most) {
+        const unsigned sweeps = (unsigned)std::min(most, iterations - it);
+        int rc;
+        if (p->coarse)
+            rc = launch_flow<true, float>(p, s, p->g->d_slab, stencil, dt, clamp01, sweeps);
+        else if (p->slab16)
+            rc = launch_flow<false, uint16_t>(p, s, p->slab16, stencil, dt, clamp01, sweeps);
+        else if (p->slab8)
+            rc = launch_flow<false, uint8_t>(p, s, p->slab8, stencil, dt, clamp01, sweeps);
+        else
+            rc = launch_flow<false, float>(p, s, p->g->d_slab, stencil, dt, clamp01, sweeps);
+        if (rc) return rc;
+        if (p->slab8) {
+            hipLaunchKernelGGL(sr_advance_kernel, dim3(1), dim3(64), 0, s, p->d_sr_ctr);
+            MSBG_HIP(hipGetLastError());
+        }
+    }
+    return MSBG_OK;
+}
+
 // The 8 colour passes of an all-level plan: one launch per colour covers
 // the level-0 blocks and the coarse work items of that colour.
 int launch_sweep_levels(msbg_sweep_plan *p, hipStream_t s, int stencil, float dt, int clamp01,
@@ -1053,6 +1321,7 @@ int launch_iterations(msbg_sweep_plan *p, hipStream_t s, int stencil, float dt, 
     MSBG_CHECK(!(p->has_edge1 && stencil == MSBG_BILAPLACIAN), MSBG_EINVAL,
                "the radius-2 bi-Laplacian needs blocks of edge >= 2 (a level-4 halo would reach past its "
                "neighbour blocks)");
+    if (p->flow.n && !ev) return launch_flow_sweeps(p, s, stencil, dt, iterations, clamp01);
     for (int it = 0; it < iterations; ++it) {
         int rc = p->n_levels ? launch_sweep_levels(p, s, stencil, dt, clamp01, ev)
                  : p->coarse ? launch_sweep<true>(p, s, stencil, dt, clamp01, ev)
@@ -1099,7 +1368,7 @@ int plan_new_levels(msbg_grid *const *grids, int n_levels, const uint8_t *d_leve
         coarse[color][l].push_back({spread21(bx) | (spread21(by) << 1) | (spread21(bz) << 2), (int32_t)bid});
     }
     msbg_sweep_plan *p = nullptr;
-    int rc = plan_new(grids[0], grids[1], d_levels, fine.data(), (int64_t)fine.size(), &p);
+    int rc = plan_new(grids[0], grids[1], d_levels, fine.data(), (int64_t)fine.size(), &p, false);
     if (rc) return rc;
     p->n_levels = n_levels;
     for (int l = 0; l < n_levels; ++l) p->lv[l] = grids[l];
@@ -1312,6 +1581,7 @@ int msbg_sweep_plan_free(msbg_sweep_plan *p) {
     for (int32_t *t : p->d_topo)
         if (t) (void)hipFree(t);
     if (p->d_sr_ctr) (void)hipFree(p->d_sr_ctr);
+    if (p->flow.ticket) (void)hipFree(p->flow.ticket);
     if (p->d_cbids) (void)hipFree(p->d_cbids);
     if (p->d_ctopo) (void)hipFree(p->d_ctopo);
     for (CoarseItem *it : p->d_items)
@@ -1334,6 +1604,8 @@ int msbg_sweep_plan_run_graph_async(msbg_sweep_plan *p, int stencil, float dt, i
     if (rc) return rc;
     MSBG_CHECK(iterations >= 0, MSBG_EINVAL, "negative iterations");
     if (iterations == 0 || p->n == 0) return MSBG_OK;
+    // one launch needs no graph
+    if (p->flow.n && !p->slab8) return launch_iterations(p, stream(), stencil, dt, iterations, clamp01);
     // a hit, else an empty entry, else the least recently used one
     msbg_sweep_plan::GraphEntry *hit = nullptr, *lru = nullptr;
     for (auto &e : p->graphs) {

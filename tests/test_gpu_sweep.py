@@ -393,3 +393,57 @@ def test_density_sweep_bitexact(pkg, orc, hip, stencil, dt, s):
     hip.synchronize()
     hip.call("msbg_sweep_plan_free", plan)
     assert np.array_equal(d2.get(), want)
+
+
+def shuffled_plan_problem(pkg, n, shape, seed):
+    """`n` value blocks of a random grid in random order, the rest of the grid
+    value, full and empty blocks."""
+    g = random_grid(pkg, *shape, seed=seed, frac=1.0 if n < 100 else 0.7, lo=0.0, hi=1.0)
+    rng = np.random.default_rng(seed)
+    active = np.nonzero(g.b2s >= 2)[0].astype(np.int64)
+    assert active.size >= n
+    active = rng.permutation(active)[:n]
+    return g, active
+
+
+@pytest.mark.parametrize("stencil,dt", [(0, 0.1), (1, 0.02), (2, 0.005)])
+@pytest.mark.parametrize("n,shape", [(1, (16, 16, 16)), (1, (9, 9, 9)), (27, (48, 41, 35)), (60, (32, 33, 16 * 64)),
+                                     (1023, (208, 193, 181)), (1024, (208, 193, 181)), (1025, (208, 193, 181))])
+def test_one_launch_sweeps_equal_the_colour_passes(pkg, hip, stencil, dt, n, shape):
+    """run_async and run_graph_async (one launch up to 1,024 blocks) against
+    run_timed (a launch per colour): 1, 3 and 2 sweeps in a row without a
+    synchronisation, bit for bit; domains whose halo mirrors inside one block."""
+    g, active = shuffled_plan_problem(pkg, n, shape, 100 + n)
+    ga, gb = pkg.DeviceGrid.from_host(g, lib=hip), pkg.DeviceGrid.from_host(g, lib=hip)
+    pa, pb = pkg.SweepPlan(ga, active), pkg.SweepPlan(gb, active)
+    for it, graph in ((1, False), (3, True), (2, False)):
+        (pa.run_graph_async if graph else pa.run_async)(stencil, dt, it, True)
+    for it in (1, 3, 2):
+        pb.run_timed(stencil, dt, it, True)
+    hip.synchronize()
+    assert_bitexact(ga.to_host().slab, gb.to_host().slab, "one launch against colour passes")
+
+
+def test_one_launch_sweeps_of_many_iterations(pkg, hip):
+    """200 sweeps of 800 blocks in one launch (the flags' longest chain in the
+    tests) against 200 rounds of colour passes, u16 and FP32 storage."""
+    import ctypes as C
+    g, active = shuffled_plan_problem(pkg, 800, (176, 176, 160), 5)
+    ga, gb = pkg.DeviceGrid.from_host(g, lib=hip), pkg.DeviceGrid.from_host(g, lib=hip)
+    pkg.SweepPlan(ga, active).run_async(1, 0.02, 200, True)
+    pkg.SweepPlan(gb, active).run_timed(1, 0.02, 200, True)
+    assert_bitexact(ga.to_host().slab, gb.to_host().slab, "200 sweeps")
+    q = (np.clip(g.slab, 0, 1) * 65535).astype(np.uint16)
+    out = []
+    for timed in (False, True):
+        d, plan = hip.to_device(q), C.c_void_p()
+        hip.call("msbg_sweep_plan_new_density", ga.h, d.ptr, active.ctypes.data, active.size, C.byref(plan))
+        if timed:
+            ms, k = C.c_float(), C.c_int64()
+            hip.call("msbg_sweep_plan_run_timed", plan, 2, 0.005, 50, 1, C.byref(ms), C.byref(k))
+        else:
+            hip.call("msbg_sweep_plan_run_async", plan, 2, 0.005, 50, 1)
+        hip.synchronize()
+        hip.call("msbg_sweep_plan_free", plan)
+        out.append(d.get())
+    assert np.array_equal(out[0], out[1])
