@@ -4,10 +4,10 @@
 //    with gather_map (math/gather.rs:54-158), per particle, plus the MAC
 //    face sampler (fluid/g2p.rs:26-32) and the FLIP/PIC blend (g2p.rs:42-45).
 //  * MAC P2G of the reference (fluid/p2g.rs:141-412): particles bucketed by
-//    block; per face direction and colour one launch, each workgroup stages
-//    its block's (16+2m)^3 window in LDS (mass + momentum) and commits the 27
-//    regions to the grid; blocks of one colour never overlap, so the commit
-//    needs no global atomics.  Then u = P/M (mac.rs:106-132).
+//    block; per face direction each workgroup stages a block's particles in
+//    its (16+2m)^3 window in LDS (mass + momentum) and writes the window out,
+//    then every cell adds the windows that cover it, in a fixed order, and
+//    divides, u = P/M (mac.rs:106-132).
 //  * B-spline P2G / G2P (trilinear, quadratic): particles Morton-sorted by
 //    voxel; every cell gathers its 27 neighbour voxels in a fixed order, so
 //    the result is deterministic and needs neither atomics nor colouring.
@@ -210,36 +210,33 @@ __global__ void g2p_flip_kernel(MacViews u, MacViews ut, const float *__restrict
 // ---------------------------------------------------------------------------
 // Reference MAC P2G (fluid/p2g.rs:221-412).
 // ---------------------------------------------------------------------------
-__global__ void bucket_keys_kernel(const float *__restrict__ pos, int64_t n, int32_t nx, int32_t ny,
-                                   uint32_t *__restrict__ keys, uint32_t *__restrict__ idx) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const uint32_t x = trunc_index(pos[3 * i]), y = trunc_index(pos[3 * i + 1]), z = trunc_index(pos[3 * i + 2]);
-        keys[i] = (x >> 4) + (y >> 4) * (uint32_t)nx + (z >> 4) * (uint32_t)nx * (uint32_t)ny;
-        idx[i] = (uint32_t)i;
-    }
-}
-
 __global__ void set_flag_kernel(int32_t *p, int32_t v) { *p = v; }
 
-// bucket_keys_kernel, and *ungrouped set to 1 when some particle's block
-// precedes the previous particle's in Morton order: otherwise (Morton-sorted
-// input) each block's particles already form one run in input order, which is
-// the order the stable bucket sort gives within a block.
+__global__ void fill_i32_kernel(int32_t *p, int64_t n, int32_t v) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        p[i] = v;
+}
+
+// Block ids as keys, at most `most` (particles far outside the domain), and
+// *ungrouped set to 1 when some particle's block precedes the previous
+// particle's in Morton order or lies past 1,023 on an axis: otherwise
+// (Morton-sorted input) each block's particles already form one run in input
+// order, which is the order the stable bucket sort gives within a block.
 __global__ void bucket_keys_grouped_kernel(const float *__restrict__ pos, int64_t n, int32_t nx, int32_t ny,
-                                           uint32_t *__restrict__ keys, uint32_t *__restrict__ idx,
+                                           uint32_t most, uint32_t *__restrict__ keys, uint32_t *__restrict__ idx,
                                            int32_t *__restrict__ ungrouped) {
     auto mblock = [](uint32_t x, uint32_t y, uint32_t z) {
         return spread10(x >> 4) | (spread10(y >> 4) << 1) | (spread10(z >> 4) << 2);
     };
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         const uint32_t x = trunc_index(pos[3 * i]), y = trunc_index(pos[3 * i + 1]), z = trunc_index(pos[3 * i + 2]);
-        keys[i] = (x >> 4) + (y >> 4) * (uint32_t)nx + (z >> 4) * (uint32_t)nx * (uint32_t)ny;
+        keys[i] = min((x >> 4) + (y >> 4) * (uint32_t)nx + (z >> 4) * (uint32_t)nx * (uint32_t)ny, most);
         idx[i] = (uint32_t)i;
-        bool down = false;
+        bool down = ((x | y | z) >> 14) != 0;
         if (i > 0) {
             const uint32_t px = trunc_index(pos[3 * i - 3]), py = trunc_index(pos[3 * i - 2]),
                            pz = trunc_index(pos[3 * i - 1]);
-            down = mblock(x, y, z) < mblock(px, py, pz);
+            down = down || mblock(x, y, z) < mblock(px, py, pz);
         }
         if (__any(down) && (threadIdx.x & 63) == 0) *ungrouped = 1;  // one store per wave
     }
@@ -261,227 +258,88 @@ __global__ void gather_payload_kernel(const float *__restrict__ pos, const float
     }
 }
 
-// A work item of the MAC splat: particles p0 .. p1 - 1 (sorted) of occupied
-// block k; `shared` when the block's particles are split over several items.
+// A work item of the MAC splat: particles p0 .. p1 - 1 (sorted) of block bid.
 struct SplatItem {
-    int32_t k, p0, p1, shared;
+    int32_t bid, p0, p1;
 };
-constexpr int kSplatThreads = 1024;  // one group per CU holds the 144 KB window of r_p <= 2: 16 waves
-constexpr int kSplatChunk = 4096;  // particles per item (4 per lane)
+constexpr int kSplatThreads = 1024;  // one group per CU holds the 128 KB window of r_p <= 2: 16 waves
+// Particles per item: an item per CU, at most 16,384 and not below 256, where a
+// window's clearing and writing outweigh its particles (100,000 particles in 48
+// blocks: 20 + 14 us a direction for splat and commit, 25 + 23 with two items
+// per CU).
+constexpr int kSplatMost = 16384, kSplatLeast = 256, kSplatItems = 256;
+constexpr int kSplatMaxCells = 8192;  // window cells of the two-channel kernels (m <= 2: 20^3)
 
-// Sum over the work-group (every thread receives it); s_red holds one slot per wave.
-__device__ __forceinline__ float splat_wg_sum(float v, float *s_red) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    float t = 0.0f;
-    for (int w = 0; w < kSplatThreads / 64; ++w) t += s_red[w];
-    __syncthreads();
-    return t;
-}
-
-// One (direction a, colour) pass of the MAC splat (p2g.rs:261-333):
-// workgroup i stages the particles of items[i] into its window and commits
-// it (with global atomics when other items of the same colour pass share the
-// block).  CH 0 splats the mass m w, CH 1 the momentum m u_a w, CH 2 both.
+// One face direction of the MAC splat (p2g.rs:261-333): work-group i adds up
+// the particles of items[i] in its (16 + 2m)^3 window and writes the window's
+// (mass, momentum) pairs to win + i (16 + 2m)^3 (mac_commit_kernel adds the
+// windows up): first the 16 middle cells of every row, then the rows' m cells
+// below, then those above, so that a reader of a margin takes whole lines.
+// CH 0 splats the mass m w, CH 1 the momentum m u_a w, CH 2 both.
 //
-// The window accumulates in fixed point: with B >= the item's sum of
-// |contribution| and B < 2^e, every contribution c is scaled by 2^S,
-// S = 61 - e, so |window sum| 2^S < 2^61.  A scaled contribution of
-// magnitude >= 2^24 is an integer in float, and its int64 LDS add is exact:
-// those sums carry no rounding and do not depend on order.  The rare smaller
-// ones (below ~2^-37 B: a particle at the edge of a cell's support) are added
-// in float: into a float window (CH 0 / 1), or (CH 2, where two int64
-// windows leave no room for it) into a list of kResCap entries applied at the
-// commit; past kResCap they are rounded to the fixed-point grid (absolute
-// error <= 2^-S-1 each).  The commit adds (double) acc 2^-S + the float part,
-// rounded once.  Integer LDS atomics run ~3x faster than float ones here.
-constexpr int kResCap = 2048;
-constexpr int kSplatMaxCells = 8192;  // window cells of CH 2 (m <= 2: 20^3)
-
-// |q| of an integral float, 2^24 <= |q| < 2^62, as a 64-bit integer:
-// |q| = t 2^32 + lo with t = trunc(|q| 2^-32) and 0 <= lo < 2^32, both exact
-// in float (below 2^32 lo is |q| itself; above, the ulp of |q| is >= 2^9, so
-// lo needs at most 23 bits).
-__device__ __forceinline__ unsigned long long integral_mag_u64(float q) {
-    const float a = fabsf(q);
-    const float t = truncf(a * 0x1p-32f);
-    const float lo = __builtin_fmaf(t, -0x1p32f, a);
-    return (unsigned long long)(uint32_t)t << 32 | (unsigned long long)(uint32_t)lo;
-}
-
-// AT is the face direction when it is a template constant (the one-pass
-// CH 2 kernels), or -1 when it comes in `a_rt`.
+// The window holds float64 sums of the float contributions w m and w (m u_a)
+// (16,384 of one sign lose at most 2^-39 of their sum), so it needs no scale,
+// and NaN and infinities propagate as in a float sum.  It is bound by its LDS
+// adds: 8.4 ns a wave and CU for float64 at random cells.  int64 adds of a
+// fixed-point window take 4.4 ns, but small contributions (a slow particle
+// beside a fast one, the edge of a support) don't fit one scale, and the
+// special path that they need cost six times the adds.
+//
+// AT is the face direction when it is a template constant (the two-channel
+// kernels), or -1 when it comes in `a_rt`.
 template <int CH, int AT>
-__global__ __launch_bounds__(kSplatThreads) void mac_splat_kernel(GridView gm, GridView gv, int a_rt,
+__global__ __launch_bounds__(kSplatThreads) void mac_splat_kernel(int nx, int ny, int a_rt,
                                                                   const SplatItem *__restrict__ items,
-                                                                  const int32_t *__restrict__ pblocks,
                                                                   const float *__restrict__ spos,
                                                                   const float *__restrict__ svel,
                                                                   const float *__restrict__ smass, float r_p,
-                                                                  float inv_r2, int m) {
-    extern __shared__ __attribute__((aligned(8))) unsigned char smem_raw[];
-    __shared__ float s_red[kSplatThreads / 64];
-    __shared__ int s_nres;
-    __shared__ int s_slot[2][27];  // mass / velocity slot of each committed region, -1 where not committed
+                                                                  float inv_r2, int m, float2 *__restrict__ win) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     constexpr int NC = CH == 2 ? 2 : 1;  // channels of this pass
     const int a = AT >= 0 ? AT : a_rt;
     const int MSX = 16 + 2 * m, NS = MSX * MSX * MSX;
-    unsigned long long *acc = reinterpret_cast<unsigned long long *>(smem_raw);  // NC windows
-    float *res = reinterpret_cast<float *>(acc + NC * NS);                         // CH 0 / 1: float window
-    uint2 *rlist = reinterpret_cast<uint2 *>(acc + NC * NS);                       // CH 2: (cell | channel << 31, value)
-    for (int s = threadIdx.x; s < NC * NS; s += blockDim.x) acc[s] = 0ull;
-    if (CH != 2)
-        for (int s = threadIdx.x; s < NS; s += blockDim.x) res[s] = 0.0f;
-    if (threadIdx.x == 0) s_nres = 0;
+    double *acc = reinterpret_cast<double *>(smem_raw);  // NC windows
+    for (int s = threadIdx.x; s < NC * NS / 2; s += kSplatThreads)
+        reinterpret_cast<double2 *>(acc)[s] = make_double2(0.0, 0.0);
     const SplatItem item = items[blockIdx.x];
-    const int bid = pblocks[item.k];
-    const int bx = bid % gm.nx, by = (bid / gm.nx) % gm.ny, bz = bid / (gm.nx * gm.ny);
+    const int bx = item.bid % nx, by = (item.bid / nx) % ny, bz = item.bid / (nx * ny);
     const int b0x = bx * 16, b0y = by * 16, b0z = bz * 16;
     const int x0s = b0x - m, y0s = b0y - m, z0s = b0z - m, whi = 16 + m - 1;
     const float ofx = a == 0 ? 1.0f : 0.5f, ofy = a == 1 ? 1.0f : 0.5f, ofz = a == 2 ? 1.0f : 0.5f;
-    if (threadIdx.x < 27) {
-        // Commit regions (p2g.rs:342-411): window region (rx, ry, rz) is the
-        // margin below, the block's own 16 cells or the margin above on each
-        // axis; it is committed when it lies inside the domain and its block
-        // holds both a mass and a velocity slot.
-        const int t = threadIdx.x, rx = t % 3, ry = (t / 3) % 3, rz = t / 9;
-        const int xlo = rx == 0 ? 0 : (rx == 1 ? m : m + 16), xlen = rx == 1 ? 16 : m;
-        const int ylo = ry == 0 ? 0 : (ry == 1 ? m : m + 16), ylen = ry == 1 ? 16 : m;
-        const int zlo = rz == 0 ? 0 : (rz == 1 ? m : m + 16), zlen = rz == 1 ? 16 : m;
-        const int gx0 = x0s + xlo, gy0 = y0s + ylo, gz0 = z0s + zlo;
-        int ms = -1, vs = -1;
-        if (gx0 >= 0 && gy0 >= 0 && gz0 >= 0 && gx0 + xlen <= gm.sx && gy0 + ylen <= gm.sy && gz0 + zlen <= gm.sz) {
-            const int64_t nb = (int64_t)(bx + rx - 1) + (int64_t)(by + ry - 1) * gm.nx +
-                               (int64_t)(bz + rz - 1) * gm.nx * gm.ny;
-            ms = gm.b2s[nb];
-            vs = gv.b2s[nb];
-            if (ms < 2 || vs < 2) ms = vs = -1;
-        }
-        s_slot[0][t] = ms;
-        s_slot[1][t] = vs;
-    }
-    // Lane t takes a contiguous run of the item's particles.
-    const int p_beg = item.p0, p_cnt = item.p1 - item.p0;
-    const int per = (p_cnt + (int)blockDim.x - 1) / (int)blockDim.x;
-    // channel k of this pass is the mass when CH is 0, or CH is 2 and k is 0
-    auto is_mass = [](int k) { return CH == 2 ? k == 0 : CH == 0; };
-    auto scale_of = [&](int pi, int k) { return is_mass(k) ? smass[pi] : smass[pi] * svel[3 * pi + a]; };
-    // A particle whose mass or mass * velocity is not finite stays out of the
-    // fixed-point window (its sum has no scale); it is added in float after
-    // the commit, so only its own footprint turns non-finite.
-    float bsum[NC];
-    bool nonfin = false;
-#pragma unroll
-    for (int k = 0; k < NC; ++k) bsum[k] = 0.0f;
-    for (int j = 0; j < per; ++j) {
-        const int pi = p_beg + (int)threadIdx.x * per + j;
-        if (pi < p_beg + p_cnt)
-#pragma unroll
-            for (int k = 0; k < NC; ++k) {
-                const float v = scale_of(pi, k);
-                if (isfinite(v))
-                    bsum[k] += fabsf(v);
-                else
-                    nonfin = true;
-            }
-    }
-    // w <= 1; the FP32 sum of the bounds is within a factor 1 + 2^-12 of its
-    // value, and e leaves a factor 2 spare.
-    float up[NC];
-    int ex[NC];
-    bool any = false;
-#pragma unroll
-    for (int k = 0; k < NC; ++k) {
-        const float bound = splat_wg_sum(bsum[k], s_red);
-        any = any || bound > 0.0f;
-        frexpf(bound > 0.0f && isfinite(bound) ? bound : 1.0f, &ex[k]);  // bound < 2^e
-        // S = 61 - e, at most 126: 2^S stays a float, and a contribution
-        // reaching 2^24 after scaling comes from a normal float
-        ex[k] = max(ex[k], 61 - 126);
-        up[k] = ldexpf(1.0f, 61 - ex[k]);  // 2^S
-    }
-    const bool item_nonfin = splat_wg_sum(nonfin ? 1.0f : 0.0f, s_red) > 0.0f;  // uniform per group
-    // S >= 0 on every channel: a finite nonzero scale times 2^S is nonzero,
-    // so a zero scaled contribution is a zero contribution
-    bool unit_scales = true;
-#pragma unroll
-    for (int k = 0; k < NC; ++k) unit_scales = unit_scales && ex[k] <= 61;
-    // Nothing but zero contributions: the item adds nothing.  Uniform per group.
-    if (!any && !item_nonfin) return;
-    constexpr float kExact = 16777216.0f;  // 2^24
-    auto footprint = [&](int pi, int &ix1, int &ix2, int &iy1, int &iy2, int &iz1, int &iz2) {
-        const float px = spos[3 * pi], py = spos[3 * pi + 1], pz = spos[3 * pi + 2];
-        ix1 = min(max((int)ceilf(px - r_p - ofx), b0x - m), b0x + whi);
-        ix2 = min(max((int)floorf(px + r_p - ofx), b0x - m), b0x + whi);
-        iy1 = min(max((int)ceilf(py - r_p - ofy), b0y - m), b0y + whi);
-        iy2 = min(max((int)floorf(py + r_p - ofy), b0y - m), b0y + whi);
-        iz1 = min(max((int)ceilf(pz - r_p - ofz), b0z - m), b0z + whi);
-        iz2 = min(max((int)floorf(pz + r_p - ofz), b0z - m), b0z + whi);
-    };
-    // Eq. 6 weight of face cell (ix, iy, iz) for the particle at p0 = p - 1/2.
-    auto weight = [&](float px0, float py0, float pz0, int ix, int iy, int iz) {
-        const float dz = (float)iz - pz0, dy = (float)iy - py0, dx = (float)ix - px0;
-        const float dist_sq = dx * dx + (dz * dz + dy * dy);
-        const float d_a = a == 0 ? dx : (a == 1 ? dy : dz);
-        const float df2 = dist_sq + d_a + 0.25f;
-        const float w = fmaxf(1.0f - df2 * inv_r2, 0.0f);
-        return w * w * w;
-    };
-    // One contribution w * sc[k] of a particle whose scales are finite (sf =
-    // sc, sq = sc 2^S; both 0 for a non-finite channel).  q = w sq equals
-    // (w sc) 2^S bit for bit whenever |q| >= 2^24 (2^S is a power of two and
-    // w sc is then a normal float), so the window receives the same integers
-    // as from scaling the float contribution.
-    auto contrib = [&](int cell, float w, const float *sf, const float *sq) {
+    const int cnt = item.p1 - item.p0;
+    __syncthreads();
+    // A wave takes 64 particles, `chunks` apart: particles sorted along a curve
+    // share cells with their successors, and adds of one wave to one address
+    // run one after the other (67 M particles: 2.8 ms a direction and half of
+    // them with neighbouring particles in neighbouring lanes, 2.3 so).
+    const int chunks = (cnt + 63) >> 6, lane = threadIdx.x & 63;
+    for (int t = threadIdx.x >> 6; t < chunks; t += kSplatThreads / 64) {
+        const int q = lane * chunks + t;
+        if (q >= cnt) continue;
+        const int pi = item.p0 + q;
+        float sc[NC];
+        bool fin = true, live = false;
 #pragma unroll
         for (int k = 0; k < NC; ++k) {
-            const float q = w * sq[k];
-            if (fabsf(q) >= kExact) {
-                const unsigned long long u = integral_mag_u64(q);
-                if (q > 0.0f)
-                    atomicAdd(&acc[k * NS + cell], u);
-                else
-                    __hip_atomic_fetch_sub(&acc[k * NS + cell], u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            } else {
-                const float c = w * sf[k];
-                if (c == 0.0f) continue;  // +-0 keeps the value
-                if (CH != 2) {
-                    atomicAdd(&res[cell], c);
-                } else {
-                    const int slot = atomicAdd(&s_nres, 1);
-                    if (slot < kResCap)
-                        rlist[slot] = make_uint2((uint32_t)cell | (uint32_t)k << 31, __float_as_uint(c));
-                    else
-                        atomicAdd(&acc[k * NS + cell], (unsigned long long)llrintf(c * up[k]));
-                }
-            }
-        }
-    };
-    for (int j = 0; j < per; ++j) {
-        const int pi = p_beg + (int)threadIdx.x * per + j;
-        if (pi >= p_beg + p_cnt) break;
-        float sf[NC], sq[NC];
-        unsigned long long sgn[NC];  // all ones where the channel's contributions are negative
-        bool live = false;
-#pragma unroll
-        for (int k = 0; k < NC; ++k) {
-            const float v = scale_of(pi, k);
-            const bool fin = isfinite(v);  // non-finite: added after the commit
-            sf[k] = fin ? v : 0.0f;
-            sq[k] = fin ? v * up[k] : 0.0f;
-            sgn[k] = sq[k] < 0.0f ? ~0ull : 0ull;
-            live = live || (fin && v != 0.0f);
+            // channel k of this pass is the mass when CH is 0, or CH is 2 and k is 0
+            sc[k] = (CH == 2 ? k == 0 : CH == 0) ? smass[pi] : smass[pi] * svel[3 * pi + a];
+            fin = fin && isfinite(sc[k]);
+            live = live || sc[k] != 0.0f;
         }
         if (!live) continue;
-        const float px0 = spos[3 * pi] - 0.5f, py0 = spos[3 * pi + 1] - 0.5f, pz0 = spos[3 * pi + 2] - 0.5f;
-        int ix1, ix2, iy1, iy2, iz1, iz2;
-        footprint(pi, ix1, ix2, iy1, iy2, iz1, iz2);
-        if (AT >= 0 && unit_scales && ix2 - ix1 <= 3 && iy2 - iy1 <= 3 && iz2 - iz1 <= 3) {
+        const float px = spos[3 * pi], py = spos[3 * pi + 1], pz = spos[3 * pi + 2];
+        const float px0 = px - 0.5f, py0 = py - 0.5f, pz0 = pz - 0.5f;
+        const int ix1 = min(max((int)ceilf(px - r_p - ofx), x0s), b0x + whi);
+        const int ix2 = min(max((int)floorf(px + r_p - ofx), x0s), b0x + whi);
+        const int iy1 = min(max((int)ceilf(py - r_p - ofy), y0s), b0y + whi);
+        const int iy2 = min(max((int)floorf(py + r_p - ofy), y0s), b0y + whi);
+        const int iz1 = min(max((int)ceilf(pz - r_p - ofz), z0s), b0z + whi);
+        const int iz2 = min(max((int)floorf(pz + r_p - ofz), z0s), b0z + whi);
+        if (AT >= 0 && fin && ix2 - ix1 <= 3 && iy2 - iy1 <= 3 && iz2 - iz1 <= 3) {
             // r_p <= 2: the footprint is at most 4 cells wide on an axis
             // unless p - of is an integer there (5 wide: the loop below).
-            // The 4^3 box is unrolled; offsets past the footprint get an
-            // infinite squared distance, hence weight 0 and no LDS access.
+            // Offsets past the footprint get an infinite squared distance,
+            // hence weight 0.
             float cx[4], cx2[4], cy[4], cy2[4], cz[4], cz2[4];
 #pragma unroll
             for (int o = 0; o < 4; ++o) {
@@ -492,188 +350,237 @@ __global__ __launch_bounds__(kSplatThreads) void mac_splat_kernel(GridView gm, G
                 cy2[o] = iy1 + o <= iy2 ? cy[o] * cy[o] : __builtin_inff();
                 cz2[o] = iz1 + o <= iz2 ? cz[o] * cz[o] : __builtin_inff();
                 // computed once per particle: the empty statements keep the
-                // compiler from recomputing them at each of the 64 cells
+                // compiler from recomputing them at each of the cells
                 asm volatile("" : "+v"(cx[o]), "+v"(cx2[o]));
             }
-            const int base = ((iz1 - z0s) * MSX + (iy1 - y0s)) * MSX + ix1 - x0s;
-            // A cell can hold a contribution 0 < |q| < 2^24 only if its weight
-            // is below wthr: |q| = fl(w |sq|) < 2^24 needs w |sq| < 2^24, and
-            // wthr >= 2^24 / |sq| on every channel with sq != 0 (the quotient
-            // rounded, then raised by 2^-21).  Cells with 0 < w < wthr take the
-            // vote, a superset of those that need it.
-            float wthr = 0.0f;
+            const int row = MSX, plane = MSX * MSX;
+            double *base = acc + ((iz1 - z0s) * MSX + (iy1 - y0s)) * MSX + ix1 - x0s;
+            // 1 - df2 / r_p^2 (Eq. 6) of face cell (ox, oy, oz) for the particle at p - 1/2
+            auto t_of = [&](int ox, int oy, int oz) {
+                const float dist_sq = cx2[ox] + (cz2[oz] + cy2[oy]);
+                const float d_a = AT == 0 ? cx[ox] : (AT == 1 ? cy[oy] : cz[oz]);
+                const float df2 = dist_sq + d_a + 0.25f;
+                return 1.0f - df2 * inv_r2;
+            };
+            auto add = [&](double *at, float w) {
+                if (w > 0.0f) {
+                    const float w3 = w * w * w;
 #pragma unroll
-            for (int k = 0; k < NC; ++k)
-                if (sq[k] != 0.0f) wthr = fmaxf(wthr, (kExact / fabsf(sq[k])) * (1.0f + 0x1p-21f));
-#pragma unroll
-            for (int oz = 0; oz < 4; ++oz)
-#pragma unroll
-                for (int oy = 0; oy < 4; ++oy) {
-                    const float dyz = cz2[oz] + cy2[oy];
-                    const int row = base + (oz * MSX + oy) * MSX;
-#pragma unroll
-                    for (int ox = 0; ox < 4; ++ox) {
-                        const float dist_sq = cx2[ox] + dyz;
-                        const float d_a = AT == 0 ? cx[ox] : (AT == 1 ? cy[oy] : cz[oz]);
-                        const float df2 = dist_sq + d_a + 0.25f;
-                        float w = fmaxf(1.0f - df2 * inv_r2, 0.0f);
-                        w = w * w * w;
-                        // Common case, no branch: every lane's scaled
-                        // contribution is 0 or at least 2^24 in magnitude,
-                        // so its magnitude converts exactly and the signed
-                        // add (zero included) goes straight to the window.
-                        if (__any((w > 0.0f) & (w < wthr))) {  // no short circuit
-                            contrib(row + ox, w, sf, sq);
-                        } else {
-#pragma unroll
-                            for (int k = 0; k < NC; ++k)
-                                atomicAdd(&acc[k * NS + row + ox], (integral_mag_u64(w * sq[k]) ^ sgn[k]) - sgn[k]);
-                        }
-                    }
+                    for (int k = 0; k < NC; ++k) unsafeAtomicAdd(at + k * NS, (double)(w3 * sc[k]));
                 }
+            };
+            auto cell = [&](int ox, int oy, int oz) { add(base + oz * plane + oy * row + ox, t_of(ox, oy, oz)); };
+            // Two cells of which at most one has a positive weight share an add.
+            auto either = [&](int ax, int ay, int az, int bx, int by, int bz) {
+                const float ta = t_of(ax, ay, az), tb = t_of(bx, by, bz);
+                add(base + (tb > 0.0f ? bz * plane + by * row + bx : az * plane + ay * row + ax), fmaxf(ta, tb));
+            };
+            // On an axis the cells 0 and 3 lie d and 3 - d from the particle,
+            // both at least r_p - 1 (a footprint cut at the domain's lower
+            // bound has no cell 3, and its cell 0 is outside the domain).
+            // Cells that swap 0 and 3 on two axes have squared distances that
+            // sum to at least 4 (3/2)^2 = 9 > 2 r_p^2, so one of them is
+            // outside the support.  Two of the 8 corners that differ on one
+            // axis only sum to at least 9/2 + 4 (r_p - 1)^2, 1/2 + 2 (r_p - 2)^2
+            // above 2 r_p^2: one corner at most is inside.  So 45 adds a
+            // channel instead of 64 (4.55 -> 4.16 ms a direction; an add takes
+            // 12 to 19 cycles, growing with the lanes that take part).
+            float best = t_of(0, 0, 0);
+            int at = 0;
+#pragma unroll
+            for (int c = 1; c < 8; ++c) {
+                const int ox = c & 1 ? 3 : 0, oy = c & 2 ? 3 : 0, oz = c & 4 ? 3 : 0;
+                const float tc = t_of(ox, oy, oz);
+                at = tc > best ? oz * plane + oy * row + ox : at;
+                best = fmaxf(best, tc);
+            }
+            add(base + at, best);
+#pragma unroll
+            for (int o = 1; o < 3; ++o) {
+                either(0, o, 0, 3, o, 3);
+                either(3, o, 0, 0, o, 3);
+                either(o, 0, 0, o, 3, 3);
+                either(o, 3, 0, o, 0, 3);
+                either(0, 0, o, 3, 3, o);
+                either(3, 0, o, 0, 3, o);
+#pragma unroll
+                for (int i = 1; i < 3; ++i) {
+                    cell(o, i, 0);
+                    cell(o, i, 3);
+                    cell(o, 0, i);
+                    cell(o, 3, i);
+                    cell(0, o, i);
+                    cell(3, o, i);
+                    cell(1, o, i);
+                    cell(2, o, i);
+                }
+            }
         } else {
             for (int iz = iz1; iz <= iz2; ++iz)
                 for (int iy = iy1; iy <= iy2; ++iy)
-                    for (int ix = ix1; ix <= ix2; ++ix)
-                        contrib(((iz - z0s) * MSX + (iy - y0s)) * MSX + ix - x0s, weight(px0, py0, pz0, ix, iy, iz),
-                                sf, sq);
-        }
-    }
-    __syncthreads();
-    // Window values in float: CH 0 / 1 into the residue window; CH 2 into
-    // the first half of each int64 window's bytes (read all, barrier, write),
-    // then the listed small terms on top.
-    float *fv[NC];
-    if (CH != 2) {
-        const double down = ldexp(1.0, ex[0] - 61);
-        for (int s = threadIdx.x; s < NS; s += blockDim.x) {
-            const long long ia = (long long)acc[s];
-            res[s] = (float)((double)ia * down + (double)res[s]);
-        }
-        fv[0] = res;
-    } else {
-        float v[NC][kSplatMaxCells / kSplatThreads];
+                    for (int ix = ix1; ix <= ix2; ++ix) {
+                        const float dz = (float)iz - pz0, dy = (float)iy - py0, dx = (float)ix - px0;
+                        const float dist_sq = dx * dx + (dz * dz + dy * dy);
+                        const float d_a = a == 0 ? dx : (a == 1 ? dy : dz);
+                        const float df2 = dist_sq + d_a + 0.25f;
+                        float w = fmaxf(1.0f - df2 * inv_r2, 0.0f);
+                        w = w * w * w;
+                        // a non-finite scale reaches its whole footprint, weights of 0 included
+                        if (w > 0.0f || !fin) {
+                            const int cell = ((iz - z0s) * MSX + (iy - y0s)) * MSX + ix - x0s;
 #pragma unroll
-        for (int k = 0; k < NC; ++k) {
-            const double down = ldexp(1.0, ex[k] - 61);
-#pragma unroll
-            for (int i = 0; i < kSplatMaxCells / kSplatThreads; ++i) {
-                const int s = threadIdx.x + i * kSplatThreads;
-                v[k][i] = s < NS ? (float)((double)(long long)acc[k * NS + s] * down) : 0.0f;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < NC; ++k) {
-            fv[k] = reinterpret_cast<float *>(acc + k * NS);
-#pragma unroll
-            for (int i = 0; i < kSplatMaxCells / kSplatThreads; ++i) {
-                const int s = threadIdx.x + i * kSplatThreads;
-                if (s < NS) fv[k][s] = v[k][i];
-            }
-        }
-        __syncthreads();
-        const int nl = min(s_nres, kResCap);
-        for (int i = threadIdx.x; i < nl; i += blockDim.x) {
-            const uint2 e = rlist[i];
-            atomicAdd(&fv[e.x >> 31][e.x & 0x7fffffffu], __uint_as_float(e.y));
-        }
-    }
-    __syncthreads();
-    // Commit (p2g.rs:342-411): staging cell -> its region -> the region's
-    // block (the region table above).  Window cell s = (lz MSX + ly) MSX + lx
-    // is split in float: (s + 1/2) / n is at least 1/(2n) away from an
-    // integer, far beyond its rounding.
-    const float inv_m1 = 1.0f / (float)MSX, inv_m2 = 1.0f / (float)(MSX * MSX);
-    auto region = [&](int l) { return l < m ? 0 : (l < m + 16 ? 1 : 2); };
-    // The target of staging cell s for channel k, or null where its region is not committed.
-    auto target = [&](int s, int k) -> float * {
-        const int lz = (int)(((float)s + 0.5f) * inv_m2), r = s - lz * MSX * MSX;
-        const int ly = (int)(((float)r + 0.5f) * inv_m1), lx = r - ly * MSX;
-        const int slot = s_slot[is_mass(k) ? 0 : 1][region(lx) + 3 * region(ly) + 9 * region(lz)];
-        if (slot < 0) return nullptr;
-        const int vid = ((x0s + lx) & 15) | (((y0s + ly) & 15) << 4) | (((z0s + lz) & 15) << 8);
-        return (is_mass(k) ? gm.slab : gv.slab) + (int64_t)slot * 4096 + vid;
-    };
-    // Four window cells per lane at a time, their reads issued before their writes.
-    for (int s0 = threadIdx.x; s0 < NS; s0 += 4 * kSplatThreads) {
-        float *pt[4][NC];
-        float val[4][NC];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int s = s0 + i * kSplatThreads;
-            const bool in = s < NS;
-            const int sc = in ? s : 0;
-#pragma unroll
-            for (int k = 0; k < NC; ++k) {
-                val[i][k] = in ? fv[k][sc] : 0.0f;
-                pt[i][k] = val[i][k] != 0.0f ? target(sc, k) : nullptr;
-            }
-        }
-        if (item.shared) {  // blocks of one colour never share a window: only the block's own items race
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int k = 0; k < NC; ++k)
-                    if (pt[i][k]) unsafeAtomicAdd(pt[i][k], val[i][k]);
-        } else {
-            float old[4][NC];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int k = 0; k < NC; ++k) old[i][k] = pt[i][k] ? *pt[i][k] : 0.0f;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int k = 0; k < NC; ++k)
-                    if (pt[i][k]) *pt[i][k] = old[i][k] + val[i][k];
-        }
-    }
-    if (!item_nonfin) return;
-    // Particles with a non-finite mass or momentum scale: their float
-    // contributions go straight to the committed cells (NaN / Inf propagate
-    // as in a float sum; finite cells outside their footprints keep the exact
-    // result above).
-    __syncthreads();
-    for (int j = 0; j < per; ++j) {
-        const int pi = p_beg + (int)threadIdx.x * per + j;
-        if (pi >= p_beg + p_cnt) break;
-        float sc[NC];
-        bool bad = false;
-#pragma unroll
-        for (int k = 0; k < NC; ++k) {
-            sc[k] = scale_of(pi, k);
-            bad = bad || !isfinite(sc[k]);
-        }
-        if (!bad) continue;
-        const float px0 = spos[3 * pi] - 0.5f, py0 = spos[3 * pi + 1] - 0.5f, pz0 = spos[3 * pi + 2] - 0.5f;
-        int ix1, ix2, iy1, iy2, iz1, iz2;
-        footprint(pi, ix1, ix2, iy1, iy2, iz1, iz2);
-        for (int iz = iz1; iz <= iz2; ++iz)
-            for (int iy = iy1; iy <= iy2; ++iy)
-                for (int ix = ix1; ix <= ix2; ++ix) {
-                    const float w = weight(px0, py0, pz0, ix, iy, iz);
-                    const int cell = ((iz - z0s) * MSX + (iy - y0s)) * MSX + ix - x0s;
-#pragma unroll
-                    for (int k = 0; k < NC; ++k) {
-                        if (isfinite(sc[k])) continue;
-                        float *po = target(cell, k);
-                        if (po) atomicAdd(po, w * sc[k]);
+                            for (int k = 0; k < NC; ++k) unsafeAtomicAdd(&acc[k * NS + cell], (double)(w * sc[k]));
+                        }
                     }
+        }
+    }
+    __syncthreads();
+    float2 *out = win + (int64_t)blockIdx.x * NS;
+    auto put = [&](int at, int s) {
+        if (CH == 2)
+            out[at] = make_float2((float)acc[s], (float)acc[NS + s]);
+        else
+            reinterpret_cast<float *>(out + at)[CH] = (float)acc[s];
+    };
+    const int rows = MSX * MSX;
+    for (int s = threadIdx.x; s < rows * 16; s += kSplatThreads) put(s, (s >> 4) * MSX + m + (s & 15));
+    for (int r = threadIdx.x; r < rows; r += kSplatThreads)
+        for (int x = 0; x < m; ++x) {
+            put(rows * 16 + r * m + x, r * MSX + x);
+            put(rows * (16 + m) + r * m + x, r * MSX + 16 + m + x);
+        }
+}
+
+// The commit (p2g.rs:342-411) and MacGrid::normalize_velocity (mac.rs:106-132)
+// of one face direction: every cell of the active blocks takes the sum of the
+// windows that cover it, in float64 and in a fixed order (own block, then the
+// neighbours whose margin it lies in, each block's items in order), rounded
+// once, and u = P / M (0 where M <= 0).  `first[b]` is the first item of block
+// b and `count[b]` their number.  Source block S commits window region (rx,
+// ry, rz), the margin below, its own 16 cells or the margin above on each
+// axis, only when that lies inside the domain; a particle on the domain's
+// upper z bound makes S a block of the layer above it.  Where the windows come
+// in several passes, all but the first add to the grid's cells and only the
+// last divides.  Adding the windows into the grid from the splat took 8 colour
+// passes a direction, a zero fill before and a division pass after (67 M
+// particles: 26 ms, 16 so; 100,000: 2.5 ms, 0.1).  It is bound by the windows'
+// bytes on large sets and by its dependent loads on small ones.
+//
+// A work-group of 256 lanes takes one block, plane after plane; with SPLIT its
+// 1,024 lanes take one plane, and the four groups of 256 share the items of
+// every region (few blocks of many items).  One plane per work-group
+// everywhere took twice as long on large sets (67 M particles: 3.9 ms a
+// direction, 1.08 so): its chain of dependent loads (list, slots, ranges,
+// windows) weighs as much as the cells of a plane.
+template <bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 1024 : 256) void mac_commit_kernel(GridView gm, GridView gv,
+                                                                        const int32_t *__restrict__ active,
+                                                                        const int32_t *__restrict__ first,
+                                                                        const int32_t *__restrict__ count,
+                                                                        const float2 *__restrict__ win, int m,
+                                                                        bool head, bool last) {
+    __shared__ int s_first[27], s_count[27];
+    __shared__ double s_part[2][3][SPLIT ? 256 : 1];
+    const int bid = active[SPLIT ? blockIdx.x >> 4 : blockIdx.x];
+    const int ms = gm.b2s[bid], vs = gv.b2s[bid];
+    if (ms < 2 || vs < 2) return;
+    const int bx = bid % gm.nx, by = (bid / gm.nx) % gm.ny, bz = bid / (gm.nx * gm.ny);
+    if (threadIdx.x < 27) {
+        const int t = threadIdx.x;
+        const int o[3] = {t % 3 - 1, (t / 3) % 3 - 1, t / 9 - 1};
+        const int b[3] = {bx + o[0], by + o[1], bz + o[2]}, nb[3] = {gm.nx, gm.ny, gm.nz + 1}, s[3] = {gm.sx, gm.sy, gm.sz};
+        bool in = true;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            in = in && b[d] >= 0 && b[d] < nb[d];
+            // this block is S's upper margin (o < 0), its own cells (0) or its lower margin
+            in = in && b[d] * 16 + (o[d] > 0 ? 0 : 16) + (o[d] < 0 ? m : 0) <= s[d];
+        }
+        const int src = b[0] + gm.nx * (b[1] + gm.ny * b[2]);
+        s_count[t] = in ? count[src] : 0;
+        s_first[t] = in ? first[src] : 0;
+    }
+    __syncthreads();
+    const int MSX = 16 + 2 * m, NS = MSX * MSX * MSX, rows = MSX * MSX;
+    const int cell = threadIdx.x & 255, group = threadIdx.x >> 8;
+    const int cx = cell & 15, cy = cell >> 4;
+    // the one neighbour on each axis whose margin the cell lies in, or 0
+    const int ox = cx < m ? -1 : (cx >= 16 - m ? 1 : 0), oy = cy < m ? -1 : (cy >= 16 - m ? 1 : 0);
+    const int step = SPLIT ? 4 : 1;
+#pragma unroll 1
+    for (int cz = SPLIT ? (int)(blockIdx.x & 15) : 0; cz < 16; cz += SPLIT ? 16 : 1) {
+        const int oz = cz < m ? -1 : (cz >= 16 - m ? 1 : 0);
+        float *pm = gm.slab + (int64_t)ms * 4096 + cz * 256 + cell;
+        float *pv = gv.slab + (int64_t)vs * 4096 + cz * 256 + cell;
+        double sm = 0.0, sv = 0.0;
+        if (!head && group == 0) {
+            sm = (double)*pm;
+            sv = (double)*pv;
+        }
+        // the first window of each region, all loads in flight together, then the rest four at a time
+        float2 f[8];
+        int n[8], at[8];  // a pass's windows are below 2^31 cells
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            n[k] = 0;
+            f[k] = make_float2(0.0f, 0.0f);
+            if ((k & 4) && !oz) continue;  // uniform
+            const int kx = (k & 1) ? ox : 0, ky = (k & 2) ? oy : 0, kz = (k & 4) ? oz : 0;
+            const int t = (kx + 1) + 3 * (ky + 1) + 9 * (kz + 1);
+            n[k] = ((k & 1) && !ox) || ((k & 2) && !oy) ? 0 : s_count[t];
+            const int row = (cz - 16 * kz + m) * MSX + cy - 16 * ky + m;
+            at[k] = (s_first[t] + group) * NS +
+                    (kx == 0 ? row * 16 + cx
+                             : (kx < 0 ? rows * (16 + m) + row * m + cx : rows * 16 + row * m + cx - 16 + m));
+            if (n[k] > group) f[k] = win[at[k]];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            sm += (double)f[k].x;
+            sv += (double)f[k].y;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            for (int j = group + step; j < n[k]; j += 4 * step) {
+                float2 g[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    g[i] = j + i * step < n[k] ? win[at[k] + (j + i * step - group) * NS] : make_float2(0.0f, 0.0f);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    sm += (double)g[i].x;
+                    sv += (double)g[i].y;
                 }
+            }
+        if (SPLIT) {
+            if (group > 0) {
+                s_part[0][group - 1][cell] = sm;
+                s_part[1][group - 1][cell] = sv;
+            }
+            __syncthreads();
+            if (group > 0) return;
+            for (int g = 0; g < 3; ++g) {
+                sm += s_part[0][g][cell];
+                sv += s_part[1][g][cell];
+            }
+        }
+        const float mm = (float)sm, mv = (float)sv;
+        *pm = mm;
+        *pv = !last ? mv : (mm > 0.0f ? mv / mm : 0.0f);
     }
 }
 
-// MacGrid::normalize_velocity (mac.rs:106-132): u = P/M, 0 where M <= 0.
-__global__ void normalize_kernel(GridView vg, GridView mg, const int32_t *__restrict__ active) {
-    const int64_t bid = active[blockIdx.x];
-    const int vs = vg.b2s[bid], ms = mg.b2s[bid];
-    if (vs < 2) return;
-    for (int j = threadIdx.x; j < 4096; j += blockDim.x) {
-        const float mm = mg.slab[(int64_t)ms * 4096 + j];
-        float &v = vg.slab[(int64_t)vs * 4096 + j];
-        v = mm > 0.0f ? v / mm : 0.0f;
-    }
+// first / count of each block from its items (first at its first one).
+__global__ void splat_ranges_kernel(const SplatItem *__restrict__ items, int n, int32_t *__restrict__ first,
+                                    int32_t *__restrict__ count) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int bid = items[i].bid;
+    if (i > 0 && items[i - 1].bid == bid) return;
+    int e = i + 1;
+    while (e < n && items[e].bid == bid) ++e;
+    first[bid] = i;
+    count[bid] = e - i;
 }
 
 // ---------------------------------------------------------------------------
@@ -1138,13 +1045,16 @@ int msbg_particles_to_grid_mac(msbg_grid *const *vel, msbg_grid *const *mass, co
     MSBG_CHECK(n >= 0 && n < ((int64_t)1 << 31) && (n == 0 || (d_pos && d_vel && d_mass)), MSBG_EINVAL,
                "particles_to_grid: bad particle arrays");
     const msbg_grid *g = vel[0];
-    // active blocks with the (r_p + 1)/bsx footprint (p2g.rs:104-107), zeroed
+    // active blocks with the (r_p + 1)/bsx footprint (p2g.rs:104-107); the
+    // commit writes every cell of them
     std::vector<int64_t> act;
     int32_t *d_act = nullptr;
     rc = active_list(g, d_pos, n, r_p + 1.0f, act, &d_act);
     if (rc) return rc;
-    rc = zero_blocks(all, 6, act);
-    if (rc) return rc;
+    for (msbg_grid *c : all) {
+        rc = msbg_grid_ensure_blocks(c, act.data(), (int64_t)act.size());
+        if (rc) return rc;
+    }
     *n_active = (int64_t)act.size();
     if (n == 0) return MSBG_OK;
     // bucket by block (p2g.rs:149-158).  Particles that arrive grouped by
@@ -1155,8 +1065,10 @@ int msbg_particles_to_grid_mac(msbg_grid *const *vel, msbg_grid *const *mass, co
     uint32_t *perm = keys + n;
     int32_t *d_ungrouped = (int32_t *)(perm + n);
     hipLaunchKernelGGL(set_flag_kernel, dim3(1), dim3(1), 0, stream(), d_ungrouped, 0);
+    // block ids, one layer past the upper z bound included, and `most` for all beyond
+    const int64_t most = g->n_blocks + (int64_t)g->nx * g->ny;
     hipLaunchKernelGGL(bucket_keys_grouped_kernel, dim3(grid_for(n, 256)), dim3(256), 0, stream(), d_pos, n,
-                       (int32_t)g->nx, (int32_t)g->ny, keys, perm, d_ungrouped);
+                       (int32_t)g->nx, (int32_t)g->ny, (uint32_t)most, keys, perm, d_ungrouped);
     MSBG_HIP(hipGetLastError());
     int32_t ungrouped = 1;
     MSBG_HIP(hipMemcpyAsync(&ungrouped, d_ungrouped, sizeof(int32_t), hipMemcpyDeviceToHost, stream()));
@@ -1167,7 +1079,7 @@ int msbg_particles_to_grid_mac(msbg_grid *const *vel, msbg_grid *const *mass, co
     int32_t *pblocks = (int32_t *)(pay + 7 * n), *starts = pblocks + n;
     if (ungrouped) {
         int key_bits = 1;
-        while (key_bits < 32 && ((int64_t)1 << key_bits) < g->n_blocks) ++key_bits;
+        while (key_bits < 32 && ((int64_t)1 << key_bits) <= most) ++key_bits;
         rc = radix_sort_pairs(keys, perm, n, key_bits);
         if (rc) return rc;
         hipLaunchKernelGGL(gather_payload_kernel, dim3(grid_for(n, 256)), dim3(256), 0, stream(), d_pos, d_vel, d_mass,
@@ -1180,37 +1092,41 @@ int msbg_particles_to_grid_mac(msbg_grid *const *vel, msbg_grid *const *mass, co
     int64_t nocc = 0;
     rc = run_lengths(keys, n, pblocks, starts, &nocc);
     if (rc) return rc;
-    // colour lists of occupied-block indices (p2g.rs:186-191), each block's
-    // particles cut into items of at most kSplatChunk (dense blocks, e.g. a
-    // droplet's, would otherwise serialise a whole colour pass on one work-group)
+    // the blocks' particles, cut into items
     std::vector<int32_t> hb((size_t)nocc), hs((size_t)nocc + 1);
     MSBG_HIP(hipMemcpy(hb.data(), pblocks, sizeof(int32_t) * nocc, hipMemcpyDeviceToHost));
     MSBG_HIP(hipMemcpy(hs.data(), starts, sizeof(int32_t) * (nocc + 1), hipMemcpyDeviceToHost));
+    int32_t cut = kSplatLeast;
+    while (cut < kSplatMost && (int64_t)cut * kSplatItems < n) cut *= 2;
     std::vector<SplatItem> order;
-    int64_t cnt[8] = {0};
-    for (int c = 0; c < 8; ++c)
-        for (int64_t i = 0; i < nocc; ++i) {
-            const int64_t b = hb[i];
-            const int64_t bx = b % g->nx, by = (b / g->nx) % g->ny, bz = b / g->nxy;
-            if ((int)((bx & 1) | ((by & 1) << 1) | ((bz & 1) << 2)) != c) continue;
-            const int32_t p0 = hs[i], p1 = hs[i + 1];
-            const int32_t shared = p1 - p0 > kSplatChunk ? 1 : 0;
-            for (int32_t q = p0; q < p1; q += kSplatChunk) {
-                order.push_back(SplatItem{(int32_t)i, q, std::min(p1, q + kSplatChunk), shared});
-                ++cnt[c];
-            }
-        }
-    SplatItem *d_order =
-        (SplatItem *)workspace(3, sizeof(SplatItem) * std::max<size_t>(order.size(), 1), &rc);
-    if (rc) return rc;
-    MSBG_HIP(hipMemcpyAsync(d_order, order.data(), sizeof(SplatItem) * order.size(), hipMemcpyHostToDevice, stream()));
+    order.reserve((size_t)(nocc + n / cut));
+    for (int64_t i = 0; i < nocc; ++i) {
+        if (hb[i] >= most) continue;
+        const int64_t cnt = hs[i + 1] - hs[i], parts = (cnt + cut - 1) / cut;
+        for (int64_t p = 0; p < parts; ++p)
+            order.push_back(SplatItem{hb[i], (int32_t)(hs[i] + cnt * p / parts), (int32_t)(hs[i] + cnt * (p + 1) / parts)});
+    }
+    const int n_items = (int)order.size();
     const int m = (int)ceilf(r_p);
-    const int msx = 16 + 2 * m;
-    // both channels in one pass when two int64 windows and the residue list
-    // fit (r_p <= 2), else a pass per channel with a float residue window
-    const bool both = msx * msx * msx <= kSplatMaxCells;
-    const size_t lds = both ? 2 * sizeof(unsigned long long) * msx * msx * msx + sizeof(uint2) * kResCap
-                            : (sizeof(unsigned long long) + sizeof(float)) * msx * msx * msx;
+    const int msx = 16 + 2 * m, ns = msx * msx * msx;
+    // items, and the item range of each block
+    SplatItem *d_order = (SplatItem *)workspace(3, sizeof(SplatItem) * n_items + sizeof(int32_t) * 2 * most, &rc);
+    if (rc) return rc;
+    int32_t *d_first = (int32_t *)(d_order + n_items), *d_count = d_first + most;
+    // the windows of at most `chunk` items: up to 2 GiB, less where that does not fit the device
+    int chunk = std::max(1, std::min(n_items, (int)(((int64_t)1 << 31) / ((int64_t)sizeof(float2) * ns))));
+    float2 *win = nullptr;
+    for (;; chunk = (chunk + 1) / 2) {
+        win = (float2 *)workspace(24, sizeof(float2) * ns * (size_t)chunk, &rc);
+        if (!rc) break;
+        if (rc != MSBG_ENOMEM || chunk <= 16) return rc;
+        (void)hipGetLastError();
+    }
+    if (n_items)
+        MSBG_HIP(hipMemcpyAsync(d_order, order.data(), sizeof(SplatItem) * n_items, hipMemcpyHostToDevice, stream()));
+    // both channels in one pass when two float64 windows fit (r_p <= 2), else a pass per channel
+    const bool both = ns <= kSplatMaxCells;
+    const size_t lds = (both ? 2 : 1) * sizeof(double) * ns;
     {
         int dev = 0, max_lds = 0;
         MSBG_HIP(hipGetDevice(&dev));
@@ -1226,38 +1142,41 @@ int msbg_particles_to_grid_mac(msbg_grid *const *vel, msbg_grid *const *mass, co
         }
     }
     const float inv_r2 = 1.0f / (r_p * r_p);
-    for (int a = 0; a < 3; ++a) {
-        int64_t off = 0;
-        for (int c = 0; c < 8; ++c) {
-            if (cnt[c] && both) {
-                const dim3 grid((unsigned)cnt[c]), block(kSplatThreads);
-                const GridView mv = mass[a]->view(), vv = vel[a]->view();
-                if (a == 0)
-                    mac_splat_kernel<2, 0><<<grid, block, lds, stream()>>>(mv, vv, a, d_order + off, pblocks, spos,
-                                                                          svel, smass, r_p, inv_r2, m);
-                else if (a == 1)
-                    mac_splat_kernel<2, 1><<<grid, block, lds, stream()>>>(mv, vv, a, d_order + off, pblocks, spos,
-                                                                          svel, smass, r_p, inv_r2, m);
-                else
-                    mac_splat_kernel<2, 2><<<grid, block, lds, stream()>>>(mv, vv, a, d_order + off, pblocks, spos,
-                                                                          svel, smass, r_p, inv_r2, m);
-            } else if (cnt[c]) {
-                hipLaunchKernelGGL((mac_splat_kernel<0, -1>), dim3((unsigned)cnt[c]), dim3(kSplatThreads), lds,
-                                   stream(), mass[a]->view(), vel[a]->view(), a, d_order + off, pblocks, spos, svel,
-                                   smass, r_p, inv_r2, m);
-                hipLaunchKernelGGL((mac_splat_kernel<1, -1>), dim3((unsigned)cnt[c]), dim3(kSplatThreads), lds,
-                                   stream(), mass[a]->view(), vel[a]->view(), a, d_order + off, pblocks, spos, svel,
-                                   smass, r_p, inv_r2, m);
+    for (int at = 0; at == 0 || at < n_items; at += chunk) {
+        const int cnt = std::min(chunk, n_items - at);
+        const bool head = at == 0, last = at + chunk >= n_items;
+        hipLaunchKernelGGL(fill_i32_kernel, dim3(grid_for(most, 256)), dim3(256), 0, stream(), d_count, most, 0);
+        if (cnt > 0)
+            hipLaunchKernelGGL(splat_ranges_kernel, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, stream(),
+                               d_order + at, cnt, d_first, d_count);
+        for (int a = 0; a < 3; ++a) {
+            const auto splat = [&](auto kernel) {
+                if (cnt > 0)
+                    kernel<<<cnt, kSplatThreads, lds, stream()>>>((int)g->nx, (int)g->ny, a, d_order + at, spos, svel,
+                                                                  smass, r_p, inv_r2, m, win);
+            };
+            if (!both) {
+                splat(mac_splat_kernel<0, -1>);
+                splat(mac_splat_kernel<1, -1>);
+            } else if (a == 0) {
+                splat(mac_splat_kernel<2, 0>);
+            } else if (a == 1) {
+                splat(mac_splat_kernel<2, 1>);
+            } else {
+                splat(mac_splat_kernel<2, 2>);
             }
-            off += cnt[c];
+            // below four blocks a CU a plane per work-group, or the chip idles
+            // (48 blocks: 14 us, 106 with a block's items read by one group of lanes)
+            const unsigned nact = (unsigned)act.size();
+            if (nact > 0 && nact < 1024)
+                mac_commit_kernel<true><<<16 * nact, 1024, 0, stream()>>>(mass[a]->view(), vel[a]->view(), d_act, d_first,
+                                                                         d_count, win, m, head, last);
+            else if (nact > 0)
+                mac_commit_kernel<false><<<nact, 256, 0, stream()>>>(mass[a]->view(), vel[a]->view(), d_act, d_first,
+                                                                     d_count, win, m, head, last);
+            MSBG_HIP(hipGetLastError());
         }
-        MSBG_HIP(hipGetLastError());
     }
-    if (!act.empty())
-        for (int a = 0; a < 3; ++a)
-            hipLaunchKernelGGL(normalize_kernel, dim3((unsigned)act.size()), dim3(256), 0, stream(), vel[a]->view(),
-                               mass[a]->view(), d_act);
-    MSBG_HIP(hipGetLastError());
     MSBG_HIP(hipStreamSynchronize(stream()));
     return MSBG_OK;
 }

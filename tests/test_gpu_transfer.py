@@ -171,6 +171,59 @@ def test_particles_to_grid_mac_dense_cluster(pkg, orc, hip):
     print("MAC P2G dense cluster: worst error / (1e-6 bound) = %.3f" % worst)
 
 
+def test_particles_to_grid_mac_windows_in_two_passes(pkg, hip):
+    """33^3 occupied blocks are more windows than one pass holds (33,554):
+    the blocks around the seam get the values of a call with the particles of
+    the upper four layers alone, up to a rounding of each partial sum."""
+    nb, s = 33, (528, 528, 528)
+    rng = np.random.default_rng(2)
+    b = np.arange(nb ** 3)
+    corner = 16.0 * np.stack([b % nb, (b // nb) % nb, b // nb ** 2], 1)
+    pos = (corner + rng.uniform(0.0, 15.99, corner.shape)).astype(np.float32)
+    vel = rng.uniform(1.0, 2.0, pos.shape).astype(np.float32)
+    mass = rng.uniform(0.5, 2.0, nb ** 3).astype(np.float32)
+    up = b // nb ** 2 >= 28
+    whole, part = (T.MacGrid(*s, capacity_blocks=nb ** 3 + 8, lib=hip) for _ in range(2))
+    assert T.particles_to_grid(whole, pos, vel, mass, 2.0) == nb ** 3
+    T.particles_to_grid(part, pos[up], vel[up], mass[up], 2.0)
+    for a in range(3):
+        for gw, gp in ((whole.mass[a], part.mass[a]), (whole.velocity[a], part.velocity[a])):
+            hw, hp = gw.to_host(), gp.to_host()
+            bids = np.nonzero(b // nb ** 2 >= 29)[0]
+            vw, vp = hw.slab[hw.b2s[bids]], hp.slab[hp.b2s[bids]]
+            np.testing.assert_allclose(vw, vp, rtol=8 * 2.0 ** -24, atol=0)
+            assert (vw != 0).any()
+
+
+@pytest.mark.parametrize("s", [(48, 32, 48), (32, 48, 40)])
+def test_particles_to_grid_mac_on_the_upper_bound(pkg, hip, s):
+    """Particles on and just past the domain's upper z bound: the block above
+    the domain commits its lower margin where that margin lies inside the
+    domain.  Against the sums in float64: w is 1 - df2 / r_p^2 to about four
+    roundings of values up to 5, so w^3 to 4e-6."""
+    rng = np.random.default_rng(8)
+    n = 40
+    pos = rng.uniform(3.0, 28.0, (n, 3)).astype(np.float32)
+    pos[:, 2] = s[2] + np.float32([0.0, 0.5, 1.25, 2.0])[np.arange(n) % 4]
+    vel = np.ones((n, 3), np.float32)
+    mass = np.ones(n, np.float32)
+    mac = T.MacGrid(*s, capacity_blocks=64, lib=hip)
+    T.particles_to_grid(mac, pos, vel, mass, 2.0)
+    if s[2] % 16:
+        return  # the margin is cut by the bound: nothing is committed, and the call returned
+    z, y, x = np.meshgrid(*[np.arange(k) for k in s[::-1]], indexing="ij")
+    for a in range(3):
+        M64 = np.zeros(s[::-1])
+        for p in pos.astype(np.float64) - 0.5:
+            d = np.stack([x - p[0], y - p[1], z - p[2]])
+            w = np.maximum(1.0 - ((d ** 2).sum(0) + d[a] + 0.25) / 4.0, 0.0)
+            M64 += w ** 3
+        M64[: s[2] - 2] = 0.0  # beyond the window of the block above
+        M = mac.mass[a].to_host().to_dense()
+        assert M64.max() > 0.1
+        assert np.abs(M - M64).max() <= 4e-6 * n, a
+
+
 def test_particles_to_grid_mac_nonfinite_velocity(pkg, orc, hip):
     """One particle with a NaN velocity and one with an infinite one: their
     momentum footprints turn non-finite, every mass cell and every momentum
