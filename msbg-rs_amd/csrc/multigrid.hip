@@ -74,6 +74,7 @@ struct Level {
 struct Hierarchy {
     std::vector<Level> lv;    // lv[k] is level k + 1
     int32_t *nb27 = nullptr;  // [n_active][27]: listed index of block k's neighbour (dx, dy, dz), -1 / -2
+    int32_t *slot27 = nullptr;  // its slot, -1 where not listed
 };
 
 namespace {
@@ -305,118 +306,6 @@ __global__ __launch_bounds__(kT) void prolong_blk_kernel(i64 n_active, const PBl
     x[i] += blk_interp<B / 2>(xc, nb27 + k * 27, Bk, d, k, cx, cy, cz);
 }
 
-// Level 0 -> 1: b1 = 0.5 * sum of the 8 children of the FP32 residual r
-// (slot layout); children outside the domain count 0.
-__global__ __launch_bounds__(kT) void restrict0_kernel(i64 n_active, const PBlock *__restrict__ blocks, Dom d,
-                                                       const float *__restrict__ r, float *b1) {
-    const i64 i = (i64)blockIdx.x * kT + threadIdx.x;
-    if (i >= n_active * 512) return;
-    const PBlock B = blocks[i >> 9];
-    const int v = (int)(i & 511), ux = v & 7, uy = (v >> 3) & 7, uz = v >> 6;
-    const i64 base = ((i64)B.slot << 12);
-    // the 8 children as 4 x-pairs, all loaded before the sum (same terms, same order)
-    float2 pr[4];
-#pragma unroll
-    for (int h = 0; h < 4; ++h)
-        pr[h] = *reinterpret_cast<const float2 *>(r + base + 2 * ux + 16 * (2 * uy + (h & 1)) + 256 * (2 * uz + (h >> 1)));
-    float sum = 0.0f;
-#pragma unroll
-    for (int o = 0; o < 8; ++o) {
-        const int fx = 2 * ux + (o & 1), fy = 2 * uy + ((o >> 1) & 1), fz = 2 * uz + (o >> 2);
-        if (live(B, d, 1, fx, fy, fz)) sum += (o & 1) ? pr[o >> 1].y : pr[o >> 1].x;
-    }
-    b1[i] = 0.5f * sum;
-}
-
-// Value of level-1 cell (qx, qy, qz) relative to listed block k (coordinates
-// may step one block out on each axis); 0 outside the band.
-__device__ __forceinline__ float level1_at(const float *__restrict__ x1, const int32_t *__restrict__ T, i64 k, int qx,
-                                           int qy, int qz) {
-    const int ox = qx < 0 ? -1 : (qx >= 8 ? 1 : 0), oy = qy < 0 ? -1 : (qy >= 8 ? 1 : 0),
-              oz = qz < 0 ? -1 : (qz >= 8 ? 1 : 0);
-    const i64 nbk = (ox | oy | oz) ? (i64)T[nb27_at(ox, oy, oz)] : k;
-    if (nbk < 0) return 0.0f;
-    return x1[nbk * 512 + (qx & 7) + 8 * (qy & 7) + 64 * (qz & 7)];
-}
-
-// Level 1 -> 0: e += P x1 on the in-domain cells (e in storage ST).  One
-// work-group per listed block stages the block's level-1 cells with a 1-cell
-// ring (10^3 values, 0 outside the band) in LDS; thread t then interpolates
-// the 16 cells of row (y, z) = (t & 15, t >> 4): their trilinear partners are
-// the level-1 x-positions -1 .. 8 on 4 (y, z) rows.  A partner beyond the
-// domain is the cell itself (clamp), one outside the band reads 0.
-template <int ST>
-__global__ __launch_bounds__(256) void prolong0_kernel(const PBlock *__restrict__ blocks, Dom d,
-                                                       const int32_t *__restrict__ nb27, const float *__restrict__ x1,
-                                                       typename Sto<ST>::T *e) {
-    using S = Sto<ST>;
-    __shared__ float s_c[1000];
-    const i64 k = blockIdx.x;
-    const PBlock B = blocks[k];
-    const int32_t *T = nb27 + k * 27;
-    for (int s = threadIdx.x; s < 1000; s += 256)
-        s_c[s] = level1_at(x1, T, k, s % 10 - 1, (s / 10) % 10 - 1, s / 100 - 1);
-    __syncthreads();
-    const int cy = threadIdx.x & 15, cz = threadIdx.x >> 4;
-    if (B.oy + cy >= d.sy || B.oz + cz >= d.sz) return;
-    const int py = cy >> 1, pz = cz >> 1;
-    int dy = (cy & 1) ? 1 : -1, dz = (cz & 1) ? 1 : -1;
-    if ((dy > 0 && B.oy + 2 * (py + 1) >= d.sy) || (dy < 0 && py == 0 && T[nb27_at(0, -1, 0)] == -2)) dy = 0;
-    if ((dz > 0 && B.oz + 2 * (pz + 1) >= d.sz) || (dz < 0 && pz == 0 && T[nb27_at(0, 0, -1)] == -2)) dz = 0;
-    const bool left_wall = T[nb27_at(-1, 0, 0)] == -2;
-    const float *rows[4];
-#pragma unroll
-    for (int yz = 0; yz < 4; ++yz) {
-        const int qy = py + ((yz & 1) ? dy : 0), qz = pz + ((yz & 2) ? dz : 0);
-        rows[yz] = s_c + (qz + 1) * 100 + (qy + 1) * 10 + 1;  // rows[yz][qx], qx = -1 .. 8
-    }
-    float out[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int px = i >> 1;
-        int qn = px + ((i & 1) ? 1 : -1);
-        if ((qn > px && B.ox + 2 * qn >= d.sx) || (qn < 0 && left_wall)) qn = px;  // clamp
-        float val = 0.0f;
-#pragma unroll
-        for (int yz = 0; yz < 4; ++yz) {
-            const float wyz = ((yz & 1) ? 0.25f : 0.75f) * ((yz & 2) ? 0.25f : 0.75f);
-            val += wyz * (0.75f * rows[yz][px] + 0.25f * rows[yz][qn]);
-        }
-        out[i] = val;
-    }
-    const i64 j = ((i64)B.slot << 12) + 16 * cy + 256 * cz;
-    const int n = min(16, d.sx - B.ox);
-    if (n == 16) {
-        if constexpr (ST == MSBG_STORAGE_F32) {
-            float4 *q = reinterpret_cast<float4 *>(e + j);
-#pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                float4 a = q[m];
-                a.x += out[4 * m];
-                a.y += out[4 * m + 1];
-                a.z += out[4 * m + 2];
-                a.w += out[4 * m + 3];
-                q[m] = a;
-            }
-        } else {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                uint4 q = *reinterpret_cast<const uint4 *>(e + j + 8 * h);
-                uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-                for (int m = 0; m < 4; ++m) {
-                    const float lo = S::ld(reinterpret_cast<const typename S::T *>(&w[m]), 0) + out[8 * h + 2 * m];
-                    const float hi = S::ld(reinterpret_cast<const typename S::T *>(&w[m]), 1) + out[8 * h + 2 * m + 1];
-                    w[m] = (uint32_t)S::cv(lo) | (uint32_t)S::cv(hi) << 16;
-                }
-                *reinterpret_cast<uint4 *>(e + j + 8 * h) = make_uint4(w[0], w[1], w[2], w[3]);
-            }
-        }
-    } else {
-        for (int i = 0; i < n; ++i) e[j + i] = S::cv(S::ld(e, j + i) + out[i]);
-    }
-}
-
 __device__ __forceinline__ float list_residual(const float *__restrict__ x, const float *__restrict__ b,
                                                const int32_t *__restrict__ nb, const float *__restrict__ cf,
                                                const float *__restrict__ diag, i64 i) {
@@ -594,6 +483,12 @@ __global__ __launch_bounds__(kCoarseMax) void coarse_cg_kernel(int n, const int3
     }
     if (n_sing > 0) project_singular(xi, in, n, n_comp, s_comp, sing, s_p, s_mean);
     if (in) x[t] = (float)xi;
+}
+
+__global__ void slot27_kernel(const int32_t *__restrict__ nb27, const PBlock *__restrict__ blocks, i64 n,
+                              int32_t *__restrict__ slot27) {
+    const i64 i = (i64)blockIdx.x * kT + threadIdx.x;
+    if (i < n) slot27[i] = nb27[i] >= 0 ? blocks[nb27[i]].slot : -1;
 }
 
 int grid_of(i64 n) { return (int)((n + kT - 1) / kT); }
@@ -881,6 +776,7 @@ void release(msbg_poisson *p) {
         (void)hipFree(L.sing);
     }
     (void)hipFree(H->nb27);
+    (void)hipFree(H->slot27);
     delete H;
     p->mg = nullptr;
 }
@@ -905,6 +801,11 @@ int ensure(msbg_poisson *p) {
         }
     }
     hipError_t e = upload(&H->nb27, nb27);
+    if (e == hipSuccess) e = hipMalloc(&H->slot27, sizeof(int32_t) * nb27.size());
+    if (e == hipSuccess) {
+        slot27_kernel<<<grid_of((i64)nb27.size()), kT, 0, stream()>>>(H->nb27, p->d_blocks, (i64)nb27.size(), H->slot27);
+        e = hipGetLastError();
+    }
     for (int l = 1; l <= 3 && e == hipSuccess; ++l) {
         Level L;
         L.l = l;
@@ -948,13 +849,10 @@ int ensure(msbg_poisson *p) {
 
 int n_levels(const msbg_poisson *p) { return p->mg ? (int)p->mg->lv.size() + 1 : 0; }
 
-void vcycle(msbg_poisson *p, hipStream_t s, int storage, float omega, int nu, bool first_done) {
+void vcycle(msbg_poisson *p, hipStream_t s, int storage, float omega, int nu, float extra, float *x, float *lo) {
     const Hierarchy &H = *p->mg;
-    const i64 na = p->n_active;
     const int nl = (int)H.lv.size();
-    pband::rb_sweeps(p, s, storage, p->d_e, p->d_rt, omega, nu, false, first_done);
-    pband::residual_field(p, s, storage, p->d_e, p->d_rt, p->d_r);
-    restrict0_kernel<<<grid_of(na * 512), kT, 0, s>>>(na, p->d_blocks, p->dom, p->d_r, H.lv[0].b);
+    band_before(p, s, storage, H.nb27, H.slot27, omega, nu, extra, H.lv[0].b);
     for (int k = 0; k + 1 < nl; ++k) {
         const Level &L = H.lv[k];
         smooth(p, L, s, omega, nu, false, true);
@@ -969,15 +867,7 @@ void vcycle(msbg_poisson *p, hipStream_t s, int storage, float omega, int nu, bo
         prolong_to(p, H.lv[k + 1], L, s);
         smooth(p, L, s, omega, nu, true, false);
     }
-    const int g = (int)na;  // a work-group per listed block
-    if (storage == MSBG_STORAGE_F32)
-        prolong0_kernel<MSBG_STORAGE_F32><<<g, 256, 0, s>>>(p->d_blocks, p->dom, H.nb27, H.lv[0].x, (float *)p->d_e);
-    else if (storage == MSBG_STORAGE_F16)
-        prolong0_kernel<MSBG_STORAGE_F16><<<g, 256, 0, s>>>(p->d_blocks, p->dom, H.nb27, H.lv[0].x, (uint16_t *)p->d_e);
-    else
-        prolong0_kernel<MSBG_STORAGE_BF16><<<g, 256, 0, s>>>(p->d_blocks, p->dom, H.nb27, H.lv[0].x,
-                                                             (uint16_t *)p->d_e);
-    pband::rb_sweeps(p, s, storage, p->d_e, p->d_rt, omega, nu, true);
+    band_after(p, s, storage, H.nb27, H.slot27, omega, nu, extra, H.lv[0].x, x, lo);
 }
 
 }  // namespace mg

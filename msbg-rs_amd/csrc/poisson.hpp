@@ -138,8 +138,6 @@ namespace pband {
 void residual(msbg_poisson *p, hipStream_t s, int storage, const void *x, const void *b, float *r);
 // Copies p->d_norm to the host (synchronizes the library stream).
 int read_norms(msbg_poisson *p, double *r2, double *b2);
-// r = b - A x over the listed cells (FP32), without the norm reduction.
-void residual_field(msbg_poisson *p, hipStream_t s, int storage, const void *x, const void *b, float *r);
 // `sweeps` red-black sweeps in place, colour 0 then 1 (reverse: 1 then 0);
 // skip_first: the first half sweep is already done.
 void rb_sweeps(msbg_poisson *p, hipStream_t s, int storage, void *x, const void *b, float omega, int sweeps,
@@ -154,10 +152,19 @@ int ensure(msbg_poisson *p);
 void release(msbg_poisson *p);
 // Levels including the band itself (0 before ensure).
 int n_levels(const msbg_poisson *p);
-// One V-cycle on A e = rt (p->d_e, p->d_rt in `storage`, e = 0 on entry, or
-// e after the first red half sweep when first_done): nu pre- and
-// post-smoothing red-black sweeps per level; p->d_r is scratch.
-void vcycle(msbg_poisson *p, hipStream_t s, int storage, float omega, int nu, bool first_done);
+// One V-cycle on A e = rt, rt = r / scale * extra of the residual in p->d_r,
+// from e = 0, and x (or the pair x + lo) += scale / extra * e: nu pre- and
+// post-smoothing red-black sweeps per level, fields of the band in `storage`.
+// p->d_e and p->d_rt are scratch, and so is p->d_r once rt is formed.
+void vcycle(msbg_poisson *p, hipStream_t s, int storage, float omega, int nu, float extra, float *x, float *lo);
+// The band level's part before the coarse correction (scaling, pre-smoothing,
+// restricted residual into b1) and after it (correction x1, post-smoothing,
+// update of the iterate).  nb27 / slot27: listed index and slot of the 27
+// blocks around each listed block, below 0 where not listed.
+void band_before(msbg_poisson *p, hipStream_t s, int storage, const int32_t *nb27, const int32_t *slot27, float omega, int nu, float extra,
+                 float *b1);
+void band_after(msbg_poisson *p, hipStream_t s, int storage, const int32_t *nb27, const int32_t *slot27, float omega, int nu, float extra,
+                const float *x1, float *x, float *lo);
 
 }  // namespace mg
 

@@ -811,17 +811,17 @@ void period(msbg_poisson *p, hipStream_t s, int mode, int storage, float *x, flo
         // leaving 2^12 * 65504 of headroom (entries below rms / 4 become
         // subnormal, an absolute error <= 2^-13 rms).
         const float extra = (mode == 2 && storage == MSBG_STORAGE_F16) ? 0x1p-12f : 1.0f;
-        // the first red half sweep from e = 0 is computed by the scale kernel
-        const bool fold = sweeps > 0;
-        ir_scale(p, s, storage, extra, fold ? omega / 6.0f : 0.0f);
-        if (mode == 2)
-            mg::vcycle(p, s, storage, omega, sweeps, fold);
-        else
-            pband::rb_sweeps(p, s, storage, p->d_e, p->d_rt, omega, sweeps, false, fold);
-        if (lo)
-            ir_update_pair(p, s, storage, x, lo, extra);
-        else
-            ir_update(p, s, storage, x, extra);
+        if (mode == 2) {
+            mg::vcycle(p, s, storage, omega, sweeps, extra, x, lo);
+        } else {
+            // the first red half sweep from e = 0 is computed by the scale kernel
+            ir_scale(p, s, storage, extra, omega / 6.0f);
+            pband::rb_sweeps(p, s, storage, p->d_e, p->d_rt, omega, sweeps, false, true);
+            if (lo)
+                ir_update_pair(p, s, storage, x, lo, extra);
+            else
+                ir_update(p, s, storage, x, extra);
+        }
         residual_of(p, s, x, lo, b, p->d_r);
     }
 }
@@ -863,25 +863,6 @@ int run_period_graph(msbg_poisson *p, int mode, int storage, float *x, float *lo
 
 namespace msbg {
 namespace pband {
-
-template <int ST>
-void residual_field_st(msbg_poisson *p, hipStream_t s, const void *x, const void *b, float *r) {
-    using T = typename Sto<ST>::T;
-    with_z<ST>(p, [&](auto zc) {
-        constexpr int Z = decltype(zc)::value;
-        residual_kernel<ST, Z><<<col_groups<ST, Z>(p), kThreads, 0, s>>>(p->d_blocks, p->dom, (const T *)x,
-                                                                          (const T *)b, r, p->d_partial);
-    });
-}
-
-void residual_field(msbg_poisson *p, hipStream_t s, int st, const void *x, const void *b, float *r) {
-    if (st == MSBG_STORAGE_F32)
-        residual_field_st<MSBG_STORAGE_F32>(p, s, x, b, r);
-    else if (st == MSBG_STORAGE_F16)
-        residual_field_st<MSBG_STORAGE_F16>(p, s, x, b, r);
-    else
-        residual_field_st<MSBG_STORAGE_BF16>(p, s, x, b, r);
-}
 
 void rb_sweeps(msbg_poisson *p, hipStream_t s, int st, void *x, const void *b, float omega, int sweeps,
                bool reverse, bool skip_first) {

@@ -215,3 +215,130 @@ def test_closed_box_without_dirichlet_faces_ends_cleanly(pkg, hip):
     st = pb.solve(dx, db, storage=0, multigrid=True, omega=1.0, sweeps_per_check=2, max_sweeps=4 * 40, tol=1e-5)
     assert st["converged"], st
     assert np.all(np.isfinite(dx.get()))
+
+
+# ---- one V-cycle in dense float64 arithmetic --------------------------------
+def _shifted(a, axis, step, fill):
+    """a at the neighbour `step` along axis; `fill` beyond the array."""
+    out = np.full_like(a, fill)
+    src, dst = [slice(None)] * 3, [slice(None)] * 3
+    src[axis], dst[axis] = (slice(1, None), slice(None, -1)) if step > 0 else (slice(None, -1), slice(1, None))
+    out[tuple(dst)] = a[tuple(src)]
+    return out
+
+
+FACES = [(a, d) for a in range(3) for d in (-1, 1)]
+
+
+class _Level:
+    """Cells of one level as dense arrays: their links and Dirichlet coefficients."""
+
+    def __init__(self, listed, link, direct):
+        self.m, self.link, self.dir = listed, link, direct
+        self.diag = direct + sum(link)
+        z, y, x = np.indices(listed.shape)
+        self.colour = (x + y + z) & 1
+
+    def residual(self, x, b):
+        s = sum(c * _shifted(x, a, d, 0.0) for (a, d), c in zip(FACES, self.link))
+        return np.where(self.m, b + s - self.diag * x, 0.0)
+
+    def relax(self, x, b, omega, colour, by=None):
+        diag = self.diag if by is None else by
+        on = self.m & (self.colour == colour) & (self.diag > 0)
+        return np.where(on, x + omega * self.residual(x, b) / np.where(diag > 0, diag, 1.0), x)
+
+
+def _structured(listed, w):
+    link, direct = [], np.zeros(listed.shape)
+    for a, d in FACES:
+        inside = _shifted(np.ones(listed.shape), a, d, 0.0) > 0
+        there = _shifted(listed, a, d, False)
+        link.append(np.where(listed & there, 1.0, 0.0))
+        direct += np.where(listed & inside & ~there, w, 0.0)
+    return _Level(listed, link, direct)
+
+
+def _coarse_sum(a):
+    pad = [(0, n & 1) for n in a.shape]
+    a = np.pad(a, pad)
+    return sum(a[i::2, j::2, k::2] for i in (0, 1) for j in (0, 1) for k in (0, 1))
+
+
+def _interpolated(xc, shape):
+    """Trilinear from the coarse cells: weights 3/4 and 1/4 an axis, a partner
+    beyond the domain is the cell itself."""
+    for axis in range(3):
+        n = shape[axis]
+        i = np.arange(n)
+        own, other = i >> 1, np.clip((i >> 1) + np.where(i & 1, 1, -1), 0, xc.shape[axis] - 1)
+        xc = 0.75 * np.take(xc, own, axis) + 0.25 * np.take(xc, other, axis)
+    return xc
+
+
+def dense_cycle(listed_blocks, s, r, omega, nu):
+    """One V-cycle on A e = r from e = 0 (dense (z, y, x) arrays; the block
+    lattice's level is the coarsest)."""
+    shape = tuple(s[::-1])
+    levels = []
+    for l in range(4):
+        n = tuple((k + (1 << l) - 1) >> l for k in shape)
+        e = [np.arange(k) >> (4 - l) for k in n]
+        levels.append(_structured(listed_blocks[np.ix_(*e)], 2.0 / (1.0 + 2.0 ** -l)))
+    f = levels[3]
+    link = []
+    for k, (a, d) in enumerate(FACES):  # the links that leave their block
+        edge = (np.arange(f.m.shape[a]) & 1) == (1 if d > 0 else 0)
+        out = f.link[k] * edge.reshape([-1 if i == a else 1 for i in range(3)])
+        link.append(0.25 * _coarse_sum(out))
+    wr = (2.0 / (1.0 + 2.0 ** -4)) / (2.0 / (1.0 + 2.0 ** -3))
+    levels.append(_Level(listed_blocks, link, 0.25 * wr * _coarse_sum(f.dir)))
+
+    def descend(l, b):
+        L = levels[l]
+        x = np.zeros(b.shape)
+        if l == 4:
+            cells = np.argwhere(L.m)
+            A = np.zeros((len(cells), len(cells)))
+            for i in range(len(cells)):
+                unit = np.zeros(b.shape)
+                unit[tuple(cells[i])] = 1.0
+                A[:, i] = -L.residual(unit, np.zeros(b.shape))[tuple(cells.T)]
+            x[tuple(cells.T)] = np.linalg.solve(A, b[tuple(cells.T)])
+            return x
+        by = np.full(b.shape, 6.0) if l == 0 else None
+        for _ in range(nu):
+            for c in (0, 1):
+                x = L.relax(x, b, omega, c, by)
+        x = x + np.where(L.m, _interpolated(descend(l + 1, 0.5 * _coarse_sum(L.residual(x, b))), b.shape), 0.0)
+        for _ in range(nu):
+            for c in (1, 0):
+                x = L.relax(x, b, omega, c, by)
+        return x
+
+    return descend(0, np.where(levels[0].m, r, 0.0))
+
+
+@pytest.mark.parametrize("s,seed,frac", [((40, 33, 48), 1, 0.7), ((64, 16, 31), 4, 0.6), ((17, 50, 35), 5, 0.8)])
+@pytest.mark.parametrize("storage,tol", [(0, 1e-4), (1, 2e-2), (2, 1.5e-1)])
+@pytest.mark.parametrize("nu,pair", [(1, False), (2, True), (3, False)])
+def test_one_cycle_equals_dense_arithmetic(pkg, orc, hip, s, seed, frac, storage, tol, nu, pair):
+    """One V-cycle from x against the same cycle in dense float64 arithmetic.
+    Bounds, relative to the largest correction: FP32 by the coarsest level's
+    1e-6 solve and some 50 roundings of 2^-24; FP16 / BF16 by a rounding of
+    2^-12 / 2^-9 in each of up to 14 half sweeps and the transfers, which a
+    sweep does not amplify and a V-cycle sums up at most fourfold."""
+    g, active, x, b = band_problem(pkg, *s, seed, frac)
+    r, _, _ = oracle_residual(orc, g, active, np.ascontiguousarray(x), np.ascontiguousarray(b))
+    nb = [(k + 15) // 16 for k in s[::-1]]
+    listed = np.zeros(nb[0] * nb[1] * nb[2], bool)
+    listed[active] = True
+    m = listed_mask(g, active)
+    e = dense_cycle(listed.reshape(nb), s, dense_from_slabs(g.b2s, r, s).astype(np.float64) * m, 1.0, nu)
+    _, pb = setup(pkg, hip, g, active)
+    dx, db = pb.field(0, host=x.reshape(-1)), hip.to_device(np.ascontiguousarray(b))
+    st = pb.solve(dx, db, storage=storage, multigrid=True, omega=1.0, sweeps_per_check=nu, max_sweeps=2 * nu, tol=0.0,
+                  x_lo=pb.field(0) if pair else None)
+    assert st["sweeps"] == 2 * nu and st["levels"] == 5
+    got = dense_from_slabs(g.b2s, dx.get().reshape(-1, 4096).astype(np.float64) - x, s)
+    assert np.abs(got - e)[m].max() <= tol * np.abs(e).max() + 2.0 ** -23 * np.abs(x).max()
