@@ -58,6 +58,7 @@ struct Level {
     int64_t n = 0;     // cells
     float w = 1.0f;    // Dirichlet face coefficient (structured levels)
     float *x = nullptr, *b = nullptr;
+    float *y = nullptr;       // structured levels: x and y take turns
     // cell lists (level >= 4)
     int32_t *nb = nullptr;    // [n][6]: -x, +x, -y, +y, -z, +z linked cell, -1 none
     float *cf = nullptr;      // [n][6]: coefficient of the link
@@ -87,146 +88,6 @@ __device__ __forceinline__ int nb27_at(int dx, int dy, int dz) { return (dz + 1)
 // inside the domain when its first fine cell is.
 __device__ __forceinline__ bool live(const PBlock &B, const Dom &d, int h, int cx, int cy, int cz) {
     return B.ox + cx * h < d.sx && B.oy + cy * h < d.sy && B.oz + cz * h < d.sz;
-}
-
-// (b - A x) at cell (cx, cy, cz) of listed block k on a structured level of
-// B cells per edge (h = 16 / B); *diag_out receives the diagonal.
-template <int B>
-__device__ __forceinline__ float blk_residual(const float *__restrict__ x, const float *__restrict__ b,
-                                              const int32_t *__restrict__ T, const PBlock &Bk, const Dom &d, i64 k,
-                                              int cx, int cy, int cz, float w, float *diag_out) {
-    constexpr int B3 = B * B * B, h = 16 / B;
-    const i64 i = k * B3 + cx + B * (cy + B * cz);
-    const int c[3] = {cx, cy, cz};
-    // Every face's neighbour cell first, then the neighbour blocks of the
-    // faces that leave this block in one batch of loads (they depend on the
-    // cell only), then all six values in one batch: two dependent round trips
-    // instead of one or two per face.  A load whose value goes unused reads a
-    // valid address (the block's centre entry, the block's own cells).
-    int qi[6], tix[6];
-#pragma unroll
-    for (int f = 0; f < 6; ++f) {
-        const int a = f >> 1, dir = (f & 1) ? 1 : -1;
-        int q[3] = {cx, cy, cz}, o[3] = {0, 0, 0};
-        q[a] += dir;
-        if (q[a] < 0) {
-            q[a] += B;
-            o[a] = -1;
-        } else if (q[a] >= B) {
-            q[a] -= B;
-            o[a] = 1;
-        }
-        qi[f] = q[0] + B * (q[1] + B * q[2]);
-        tix[f] = nb27_at(o[0], o[1], o[2]);  // 13 (the block itself) when the face stays inside
-    }
-    int32_t tv[6];
-#pragma unroll
-    for (int f = 0; f < 6; ++f) tv[f] = T[tix[f]];
-    i64 nbk[6];
-#pragma unroll
-    for (int f = 0; f < 6; ++f) nbk[f] = tix[f] == 13 ? k : (i64)tv[f];
-    float xv[6];
-#pragma unroll
-    for (int f = 0; f < 6; ++f) xv[f] = x[(nbk[f] >= 0 ? nbk[f] : k) * B3 + qi[f]];
-    const float bi = b[i], xc = x[i];
-    const int org[3] = {Bk.ox, Bk.oy, Bk.oz}, dom[3] = {d.sx, d.sy, d.sz};
-    float s = 0.0f, dg = 0.0f;
-#pragma unroll
-    for (int f = 0; f < 6; ++f) {
-        const int a = f >> 1, dir = (f & 1) ? 1 : -1;
-        if (dir > 0 && org[a] + (c[a] + 1) * h >= dom[a]) continue;  // beyond the domain: Neumann
-        if (nbk[f] >= 0) {
-            s += xv[f];
-            dg += 1.0f;
-        } else if (nbk[f] == -1) {
-            dg += w;
-        }
-    }
-    *diag_out = dg;
-    return bi + s - dg * xc;
-}
-
-// One half sweep over the cells of one colour: thread j of listed block k
-// takes row j / (B / 2) (y + B z) and the cell of that row with
-// (x + y + z) & 1 == color.
-template <int B>
-__global__ __launch_bounds__(kT) void relax_blk_kernel(i64 n_active, const PBlock *__restrict__ blocks, Dom d,
-                                                       const int32_t *__restrict__ nb27, float *x,
-                                                       const float *__restrict__ b, float w, float omega, int color) {
-    constexpr int B3 = B * B * B, H = B3 / 2;
-    const i64 i = (i64)blockIdx.x * kT + threadIdx.x;
-    if (i >= n_active * H) return;
-    const i64 k = i / H;
-    const int j = (int)(i % H), row = j / (B / 2), cy = row % B, cz = row / B;
-    const int cx = 2 * (j % (B / 2)) + ((cy + cz + color) & 1);  // B even: the block origin keeps the parity
-    const PBlock Bk = blocks[k];
-    if (!live(Bk, d, 16 / B, cx, cy, cz)) return;
-    float dg;
-    const float t = blk_residual<B>(x, b, nb27 + k * 27, Bk, d, k, cx, cy, cz, w, &dg);
-    const i64 c = k * B3 + cx + B * (cy + B * cz);
-    if (dg > 0.0f) x[c] += omega * t / dg;  // dg = 0: a lone cell with Neumann faces only
-}
-
-// The first half sweep from x = 0, over every cell: colour 0 takes
-// omega b / diag, colour 1 (and every cell outside the domain) 0.
-template <int B>
-__global__ __launch_bounds__(kT) void init_blk_kernel(i64 n_active, const PBlock *__restrict__ blocks, Dom d,
-                                                      const int32_t *__restrict__ nb27, float *x,
-                                                      const float *__restrict__ b, float w, float omega) {
-    constexpr int B3 = B * B * B, h = 16 / B;
-    const i64 i = (i64)blockIdx.x * kT + threadIdx.x;
-    if (i >= n_active * B3) return;
-    const i64 k = i / B3;
-    const int v = (int)(i % B3), c[3] = {v % B, (v / B) % B, v / (B * B)};
-    const PBlock Bk = blocks[k];
-    float out = 0.0f;
-    if (((c[0] + c[1] + c[2]) & 1) == 0 && live(Bk, d, h, c[0], c[1], c[2])) {
-        const int32_t *T = nb27 + k * 27;
-        const int org[3] = {Bk.ox, Bk.oy, Bk.oz}, dom[3] = {d.sx, d.sy, d.sz};
-        float dg = 0.0f;
-#pragma unroll
-        for (int f = 0; f < 6; ++f) {
-            const int a = f >> 1, dir = (f & 1) ? 1 : -1;
-            if (dir > 0 && org[a] + (c[a] + 1) * h >= dom[a]) continue;
-            const int q = c[a] + dir;
-            if (q >= 0 && q < B) {
-                dg += 1.0f;
-                continue;
-            }
-            const int32_t nbk = T[nb27_at(a == 0 ? dir : 0, a == 1 ? dir : 0, a == 2 ? dir : 0)];
-            dg += nbk >= 0 ? 1.0f : (nbk == -1 ? w : 0.0f);
-        }
-        if (dg > 0.0f) out = omega * b[i] / dg;
-    }
-    x[i] = out;
-}
-
-// b_c = 0.5 * sum of the residuals of its children (structured level of B
-// cells per edge into the level of B / 2; B = 2 gives one cell per block).
-// Lane 8 j + o evaluates child o of coarse cell j; the 8 lanes of a coarse
-// cell sum by shuffles in a fixed order.
-template <int B>
-__global__ __launch_bounds__(kT) void restrict_blk_kernel(i64 n_active, const PBlock *__restrict__ blocks, Dom d,
-                                                          const int32_t *__restrict__ nb27,
-                                                          const float *__restrict__ x, const float *__restrict__ b,
-                                                          float w, float *bc) {
-    constexpr int C = B / 2, C3 = C * C * C;
-    const i64 t = (i64)blockIdx.x * kT + threadIdx.x;
-    const i64 i = t >> 3;  // coarse cell
-    const int o = (int)(t & 7);
-    float r = 0.0f;
-    if (i < n_active * C3) {
-        const i64 k = i / C3;
-        const int v = (int)(i % C3), ux = v % C, uy = (v / C) % C, uz = v / (C * C);
-        const PBlock Bk = blocks[k];
-        const int fx = 2 * ux + (o & 1), fy = 2 * uy + ((o >> 1) & 1), fz = 2 * uz + (o >> 2);
-        float dg;
-        if (live(Bk, d, 16 / B, fx, fy, fz)) r = blk_residual<B>(x, b, nb27 + k * 27, Bk, d, k, fx, fy, fz, w, &dg);
-    }
-    r += __shfl_xor(r, 1);
-    r += __shfl_xor(r, 2);
-    r += __shfl_xor(r, 4);
-    if (o == 0 && i < n_active * C3) bc[i] = 0.5f * r;
 }
 
 // Trilinear value at fine cell (cx, cy, cz) of listed block k from the
@@ -493,65 +354,17 @@ __global__ void slot27_kernel(const int32_t *__restrict__ nb27, const PBlock *__
 
 int grid_of(i64 n) { return (int)((n + kT - 1) / kT); }
 
-// nu red-black sweeps (colour 0 then 1; rev: 1 then 0); from_zero: x = 0 on
-// entry, the first half sweep written without reading x.
-template <int B>
-void smooth_blk(const msbg_poisson *p, const Level &L, hipStream_t s, float omega, int nu, bool rev, bool from_zero) {
-    const int g = grid_of(L.n / 2);
+// nu red-black sweeps of a cell list (colour 0 then 1; rev: 1 then 0);
+// from_zero: x = 0 on entry, the first half sweep written without reading x.
+void smooth_list(const Level &L, hipStream_t s, float omega, int nu, bool rev, bool from_zero) {
     for (int it = 0; it < nu; ++it)
         for (int h = 0; h < 2; ++h) {
             if (from_zero && it == 0 && h == 0)
-                init_blk_kernel<B><<<grid_of(L.n), kT, 0, s>>>(p->n_active, p->d_blocks, p->dom, p->mg->nb27, L.x,
-                                                                L.b, L.w, omega);
+                init_list_kernel<<<grid_of(L.n), kT, 0, s>>>(L.n, L.diag, L.col, L.x, L.b, omega);
             else
-                relax_blk_kernel<B><<<g, kT, 0, s>>>(p->n_active, p->d_blocks, p->dom, p->mg->nb27, L.x, L.b, L.w,
-                                                     omega, rev ? 1 - h : h);
+                relax_list_kernel<<<grid_of(L.n), kT, 0, s>>>(L.n, L.nb, L.cf, L.diag, L.col, L.x, L.b, omega,
+                                                              rev ? 1 - h : h);
         }
-}
-
-void smooth(const msbg_poisson *p, const Level &L, hipStream_t s, float omega, int nu, bool rev, bool from_zero) {
-    if (L.B == 8)
-        smooth_blk<8>(p, L, s, omega, nu, rev, from_zero);
-    else if (L.B == 4)
-        smooth_blk<4>(p, L, s, omega, nu, rev, from_zero);
-    else if (L.B == 2)
-        smooth_blk<2>(p, L, s, omega, nu, rev, from_zero);
-    else
-        for (int it = 0; it < nu; ++it)
-            for (int h = 0; h < 2; ++h) {
-                if (from_zero && it == 0 && h == 0)
-                    init_list_kernel<<<grid_of(L.n), kT, 0, s>>>(L.n, L.diag, L.col, L.x, L.b, omega);
-                else
-                    relax_list_kernel<<<grid_of(L.n), kT, 0, s>>>(L.n, L.nb, L.cf, L.diag, L.col, L.x, L.b, omega,
-                                                                  rev ? 1 - h : h);
-            }
-}
-
-void restrict_to(const msbg_poisson *p, const Level &F, const Level &Cl, hipStream_t s) {
-    const i64 na = p->n_active;
-    const int32_t *T = p->mg->nb27;
-    const int g8 = grid_of(8 * Cl.n);  // a lane per child
-    if (F.B == 8)
-        restrict_blk_kernel<8><<<g8, kT, 0, s>>>(na, p->d_blocks, p->dom, T, F.x, F.b, F.w, Cl.b);
-    else if (F.B == 4)
-        restrict_blk_kernel<4><<<g8, kT, 0, s>>>(na, p->d_blocks, p->dom, T, F.x, F.b, F.w, Cl.b);
-    else if (F.B == 2)
-        restrict_blk_kernel<2><<<g8, kT, 0, s>>>(na, p->d_blocks, p->dom, T, F.x, F.b, F.w, Cl.b);
-    else
-        restrict_list_kernel<<<grid_of(Cl.n), kT, 0, s>>>(Cl.n, Cl.ch, F.nb, F.cf, F.diag, F.x, F.b, Cl.b);
-}
-
-void prolong_to(const msbg_poisson *p, const Level &Cl, const Level &F, hipStream_t s) {
-    const i64 na = p->n_active;
-    const int32_t *T = p->mg->nb27;
-    if (F.B == 8)
-        prolong_blk_kernel<8><<<grid_of(F.n), kT, 0, s>>>(na, p->d_blocks, p->dom, T, Cl.x, F.x);
-    else if (F.B == 4)
-        prolong_blk_kernel<4><<<grid_of(F.n), kT, 0, s>>>(na, p->d_blocks, p->dom, T, Cl.x, F.x);
-    else if (F.B == 2)
-        prolong_blk_kernel<2><<<grid_of(F.n), kT, 0, s>>>(na, p->d_blocks, p->dom, T, Cl.x, F.x);
-    else
-        prolong_list_kernel<<<grid_of(F.n), kT, 0, s>>>(F.n, F.pn, Cl.x, F.x);
 }
 
 // ---- host construction -----------------------------------------------------
@@ -765,6 +578,7 @@ void release(msbg_poisson *p) {
     Hierarchy *H = p->mg;
     for (Level &L : H->lv) {
         (void)hipFree(L.x);
+        (void)hipFree(L.y);
         (void)hipFree(L.b);
         (void)hipFree(L.nb);
         (void)hipFree(L.cf);
@@ -813,6 +627,7 @@ int ensure(msbg_poisson *p) {
         L.n = na * L.B * L.B * L.B;
         L.w = dirichlet_coef(l);
         e = hipMalloc(&L.x, sizeof(float) * L.n);
+        if (e == hipSuccess) e = hipMalloc(&L.y, sizeof(float) * L.n);
         if (e == hipSuccess) e = hipMalloc(&L.b, sizeof(float) * L.n);
         H->lv.push_back(L);
     }
@@ -854,20 +669,35 @@ void vcycle(msbg_poisson *p, hipStream_t s, int storage, float omega, int nu, fl
     const int nl = (int)H.lv.size();
     band_before(p, s, storage, H.nb27, H.slot27, omega, nu, extra, H.lv[0].b);
     for (int k = 0; k + 1 < nl; ++k) {
-        const Level &L = H.lv[k];
-        smooth(p, L, s, omega, nu, false, true);
-        restrict_to(p, L, H.lv[k + 1], s);
+        const Level &L = H.lv[k], &C = H.lv[k + 1];
+        if (L.B) {
+            level_before(p, s, H.nb27, L.B, L.w, omega, nu, L.x, L.y, L.b, C.b);
+        } else {
+            smooth_list(L, s, omega, nu, false, true);
+            restrict_list_kernel<<<grid_of(C.n), kT, 0, s>>>(C.n, C.ch, L.nb, L.cf, L.diag, L.x, L.b, C.b);
+        }
     }
     const Level &Lc = H.lv[nl - 1];
     const int cg_threads = (int)std::min<i64>(kCoarseMax, std::max<i64>(64, (Lc.n + 63) / 64 * 64));
     coarse_cg_kernel<<<1, cg_threads, 0, s>>>((int)Lc.n, Lc.nb, Lc.cf, Lc.diag, Lc.b, Lc.x, Lc.comp, Lc.sing,
                                               Lc.n_comp, Lc.n_sing);
+    const float *xc = Lc.x;  // the next coarser level's result
     for (int k = nl - 2; k >= 0; --k) {
         const Level &L = H.lv[k];
-        prolong_to(p, H.lv[k + 1], L, s);
-        smooth(p, L, s, omega, nu, true, false);
+        if (L.B == 2) {
+            // its neighbours' cells interpolate from blocks beyond the 27
+            float *x = level_field(L.x, L.y, nu);
+            prolong_blk_kernel<2><<<grid_of(L.n), kT, 0, s>>>(p->n_active, p->d_blocks, p->dom, H.nb27, xc, x);
+            xc = level_after(p, s, H.nb27, L.B, L.w, omega, nu, L.x, L.y, L.b, nullptr);
+        } else if (L.B) {
+            xc = level_after(p, s, H.nb27, L.B, L.w, omega, nu, L.x, L.y, L.b, xc);
+        } else {
+            prolong_list_kernel<<<grid_of(L.n), kT, 0, s>>>(L.n, L.pn, xc, L.x);
+            smooth_list(L, s, omega, nu, true, false);
+            xc = L.x;
+        }
     }
-    band_after(p, s, storage, H.nb27, H.slot27, omega, nu, extra, H.lv[0].x, x, lo);
+    band_after(p, s, storage, H.nb27, H.slot27, omega, nu, extra, xc, x, lo);
 }
 
 }  // namespace mg

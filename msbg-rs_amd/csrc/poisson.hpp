@@ -165,6 +165,16 @@ void band_before(msbg_poisson *p, hipStream_t s, int storage, const int32_t *nb2
                  float *b1);
 void band_after(msbg_poisson *p, hipStream_t s, int storage, const int32_t *nb27, const int32_t *slot27, float omega, int nu, float extra,
                 const float *x1, float *x, float *lo);
+// The same on a structured level of B = 8, 4 or 2 cells per block edge (fields
+// x and y in turn; Dirichlet coefficient w): before the coarse correction (the
+// restricted residual into bc), after it (correction xc, or none where it is
+// added already; returns the field that holds the result).
+void level_before(const msbg_poisson *p, hipStream_t s, const int32_t *nb27, int B, float w, float omega, int nu,
+                  float *x, float *y, const float *b, float *bc);
+const float *level_after(const msbg_poisson *p, hipStream_t s, const int32_t *nb27, int B, float w, float omega, int nu,
+                         float *x, float *y, const float *b, const float *xc);
+// The field that level_before leaves its result in.
+inline float *level_field(float *x, float *y, int nu) { return (nu & 1) ? x : y; }
 
 }  // namespace mg
 
