@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -15,6 +16,21 @@ namespace msbg {
 int fail(int code, const std::string &msg);
 int hip_fail(hipError_t e, const char *what);
 hipStream_t stream();
+
+// The stream that graphs are captured on: one per device, made on first use and
+// kept (a stream of its own per object cost 0.4 ms to make).  Holds a lock
+// while it lives, so captures of several threads take turns.
+class Capture {
+public:
+    Capture();
+    hipStream_t stream() const { return s_; }  // null: see error()
+    hipError_t error() const { return e_; }
+
+private:
+    std::lock_guard<std::mutex> lock_;
+    hipStream_t s_ = nullptr;
+    hipError_t e_ = hipSuccess;
+};
 
 #define MSBG_HIP(call)                                          \
     do {                                                        \

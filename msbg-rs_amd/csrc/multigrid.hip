@@ -44,6 +44,7 @@
 #include <vector>
 
 #include "poisson.hpp"
+#include "primitives.hpp"
 
 namespace msbg {
 namespace mg {
@@ -346,10 +347,31 @@ __global__ __launch_bounds__(kCoarseMax) void coarse_cg_kernel(int n, const int3
     if (in) x[t] = (float)xi;
 }
 
-__global__ void slot27_kernel(const int32_t *__restrict__ nb27, const PBlock *__restrict__ blocks, i64 n,
-                              int32_t *__restrict__ slot27) {
+// The listed index of every block (-1 where not listed), and from it the
+// listed index and slot of the 27 blocks around each listed block (-1 where not
+// listed, -2 and -1 beyond the lattice).
+__global__ void unlisted_kernel(int32_t *index, i64 n) {
     const i64 i = (i64)blockIdx.x * kT + threadIdx.x;
-    if (i < n) slot27[i] = nb27[i] >= 0 ? blocks[nb27[i]].slot : -1;
+    if (i < n) index[i] = -1;
+}
+__global__ void listed_kernel(const PBlock *__restrict__ blocks, i64 n, int nx, int ny, int32_t *index) {
+    const i64 k = (i64)blockIdx.x * kT + threadIdx.x;
+    if (k >= n) return;
+    const PBlock B = blocks[k];
+    index[(B.ox >> 4) + (i64)nx * ((B.oy >> 4) + (i64)ny * (B.oz >> 4))] = (int32_t)k;
+}
+__global__ void neighbours_kernel(const PBlock *__restrict__ blocks, i64 n, int nx, int ny, int nz,
+                                  const int32_t *__restrict__ index, int32_t *__restrict__ nb27,
+                                  int32_t *__restrict__ slot27) {
+    const i64 i = (i64)blockIdx.x * kT + threadIdx.x;
+    if (i >= n * 27) return;
+    const int t = (int)(i % 27);
+    const PBlock B = blocks[i / 27];
+    const int x = (B.ox >> 4) + t % 3 - 1, y = (B.oy >> 4) + (t / 3) % 3 - 1, z = (B.oz >> 4) + t / 9 - 1;
+    int32_t v = -2;
+    if (x >= 0 && x < nx && y >= 0 && y < ny && z >= 0 && z < nz) v = index[x + (i64)nx * (y + (i64)ny * z)];
+    nb27[i] = v;
+    slot27[i] = v >= 0 ? blocks[v].slot : -1;
 }
 
 int grid_of(i64 n) { return (int)((n + kT - 1) / kT); }
@@ -394,56 +416,64 @@ bool in_domain(const msbg_poisson *p, int l, const int64_t q[3]) {
     return true;
 }
 
-// Level 3 (2^3 cells per listed block) as a cell list, index k 8 + x + 2 y + 4 z.
-void level3_op(const msbg_poisson *p, HostOp &H) {
-    const i64 na = p->n_active;
-    H.l = 3;
-    H.dims[0] = 2 * p->nx;
-    H.dims[1] = 2 * p->ny;
-    H.dims[2] = 2 * p->nz;
-    H.pos.assign((size_t)na * 24, 0);
-    H.alive.assign((size_t)na * 8, 0);
-    H.dense.assign((size_t)(H.dims[0] * H.dims[1] * H.dims[2]), -1);
-    for (i64 k = 0; k < na; ++k) {
+// Level 4, one cell per listed block (cell k is block k): the Galerkin product
+// of level 3's operator (2^3 cells per block), whose cells all have the same
+// links but for the domain's bound and the unlisted blocks, so it is written
+// down per block without level 3's list (37,000 blocks: 0.6 ms, 4 ms through
+// the list).
+void level4_op(const msbg_poisson *p, HostOp &H) {
+    const size_t na = (size_t)p->n_active;
+    const int64_t dims[3] = {p->nx, p->ny, p->nz}, s[3] = {p->dom.sx, p->dom.sy, p->dom.sz};
+    const int64_t stride[3] = {1, dims[0], dims[0] * dims[1]};
+    H.l = 4;
+    H.dense.assign((size_t)(dims[0] * dims[1] * dims[2]), -1);
+    H.pos.resize(na * 3);
+    H.alive.assign(na, 1);
+    H.nb.assign(na * 6, -1);
+    H.cf.assign(na * 6, 0.0f);
+    H.dir.assign(na, 0.0f);
+    for (int a = 0; a < 3; ++a) H.dims[a] = dims[a];
+    for (size_t k = 0; k < na; ++k) H.dense[(size_t)p->bids[k]] = (int32_t)k;
+    const float w = dirichlet_coef(3), part = 0.25f * (dirichlet_coef(4) / dirichlet_coef(3));
+    for (size_t k = 0; k < na; ++k) {
         const int64_t bid = p->bids[k];
-        const int64_t bx = bid % p->nx, by = (bid / p->nx) % p->ny, bz = bid / (p->nx * p->ny);
-        for (int c = 0; c < 8; ++c) {
-            const size_t i = (size_t)k * 8 + c;
-            const int64_t q[3] = {2 * bx + (c & 1), 2 * by + ((c >> 1) & 1), 2 * bz + (c >> 2)};
-            for (int a = 0; a < 3; ++a) H.pos[i * 3 + a] = (int32_t)q[a];
-            if (in_domain(p, 3, q)) {
-                H.alive[i] = 1;
-                H.dense[H.at(q[0], q[1], q[2])] = (int32_t)i;
-            }
+        const int64_t b[3] = {bid % dims[0], (bid / dims[0]) % dims[1], bid / (dims[0] * dims[1])};
+        int children[3];  // along each axis, inside the domain
+        for (int a = 0; a < 3; ++a) {
+            H.pos[k * 3 + a] = (int32_t)b[a];
+            children[a] = (2 * b[a] + 1) << 3 < s[a] ? 2 : 1;
         }
-    }
-    const float w = dirichlet_coef(3);
-    H.nb.assign(H.n() * 6, -1);
-    H.cf.assign(H.n() * 6, 0.0f);
-    H.dir.assign(H.n(), 0.0f);
-    for (size_t i = 0; i < H.n(); ++i) {
-        if (!H.alive[i]) continue;
+        bool open[6], any = false;  // faces towards an unlisted block
         for (int f = 0; f < 6; ++f) {
-            int64_t q[3] = {H.pos[i * 3], H.pos[i * 3 + 1], H.pos[i * 3 + 2]};
-            q[f >> 1] += (f & 1) ? 1 : -1;
-            if (!in_domain(p, 3, q)) continue;  // Neumann
-            const int32_t j = H.dense[H.at(q[0], q[1], q[2])];
-            if (j >= 0) {
-                H.nb[i * 6 + f] = j;
-                H.cf[i * 6 + f] = 1.0f;
-            } else {
-                H.dir[i] += w;
-            }
+            const int a = f >> 1;
+            open[f] = false;
+            const int64_t q = b[a] + ((f & 1) ? 1 : -1);
+            if (q < 0 || q >= dims[a]) continue;  // the domain's bound
+            const int32_t j = H.dense[(size_t)(bid + ((f & 1) ? stride[a] : -stride[a]))];
+            open[f] = j < 0;
+            any = any || open[f];
+            if (j < 0) continue;
+            H.nb[k * 6 + f] = j;
+            H.cf[k * 6 + f] = 0.25f * (float)(children[(a + 1) % 3] * children[(a + 2) % 3]);
         }
+        if (!any) continue;
+        for (int z = 0; z < children[2]; ++z)
+            for (int y = 0; y < children[1]; ++y)
+                for (int x = 0; x < children[0]; ++x) {
+                    const int c[3] = {x, y, z};
+                    float d = 0.0f;
+                    for (int f = 0; f < 6; ++f)
+                        if (open[f] && c[f >> 1] == (f & 1)) d += w;
+                    H.dir[k] += part * d;
+                }
     }
 }
 
-// The next coarser level of F (Galerkin / 4) and, with `tables`, its child
-// table and F's interpolation table (level 4 needs neither: its transfers are
-// the structured kernels).  Coarse cells are numbered in the order of their
-// first child, so level 4's cell k is listed block k.
+// The next coarser level of F (Galerkin / 4), its child table and F's
+// interpolation table.  Coarse cells are numbered in the order of their first
+// child.
 void aggregate(const msbg_poisson *p, const HostOp &F, HostOp &Cl, std::vector<int32_t> &ch,
-               std::vector<int32_t> &pn, bool tables = true) {
+               std::vector<int32_t> &pn) {
     Cl.l = F.l + 1;
     for (int a = 0; a < 3; ++a) Cl.dims[a] = (F.dims[a] + 1) >> 1;
     Cl.dense.assign((size_t)(Cl.dims[0] * Cl.dims[1] * Cl.dims[2]), -1);
@@ -476,9 +506,6 @@ void aggregate(const msbg_poisson *p, const HostOp &F, HostOp &Cl, std::vector<i
             Cl.cf[(size_t)c * 6 + f] += 0.25f * F.cf[i * 6 + f];
         }
     }
-    ch.clear();
-    pn.clear();
-    if (!tables) return;
     ch.assign(nc * 8, -1);
     for (size_t c = 0; c < nc; ++c)
         for (int o = 0; o < 8; ++o) {
@@ -600,24 +627,22 @@ int ensure(msbg_poisson *p) {
     const i64 na = p->n_active;
     Hierarchy *H = new Hierarchy();
     p->mg = H;
-    // each listed block's 27 neighbours (listed index, -1 unlisted, -2 beyond the lattice)
-    std::vector<int32_t> lidx((size_t)p->n_blocks, -1);
-    for (i64 k = 0; k < na; ++k) lidx[p->bids[k]] = (int32_t)k;
-    std::vector<int32_t> nb27((size_t)na * 27);
-    for (i64 k = 0; k < na; ++k) {
-        const int64_t bid = p->bids[k];
-        const int64_t bx = bid % p->nx, by = (bid / p->nx) % p->ny, bz = bid / (p->nx * p->ny);
-        for (int t = 0; t < 27; ++t) {
-            const int64_t x = bx + t % 3 - 1, y = by + (t / 3) % 3 - 1, z = bz + t / 9 - 1;
-            int32_t v = -2;
-            if (x >= 0 && x < p->nx && y >= 0 && y < p->ny && z >= 0 && z < p->nz) v = lidx[x + p->nx * (y + p->ny * z)];
-            nb27[(size_t)k * 27 + t] = v;
-        }
+    // each listed block's 27 neighbours
+    int rc;
+    int32_t *index = (int32_t *)workspace(21, sizeof(int32_t) * (size_t)p->n_blocks, &rc);
+    if (rc) {
+        release(p);
+        return rc;
     }
-    hipError_t e = upload(&H->nb27, nb27);
-    if (e == hipSuccess) e = hipMalloc(&H->slot27, sizeof(int32_t) * nb27.size());
+    const size_t n27 = (size_t)na * 27;
+    hipError_t e = hipMalloc(&H->nb27, sizeof(int32_t) * n27);
+    if (e == hipSuccess) e = hipMalloc(&H->slot27, sizeof(int32_t) * n27);
     if (e == hipSuccess) {
-        slot27_kernel<<<grid_of((i64)nb27.size()), kT, 0, stream()>>>(H->nb27, p->d_blocks, (i64)nb27.size(), H->slot27);
+        const int nx = (int)p->nx, ny = (int)p->ny, nz = (int)p->nz;
+        unlisted_kernel<<<grid_of(p->n_blocks), kT, 0, stream()>>>(index, p->n_blocks);
+        listed_kernel<<<grid_of(na), kT, 0, stream()>>>(p->d_blocks, na, nx, ny, index);
+        neighbours_kernel<<<grid_of((i64)n27), kT, 0, stream()>>>(p->d_blocks, na, nx, ny, nz, index, H->nb27,
+                                                                 H->slot27);
         e = hipGetLastError();
     }
     for (int l = 1; l <= 3 && e == hipSuccess; ++l) {
@@ -632,10 +657,9 @@ int ensure(msbg_poisson *p) {
         H->lv.push_back(L);
     }
     // cell lists: level 4 (one cell per block) and coarser, to <= kCoarseMax cells
-    HostOp fine, cur;
-    level3_op(p, fine);
+    HostOp cur;
+    level4_op(p, cur);
     std::vector<int32_t> ch, pn;
-    aggregate(p, fine, cur, ch, pn, false);  // level 4; its children are level 3's structured cells
     bool first = true;
     while (e == hipSuccess) {
         Level L;

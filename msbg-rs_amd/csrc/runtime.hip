@@ -23,6 +23,17 @@ int hip_fail(hipError_t e, const char *what) {
 
 hipStream_t stream() { return g_stream; }
 
+static std::mutex g_capture_lock;
+static hipStream_t g_capture[64] = {nullptr};
+
+Capture::Capture() : lock_(g_capture_lock) {
+    int dev = 0;
+    e_ = hipGetDevice(&dev);
+    if (e_ == hipSuccess && (dev < 0 || dev >= 64)) e_ = hipErrorInvalidDevice;
+    if (e_ == hipSuccess && !g_capture[dev]) e_ = hipStreamCreateWithFlags(&g_capture[dev], hipStreamNonBlocking);
+    if (e_ == hipSuccess) s_ = g_capture[dev];
+}
+
 // Fills n floats with v (a kernel, not hipMemset, so it can sit in a graph).
 __global__ void fill_f32_kernel(float *p, int64_t n, float v) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;

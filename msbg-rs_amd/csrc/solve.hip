@@ -835,11 +835,12 @@ int run_period_graph(msbg_poisson *p, int mode, int storage, float *x, float *lo
           p->g_x == x && p->g_lo == lo && p->g_b == b)) {
         drop_graph(p);
         if (!p->g_done) MSBG_HIP(hipEventCreateWithFlags(&p->g_done, hipEventDisableTiming));
-        if (!p->cap_stream) MSBG_HIP(hipStreamCreateWithFlags(&p->cap_stream, hipStreamNonBlocking));
-        MSBG_HIP(hipStreamBeginCapture(p->cap_stream, hipStreamCaptureModeRelaxed));
-        period(p, p->cap_stream, mode, storage, x, lo, b, omega, sweeps);
+        Capture capture;
+        MSBG_HIP(capture.error());
+        MSBG_HIP(hipStreamBeginCapture(capture.stream(), hipStreamCaptureModeRelaxed));
+        period(p, capture.stream(), mode, storage, x, lo, b, omega, sweeps);
         hipGraph_t graph = nullptr;
-        hipError_t e = hipStreamEndCapture(p->cap_stream, &graph);
+        hipError_t e = hipStreamEndCapture(capture.stream(), &graph);
         MSBG_HIP(e);
         e = hipGraphInstantiate(&p->exec, graph, nullptr, nullptr, 0);
         (void)hipGraphDestroy(graph);
@@ -959,7 +960,6 @@ int msbg_poisson_free(msbg_poisson *p) {
     mg::release(p);
     if (p->g_done) (void)hipEventDestroy(p->g_done);
     if (p->j_done) (void)hipEventDestroy(p->j_done);
-    if (p->cap_stream) (void)hipStreamDestroy(p->cap_stream);
     (void)hipFree(p->d_blocks);
     (void)hipFree(p->d_partial);
     (void)hipFree(p->d_norm);
@@ -1008,14 +1008,15 @@ int msbg_poisson_jacobi_sweeps(msbg_poisson *p, int storage, void *x, void *tmp,
           p->j_t == tmp && p->j_b == b)) {
         drop_jacobi_graph(p);
         if (!p->j_done) MSBG_HIP(hipEventCreateWithFlags(&p->j_done, hipEventDisableTiming));
-        if (!p->cap_stream) MSBG_HIP(hipStreamCreateWithFlags(&p->cap_stream, hipStreamNonBlocking));
-        MSBG_HIP(hipStreamBeginCapture(p->cap_stream, hipStreamCaptureModeRelaxed));
+        Capture capture;
+        MSBG_HIP(capture.error());
+        MSBG_HIP(hipStreamBeginCapture(capture.stream(), hipStreamCaptureModeRelaxed));
         for (int i = 0; i < sweeps; i += 2) {
-            relax(p, p->cap_stream, storage, x, tmp, b, omega, 0, false);
-            relax(p, p->cap_stream, storage, tmp, x, b, omega, 0, false);
+            relax(p, capture.stream(), storage, x, tmp, b, omega, 0, false);
+            relax(p, capture.stream(), storage, tmp, x, b, omega, 0, false);
         }
         hipGraph_t graph = nullptr;
-        MSBG_HIP(hipStreamEndCapture(p->cap_stream, &graph));
+        MSBG_HIP(hipStreamEndCapture(capture.stream(), &graph));
         hipError_t e = hipGraphInstantiate(&p->jexec, graph, nullptr, nullptr, 0);
         (void)hipGraphDestroy(graph);
         if (e != hipSuccess) p->jexec = nullptr;

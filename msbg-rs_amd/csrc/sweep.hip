@@ -997,7 +997,6 @@ struct msbg_sweep_plan {
         uint64_t last_use = 0;
     };
     static constexpr int kGraphCache = 4;
-    hipStream_t cap_stream = nullptr;
     GraphEntry graphs[kGraphCache];
     uint64_t graph_clock = 0;
 };
@@ -1576,7 +1575,6 @@ int msbg_sweep_plan_new_multires(msbg_grid *fine, const msbg_grid *coarse, const
 int msbg_sweep_plan_free(msbg_sweep_plan *p) {
     if (!p) return MSBG_OK;
     drop_graphs(p);
-    if (p->cap_stream) (void)hipStreamDestroy(p->cap_stream);
     if (p->d_bids) (void)hipFree(p->d_bids);
     for (int32_t *t : p->d_topo)
         if (t) (void)hipFree(t);
@@ -1616,11 +1614,12 @@ int msbg_sweep_plan_run_graph_async(msbg_sweep_plan *p, int stencil, float dt, i
         hit = lru;
         drop_graph(*hit);
         if (!hit->done) MSBG_HIP(hipEventCreateWithFlags(&hit->done, hipEventDisableTiming));
-        if (!p->cap_stream) MSBG_HIP(hipStreamCreateWithFlags(&p->cap_stream, hipStreamNonBlocking));
-        MSBG_HIP(hipStreamBeginCapture(p->cap_stream, hipStreamCaptureModeRelaxed));
-        rc = launch_iterations(p, p->cap_stream, stencil, dt, iterations, clamp01);
+        Capture capture;
+        MSBG_HIP(capture.error());
+        MSBG_HIP(hipStreamBeginCapture(capture.stream(), hipStreamCaptureModeRelaxed));
+        rc = launch_iterations(p, capture.stream(), stencil, dt, iterations, clamp01);
         hipGraph_t graph = nullptr;
-        hipError_t e = hipStreamEndCapture(p->cap_stream, &graph);
+        hipError_t e = hipStreamEndCapture(capture.stream(), &graph);
         if (rc) {
             if (graph) (void)hipGraphDestroy(graph);
             return rc;
