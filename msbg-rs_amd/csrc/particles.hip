@@ -18,6 +18,18 @@ __global__ void morton_keys_kernel(const float *__restrict__ pos, int64_t n, uin
     }
 }
 
+// Keys and indices of an order to visit the particles in: the Morton keys of
+// the cells, held to the domain, so that they take no more bits than it has.
+__global__ void morton_clamped_kernel(const float *__restrict__ pos, int64_t n, uint32_t mx, uint32_t my, uint32_t mz,
+                                      uint32_t *__restrict__ keys, uint32_t *__restrict__ idx) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        const uint32_t x = min(trunc_index(pos[3 * i]), mx), y = min(trunc_index(pos[3 * i + 1]), my),
+                       z = min(trunc_index(pos[3 * i + 2]), mz);
+        keys[i] = spread10(x) | (spread10(y) << 1) | (spread10(z) << 2);
+        idx[i] = (uint32_t)i;
+    }
+}
+
 // morton_keys_kernel's keys and indices, and each particle's two 16-byte
 // records (x, y, z, m) and (u, v, w, 0) in caller order, so that the sorted
 // payload is gathered as one 32-byte record per particle instead of three
@@ -208,6 +220,20 @@ int morton_sort_async(const float *d_pos, int64_t n, uint32_t *d_keys, uint32_t 
     return radix_sort_pairs(d_keys, d_perm, n, 30);
 }
 
+int bits_for(int64_t v) {
+    int b = 1;
+    while (b < 32 && ((int64_t)1 << b) <= v) ++b;
+    return b;
+}
+
+int morton_order_async(const float *d_pos, int64_t n, int sx, int sy, int sz, uint32_t *d_keys, uint32_t *d_perm) {
+    if (n == 0) return MSBG_OK;
+    hipLaunchKernelGGL(morton_clamped_kernel, dim3(grid_for(n)), dim3(256), 0, stream(), d_pos, n, (uint32_t)sx - 1,
+                       (uint32_t)sy - 1, (uint32_t)sz - 1, d_keys, d_perm);
+    MSBG_HIP(hipGetLastError());
+    return radix_sort_pairs(d_keys, d_perm, n, 3 * std::min(10, bits_for(std::max(sx, std::max(sy, sz)) - 1)));
+}
+
 int morton_sort_pack_async(const float *d_pos, const float *d_vel, const float *d_mass, int64_t n, uint32_t *d_keys,
                            uint32_t *d_perm, float4 *d_rec) {
     if (n == 0) return MSBG_OK;
@@ -215,12 +241,6 @@ int morton_sort_pack_async(const float *d_pos, const float *d_vel, const float *
                        d_keys, d_perm, d_rec);
     MSBG_HIP(hipGetLastError());
     return radix_sort_pairs(d_keys, d_perm, n, 30);
-}
-
-int bits_for(int64_t v) {
-    int b = 1;
-    while (b < 32 && ((int64_t)1 << b) <= v) ++b;
-    return b;
 }
 
 }  // namespace msbg
@@ -240,7 +260,9 @@ int msbg_morton_keys(const float *d_pos, int64_t n, uint32_t *d_keys) {
 
 int msbg_radix_sort_pairs(uint32_t *d_keys, uint32_t *d_vals, int64_t n, int key_bits) {
     MSBG_CHECK(n == 0 || (d_keys && d_vals), MSBG_EINVAL, "radix sort: null argument");
-    int rc = radix_sort_pairs(d_keys, d_vals, n, key_bits);
+    // whole bytes, as the sort's digits are documented
+    MSBG_CHECK(key_bits >= 1 && key_bits <= 32, MSBG_EINVAL, "radix sort: key_bits must be 1..32");
+    int rc = radix_sort_pairs(d_keys, d_vals, n, (key_bits + 7) / 8 * 8);
     if (rc) return rc;
     MSBG_HIP(hipStreamSynchronize(stream()));
     return MSBG_OK;

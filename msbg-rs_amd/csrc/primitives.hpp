@@ -19,11 +19,16 @@ int scan_exclusive_u32(const uint32_t *in, uint32_t *out, int64_t n, uint32_t *t
 int scan_exclusive_u32_with(const uint32_t *in, uint32_t *out, int64_t n, uint32_t *sums, uint32_t *total_host);
 int64_t scan_sums_words(int64_t n);
 
-// Stable sort of (keys, vals) by the low `key_bits` bits of keys, in place.
+// Stable sort of (keys, vals) in place, keys below 2^key_bits.
 int radix_sort_pairs(uint32_t *keys, uint32_t *vals, int64_t n, int key_bits);
 
 // msbg_morton_sort without the final synchronization (stream-ordered).
 int morton_sort_async(const float *d_pos, int64_t n, uint32_t *d_keys, uint32_t *d_perm);
+// Some order along a Morton curve over the domain (keys and particle indices):
+// for visiting particles, not a sort by msbg_morton_keys.
+int morton_order_async(const float *d_pos, int64_t n, int sx, int sy, int sz, uint32_t *d_keys, uint32_t *d_perm);
+// The bits of v, at least 1.
+int bits_for(int64_t v);
 // morton_sort_async, also writing each particle's records (x, y, z, m), (u, v, w, 0)
 // to d_rec[2 i], d_rec[2 i + 1] in caller order (d_mass null: m = 1).
 int morton_sort_pack_async(const float *d_pos, const float *d_vel, const float *d_mass, int64_t n, uint32_t *d_keys,

@@ -610,21 +610,88 @@ __global__ void gather_records_kernel(const float4 *__restrict__ rec, const uint
     }
 }
 
-// Voxel ranges of the sorted particles: vbeg/vend indexed by slot*4096+vid.
-__global__ void voxel_ranges_kernel(const uint32_t *__restrict__ keys, const float4 *__restrict__ pm, int64_t n,
-                                    GridView g, uint32_t *__restrict__ vbeg, uint32_t *__restrict__ vend) {
+// Sort keys of the B-spline P2G, block id and voxel id (x fastest), and the
+// particles' records in caller order: x-adjacent voxels of a block are one run
+// of the sorted particles, and a voxel's particles keep their input order.  A
+// particle outside the domain adds nothing: it becomes one of no mass and no
+// velocity in a voxel of its own index's choosing.
+__global__ void block_keys_pack_kernel(const float *__restrict__ pos, const float *__restrict__ vel,
+                                       const float *__restrict__ mass, int64_t n, int sx, int sy, int sz, int nx,
+                                       int ny, uint32_t n_keys, uint32_t *__restrict__ keys,
+                                       uint32_t *__restrict__ idx, float4 *__restrict__ rec) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const bool head = i == 0 || keys[i - 1] != keys[i];
-        const bool tail = i == n - 1 || keys[i + 1] != keys[i];
-        if (!head && !tail) continue;
-        const float4 p = pm[i];
-        const uint32_t x = trunc_index(p.x), y = trunc_index(p.y), z = trunc_index(p.z);
-        if (x >= (uint32_t)g.sx || y >= (uint32_t)g.sy || z >= (uint32_t)g.sz) continue;
-        const int slot = g.b2s[(x >> 4) + (int64_t)(y >> 4) * g.nx + (int64_t)(z >> 4) * g.nx * g.ny];
-        if (slot < 2) continue;
-        const int64_t c = (int64_t)slot * 4096 + ((x & 15) | ((y & 15) << 4) | ((z & 15) << 8));
-        if (head) vbeg[c] = (uint32_t)i;
-        if (tail) vend[c] = (uint32_t)(i + 1);
+        const float px = pos[3 * i], py = pos[3 * i + 1], pz = pos[3 * i + 2];
+        const uint32_t x = trunc_index(px), y = trunc_index(py), z = trunc_index(pz);
+        float4 a = make_float4(px, py, pz, mass ? mass[i] : 1.0f);
+        float4 b = make_float4(vel[3 * i], vel[3 * i + 1], vel[3 * i + 2], 0.0f);
+        uint32_t key = ((x >> 4) + (uint32_t)nx * ((y >> 4) + (uint32_t)ny * (z >> 4))) << 12 | (x & 15) | (y & 15) << 4 |
+                       (z & 15) << 8;
+        if (x >= (uint32_t)sx || y >= (uint32_t)sy || z >= (uint32_t)sz) {
+            key = (uint32_t)i * 2654435761u % n_keys;
+            a = b = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        }
+        keys[i] = key;
+        idx[i] = (uint32_t)i;
+        rec[2 * i] = a;
+        rec[2 * i + 1] = b;
+    }
+}
+
+// The sorted particles [beg, end) of every voxel of the active blocks, indexed
+// by slot * 4096 + vid; an empty voxel's range is empty where its particles
+// would be, so neighbouring voxels' ranges join.  A work-group per block: its
+// run by search, a count per voxel in LDS, their scan.
+__global__ __launch_bounds__(256) void voxel_ranges_kernel(const uint32_t *__restrict__ keys, uint32_t n,
+                                                           const int32_t *__restrict__ active, GridView g,
+                                                           uint2 *__restrict__ range) {
+    __shared__ uint32_t s_cnt[4096];
+    __shared__ uint32_t s_run[2], s_sum[4];
+    const uint32_t bid = (uint32_t)active[blockIdx.x];
+    const int slot = g.b2s[bid], t = threadIdx.x;
+    if (slot < 2) return;
+    if (t < 128) {
+        // the first particle whose key is not below the block's (wave 0) / the
+        // next block's (wave 1): a wave probes 64 places at a time
+        const uint32_t key = (bid + (t >> 6)) << 12, lane = t & 63;
+        uint32_t lo = 0, hi = n;  // it lies in [lo, hi]
+        while (lo < hi) {
+            const uint32_t step = (hi - lo + 63) / 64, at = lo + lane * step;
+            const uint32_t below = (uint32_t)__popcll(__ballot(at < hi && keys[at] < key));  // probes 0 .. below - 1
+            if (below == 0) {
+                hi = lo;
+            } else {
+                hi = min(hi, lo + below * step);
+                lo = lo + (below - 1) * step + 1;
+            }
+        }
+        if (lane == 0) s_run[t >> 6] = lo;
+    }
+    for (int v = t; v < 4096; v += 256) s_cnt[v] = 0;
+    __syncthreads();
+    const uint32_t b0 = s_run[0], b1 = s_run[1];
+    for (uint32_t i = b0 + t; i < b1; i += 256) atomicAdd(&s_cnt[keys[i] & 4095u], 1u);
+    __syncthreads();
+    uint32_t c[16], sum = 0;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        c[v] = s_cnt[16 * t + v];
+        sum += c[v];
+    }
+    uint32_t x = sum;  // inclusive scan inside each wave, then wave sums
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o);
+        if ((t & 63) >= o) x += y;
+    }
+    if ((t & 63) == 63) s_sum[t >> 6] = x;
+    __syncthreads();
+    uint32_t at = b0 + x - sum;
+    for (int w = 0; w < t >> 6; ++w) at += s_sum[w];
+    uint4 *out = reinterpret_cast<uint4 *>(range + ((int64_t)slot << 12) + 16 * t);
+#pragma unroll
+    for (int v = 0; v < 16; v += 2) {
+        const uint32_t m = at + c[v], e = m + c[v + 1];
+        out[v / 2] = make_uint4(at, m, m, e);
+        at = e;
     }
 }
 
@@ -647,18 +714,26 @@ __device__ __forceinline__ void acc_add(Acc4 &a, float wxy, float pz, int cz, fl
 // 18 voxel planes bz*16-1 .. bz*16+16 once: plane v feeds cells v+1 (as their
 // dz = -1 plane), v (dz = 0) and v-1 (dz = +1), so each particle is read once
 // per column and every cell still receives its planes in increasing z.
-template <int ORDER>
+//
+// SPAN: cells of the column that a work-group takes.  The whole column (16) has
+// the least to read (18 planes for 16 cells); on few blocks, where a column's
+// chain of dependent reads is all the time, spans of 4 (6 planes).
+// Bound by its arithmetic and by lanes that wait for the fullest of their wave
+// (16.8 M particles in 9,000 blocks, quadratic: 1,240 us with 9 voxels a plane
+// to step through, most of them empty, 1,025 with joined rows; 1 M in 350
+// blocks, linear: 375 and 120).
+template <int ORDER, int SPAN>
 __global__ __launch_bounds__(256) void p2g_bspline_kernel(GridView mg, GridView v0, GridView v1, GridView v2,
                                                           const int32_t *__restrict__ active,
-                                                          const uint32_t *__restrict__ vbeg,
-                                                          const uint32_t *__restrict__ vend,
+                                                          const uint2 *__restrict__ range,
                                                           const float4 *__restrict__ pm,
                                                           const float4 *__restrict__ pu) {
     __shared__ int s_nb[27];
     // voxel ranges of the block's 18 x 18 plane window (the block's columns
     // and a 1-voxel ring), double-buffered: plane v + 1 loads during plane v
     __shared__ uint2 s_pl[2][18 * 18];
-    const int64_t bid = active[blockIdx.x];
+    const int64_t bid = active[blockIdx.x / (16 / SPAN)];
+    const int lz0 = (int)(blockIdx.x % (16 / SPAN)) * SPAN;  // first cell of the span
     const int bx = (int)(bid % mg.nx), by = (int)((bid / mg.nx) % mg.ny), bz = (int)(bid / ((int64_t)mg.nx * mg.ny));
     if (threadIdx.x < 27) {
         const int t = threadIdx.x;
@@ -672,10 +747,10 @@ __global__ __launch_bounds__(256) void p2g_bspline_kernel(GridView mg, GridView 
     const int s0 = v0.b2s[bid], s1 = v1.b2s[bid], s2 = v2.b2s[bid];
     if (ms < 2) return;
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
-    const int cx = bx * 16 + lx, cy = by * 16 + ly, cz0 = bz * 16;
+    const int cx = bx * 16 + lx, cy = by * 16 + ly, cz0 = bz * 16 + lz0;
     Acc4 lo = {0, 0, 0, 0}, mid = {0, 0, 0, 0}, hi = {0, 0, 0, 0};  // cells lv-1, lv, lv+1
     auto store = [&](int lz, const Acc4 &a) {
-        const int vid = lx | (ly << 4) | (lz << 8);
+        const int vid = lx | (ly << 4) | ((lz0 + lz) << 8);
         mg.slab[(int64_t)ms * 4096 + vid] = a.m;
         const bool pos_m = a.m > 0.0f;
         v0.slab[(int64_t)s0 * 4096 + vid] = pos_m ? a.u0 / a.m : 0.0f;
@@ -691,11 +766,12 @@ __global__ __launch_bounds__(256) void p2g_bspline_kernel(GridView mg, GridView 
             r[h] = make_uint2(0u, 0u);
             if (idx >= 18 * 18 || vz < 0 || vz >= mg.sz) continue;
             const int vy = by * 16 - 1 + idx / 18, vx = bx * 16 - 1 + idx % 18;
-            if (vy < 0 || vy >= mg.sy || vx < 0 || vx >= mg.sx) continue;
+            // (not past the domain's last block; a voxel past its last cell has an empty range in its place)
+            if (vy < 0 || (vy >> 4) >= mg.ny || vx < 0 || (vx >> 4) >= mg.nx) continue;
             const int slot = s_nb[((vx >> 4) - bx + 1) + 3 * ((vy >> 4) - by + 1) + 9 * ((vz >> 4) - bz + 1)];
             if (slot < 2) continue;
             const int64_t c = (int64_t)slot * 4096 + ((vx & 15) | ((vy & 15) << 4) | ((vz & 15) << 8));
-            r[h] = make_uint2(vbeg[c], vend[c]);
+            r[h] = range[c];
         }
     };
     auto put_plane = [&](int buf, const uint2 *r) {
@@ -706,50 +782,58 @@ __global__ __launch_bounds__(256) void p2g_bspline_kernel(GridView mg, GridView 
     plane_ranges(cz0 - 1, nxt);
     put_plane(0, nxt);
     __syncthreads();
-    for (int lv = -1; lv <= 16; ++lv) {
+    for (int lv = -1; lv <= SPAN; ++lv) {
         const int vz = cz0 + lv, cur = (lv + 1) & 1;
-        if (lv < 16) plane_ranges(vz + 1, nxt);  // in flight while this plane's particles are added
+        if (lv < SPAN) plane_ranges(vz + 1, nxt);  // in flight while this plane's particles are added
         if (vz >= 0 && vz < mg.sz) {
-            // This lane's 9 voxel ranges, (dy, dx) in order, are window
-            // voxels (ly + dy + 1, lx + dx + 1).  One pass over their
-            // concatenation: a wave steps as often as its fullest lane has
-            // particles, not once per voxel per the fullest lane of that
-            // voxel.  Per cell, the particles still arrive voxel by voxel in
-            // (dy, dx) order, sorted within.
+            // This lane's 9 voxels are window voxels (ly + dy + 1, lx + dx + 1).
+            // The three of a row are one run of the sorted particles, or two
+            // where a block ends between them: 6 runs, the second one of a row
+            // empty but for the first and the last lane of a row.  One pass
+            // over their concatenation: a wave steps as often as its fullest
+            // lane has particles.  Per cell, the particles still arrive voxel
+            // by voxel in (dy, dx) order, sorted within.
             const uint2 *pl = s_pl[cur] + ly * 18 + lx;
-            auto rng = [&](int t) { return pl[(t / 3) * 18 + t % 3]; };
+            auto rng = [&](int t) {
+                const uint2 *row = pl + (t >> 1) * 18;
+                const uint2 a = row[0], m = row[1], b = row[2];
+                // lane 0: {-1}, {0, 1}; lane 15: {14, 15}, {16}; the others {-1, 0, 1}
+                if (t & 1) return lx == 0 ? make_uint2(m.x, b.y) : (lx == 15 ? b : make_uint2(0u, 0u));
+                return make_uint2(a.x, lx == 0 ? a.y : (lx == 15 ? m.y : b.y));
+            };
+            const int step = lx == 0 || lx == 15 ? 1 : 2;
             int t = 0;
             uint2 rt = rng(0);
             uint32_t j = rt.x, e = rt.y;
-            while (j >= e && ++t < 9) {
+            while (j >= e && (t += step) < 6) {
                 rt = rng(t);
                 j = rt.x;
                 e = rt.y;
             }
             float4 pn = make_float4(0.f, 0.f, 0.f, 0.f), un = pn;
-            if (t < 9) {
+            if (t < 6) {
                 pn = pm[j];
                 un = pu[j];
             }
-            while (t < 9) {
+            while (t < 6) {
                 const float4 p = pn, u = un;
                 ++j;
-                while (j >= e && ++t < 9) {
+                while (j >= e && (t += step) < 6) {
                     rt = rng(t);
                     j = rt.x;
                     e = rt.y;
                 }
-                if (t < 9) {  // the next particle's records are in flight while this one is added
+                if (t < 6) {  // the next particle's records are in flight while this one is added
                     pn = pm[j];
                     un = pu[j];
                 }
                 const float wxy = bspline_w<ORDER>(p.x, cx) * bspline_w<ORDER>(p.y, cy);
                 if (lv >= 1) acc_add<ORDER>(lo, wxy, p.z, cz0 + lv - 1, p.w, u);
-                if (lv >= 0 && lv <= 15) acc_add<ORDER>(mid, wxy, p.z, cz0 + lv, p.w, u);
-                if (lv <= 14) acc_add<ORDER>(hi, wxy, p.z, cz0 + lv + 1, p.w, u);
+                if (lv >= 0 && lv <= SPAN - 1) acc_add<ORDER>(mid, wxy, p.z, cz0 + lv, p.w, u);
+                if (lv <= SPAN - 2) acc_add<ORDER>(hi, wxy, p.z, cz0 + lv + 1, p.w, u);
             }
         }
-        if (lv < 16) put_plane(cur ^ 1, nxt);  // buffer cur ^ 1 was last read before the previous barrier
+        if (lv < SPAN) put_plane(cur ^ 1, nxt);  // buffer cur ^ 1 was last read before the previous barrier
         __syncthreads();
         if (lv >= 1) store(lv - 1, lo);  // cell lv-1 has its planes lv-2, lv-1, lv
         lo = mid;
@@ -1201,35 +1285,46 @@ int msbg_p2g_bspline(int order, msbg_grid *mass, msbg_grid *const *vel, const fl
     if (rc) return rc;
     *n_active = (int64_t)act.size();
     if (n == 0 || act.empty()) return MSBG_OK;
-    // Morton sort (stable) and the sorted payload
+    // sort by block and voxel (stable) and the sorted payload
     uint32_t *keys = (uint32_t *)workspace(4, sizeof(uint32_t) * 2 * n, &rc);
     if (rc) return rc;
     uint32_t *perm = keys + n;
     float4 *rec = (float4 *)workspace(22, sizeof(float4) * 2 * n, &rc);
     if (rc) return rc;
-    rc = morton_sort_pack_async(d_pos, d_vel, d_mass, n, keys, perm, rec);
+    const uint32_t n_keys = (uint32_t)mass->n_blocks << 12;  // at most 2^30
+    hipLaunchKernelGGL(block_keys_pack_kernel, dim3(grid_for(n, 256)), dim3(256), 0, stream(), d_pos, d_vel, d_mass, n,
+                       mass->sx, mass->sy, mass->sz, (int)mass->nx, (int)mass->ny, n_keys, keys, perm, rec);
+    MSBG_HIP(hipGetLastError());
+    rc = radix_sort_pairs(keys, perm, n, bits_for((int64_t)n_keys - 1));
     if (rc) return rc;
     float4 *pay = (float4 *)workspace(7, sizeof(float4) * 2 * n, &rc);
     if (rc) return rc;
     float4 *pm = pay, *pu = pay + n;
     hipLaunchKernelGGL(gather_records_kernel, dim3(grid_for(n, 256)), dim3(256), 0, stream(), rec, perm, n, pm, pu);
-    MSBG_HIP(hipGetLastError());
-    // per-voxel ranges of the sorted particles, indexed like the mass slab
-    const int64_t ncell = mass->n_slots * 4096;
-    uint32_t *vr = (uint32_t *)workspace(8, sizeof(uint32_t) * 2 * ncell, &rc);
+    // per-voxel ranges of the sorted particles, indexed like the mass slab; the
+    // dummy slots' are never looked at
+    uint2 *range = (uint2 *)workspace(8, sizeof(uint2) * mass->n_slots * 4096, &rc);
     if (rc) return rc;
-    uint32_t *vbeg = vr, *vend = vr + ncell;
-    MSBG_HIP(hipMemsetAsync(vr, 0, sizeof(uint32_t) * 2 * ncell, stream()));
-    hipLaunchKernelGGL(voxel_ranges_kernel, dim3(grid_for(n, 256)), dim3(256), 0, stream(), keys, pm, n, mass->view(),
-                       vbeg, vend);
+    hipLaunchKernelGGL(voxel_ranges_kernel, dim3((unsigned)act.size()), dim3(256), 0, stream(), keys, (uint32_t)n, d_act,
+                       mass->view(), range);
     MSBG_HIP(hipGetLastError());
-    const dim3 grid((unsigned)act.size()), block(256);
-    if (order == 1)
-        hipLaunchKernelGGL(p2g_bspline_kernel<1>, grid, block, 0, stream(), mass->view(), vel[0]->view(), vel[1]->view(),
-                           vel[2]->view(), d_act, vbeg, vend, pm, pu);
+    const unsigned na = (unsigned)act.size();
+    const auto spread = [&](auto kernel, int span) {
+        kernel<<<na * (16 / span), 256, 0, stream()>>>(mass->view(), vel[0]->view(), vel[1]->view(), vel[2]->view(),
+                                                       d_act, range, pm, pu);
+    };
+    // Up to 8 columns of a work-group a CU fit at once, and fewer leave it idle
+    // (1 M particles, 350 blocks: 375 us whole, 141 in spans of 4, 164 of 2; 16.8 M,
+    // 9,000 blocks: 1,265 whole, 1,334 in spans of 4; all before the rows joined).
+    const bool whole = na >= 2048;
+    if (order == 1 && whole)
+        spread(p2g_bspline_kernel<1, 16>, 16);
+    else if (order == 1)
+        spread(p2g_bspline_kernel<1, 4>, 4);
+    else if (whole)
+        spread(p2g_bspline_kernel<2, 16>, 16);
     else
-        hipLaunchKernelGGL(p2g_bspline_kernel<2>, grid, block, 0, stream(), mass->view(), vel[0]->view(), vel[1]->view(),
-                           vel[2]->view(), d_act, vbeg, vend, pm, pu);
+        spread(p2g_bspline_kernel<2, 4>, 4);
     MSBG_HIP(hipGetLastError());
     MSBG_HIP(hipStreamSynchronize(stream()));
     return MSBG_OK;
@@ -1246,7 +1341,7 @@ int msbg_g2p_bspline(int order, msbg_grid *const *vel, const float *d_pos, int64
     uint32_t *keys = (uint32_t *)workspace(9, sizeof(uint32_t) * 2 * n, &rc);
     if (rc) return rc;
     uint32_t *visit = keys + n;
-    rc = morton_sort_async(d_pos, n, keys, visit);
+    rc = morton_order_async(d_pos, n, vel[0]->sx, vel[0]->sy, vel[0]->sz, keys, visit);
     if (rc) return rc;
     // one lane per particle (n < 2^31, so the chunk count fits the grid)
     const dim3 chunks((unsigned)((n + kG2pThreads - 1) / kG2pThreads)), lanes(kG2pThreads);

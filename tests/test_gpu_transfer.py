@@ -460,3 +460,32 @@ def test_g2p_flip_matches_sample_twice_and_blend(pkg, orc, hip, interp, bc, n, s
         want = np.zeros_like(uo)
         orc.orc_g2p_blend(uo, su, st, n, alpha, want)
         assert_bitexact(got, want, "g2p flip")
+
+
+@pytest.mark.parametrize("order", [1, 2])
+@pytest.mark.parametrize("s,spread", [((16, 16, 16), 1.0), ((40, 33, 21), 1.0), ((208, 208, 208), 0.9)])
+def test_p2g_bspline_rows_and_strays(pkg, orc, hip, order, s, spread):
+    """The oracle's bits where a plane's rows of voxels join (inside a block, at
+    its ends, in ragged last blocks, with crowded voxels), in spans (few blocks)
+    and whole columns (2,197 blocks), with particles outside the domain, which
+    add nothing, in between."""
+    n = 60000 if s[0] < 200 else 12000
+    rng = np.random.default_rng(sum(s) + order)
+    hi = np.array(s, np.float64)
+    pos = rng.uniform(0.0, 1.0, (n, 3)) * hi * spread + 0.5 * (1.0 - spread) * hi
+    if s[0] >= 200:  # one particle in every block, so that all of them are active
+        b = np.arange(13 ** 3)
+        pos[: b.size] = 16.0 * np.stack([b % 13, (b // 13) % 13, b // 169], 1) + 8.0
+    pos[5000:5200] = pos[7]
+    stray = rng.integers(0, n, 300)
+    pos[stray, rng.integers(0, 3, 300)] = rng.choice([hi.max() + 0.25, 1023.5, 5000.0, 1e9], 300)
+    pos = np.minimum(pos, np.where(pos < hi, np.nextafter(hi.astype(np.float32), np.float32(0)), np.inf)).astype(np.float32)
+    vel = rng.normal(size=(n, 3)).astype(np.float32)
+    mass = rng.uniform(0.5, 2.0, n).astype(np.float32)
+    inside = np.all(pos < np.float32(hi), axis=1)
+    active, b2s, slabs = oracle_p2g_bspline(orc, order, s, pos[inside], vel[inside], mass[inside])
+    tg = T.TransferGrid(*s, capacity_blocks=14 ** 3 + 8, lib=hip)
+    assert tg.p2g(order, pos, vel, mass) >= active.size
+    assert_bitexact(tg.mass.to_host().to_dense(), dense_from_slabs(b2s, slabs[0], s), "mass")
+    for a in range(3):
+        assert_bitexact(tg.velocity[a].to_host().to_dense(), dense_from_slabs(b2s, slabs[1 + a], s), "vel %d" % a)
