@@ -21,6 +21,7 @@
 // cells.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "poisson.hpp"
@@ -98,6 +99,149 @@ struct Conv2Args {
     int slabs;             // ceil(sout / kZS)
 };
 
+// Two floats as bf16, rounded to nearest even (v_cvt_pk_bf16_f32: to_bf16's
+// bits in one instruction instead of a dozen; NaNs stay NaNs).
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{lo, hi}), b2));
+}
+
+// Stages planes z0 + off .. z0 + off + zn + 1, rows and columns off .. off +
+// SP - 1 of a tile (zero outside it).
+template <int CIN, int SP>
+__device__ __forceinline__ void stage_planes(const Conv2Args &a, u4v *lds, int64_t tin, int z0, int zn) {
+    constexpr int VPC = CIN == 16 ? 2 : 1;  // staged words per cell: 2 x 16 B, or one 4-byte pair
+    using W = std::conditional_t<CIN == 16, u4v, uint32_t>;
+    const int sin = a.sin, off = a.off;
+    const int nst = (zn + 2) * SP * SP * VPC;
+    constexpr int kPer = ((kZS + 2) * SP * SP * VPC + kConvThreads - 1) / kConvThreads;
+    const W *in = reinterpret_cast<const W *>(a.in) + tin * VPC;
+    W w[kPer];
+    // all of a lane's loads before its first LDS write: one round trip, not kPer
+    // (2-channel layer, 512 tiles: 34 us, 41 with a round trip each and the
+    // rounding of the results in integer instructions)
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int i = threadIdx.x + j * kConvThreads;
+        const unsigned c = (unsigned)i / VPC, v = (unsigned)i - c * VPC;
+        const int p = (int)(c / (SP * SP)), r = (int)(c - p * (SP * SP)), y = r / SP, x = r - y * SP;
+        const int iz = z0 + off + p, iy = off + y, ix = off + x;
+        const bool inside =
+            i < nst && (unsigned)iz < (unsigned)sin && (unsigned)iy < (unsigned)sin && (unsigned)ix < (unsigned)sin;
+        const int64_t g = (((int64_t)iz * sin + iy) * sin + ix) * VPC + v;
+        if constexpr (CIN == 16) {
+            // no branch (a cell outside reads the tile's first): branches around
+            // 16-byte loads made the compiler spill hundreds of registers
+            w[j] = in[inside ? g : 0];
+            if (!inside) w[j] = W{};
+        } else {
+            w[j] = 0u;
+            if (inside) w[j] = in[g];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int i = threadIdx.x + j * kConvThreads;
+        if (i < nst) reinterpret_cast<W *>(lds)[i] = w[j];
+    }
+}
+
+// Bias, ReLU, mask and store of one cell's channels 4 kb .. 4 kb + 3 at output cell o.
+template <bool OUTF>
+__device__ __forceinline__ void put_cell(const Conv2Args &a, const f4 &acc, const float *bias, int64_t o, int kb) {
+    float v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        v[j] = acc[j] + bias[j];
+        if (a.relu) v[j] = v[j] > 0.0f ? v[j] : 0.0f;
+    }
+    if (a.mask) {
+        const uint2 mk = *reinterpret_cast<const uint2 *>(a.mask + o * 16 + 4 * kb);
+        const uint16_t mh[4] = {(uint16_t)(mk.x & 0xffffu), (uint16_t)(mk.x >> 16), (uint16_t)(mk.y & 0xffffu),
+                                (uint16_t)(mk.y >> 16)};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (!(from_bf16(mh[j]) > 0.0f)) v[j] = 0.0f;
+    }
+    if (OUTF) {
+        if (kb == 0) ((float *)a.out)[o] = v[0];
+    } else {
+        const uint2 w = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+        *reinterpret_cast<uint2 *>((uint16_t *)a.out + o * 16 + 4 * kb) = w;
+    }
+}
+
+// The 16-channel layers of output edge 16: a wave takes 8 rows of 16 cells of
+// one output plane, the row y + 0 .. 2 of an input plane pair serves three of
+// them.  Per step the wave reads one input row at its three x offsets (planes z
+// and z + 1 side by side along K) for the outputs y, y - 1 and y - 2, then the
+// five operands of plane z + 2 that finish output y - 2: 70 LDS reads for 112
+// matrix instructions, where a read for each took twice an instruction's time.
+// 512 tiles: 42 us (the last layer 32), 47 (38) with a read for each; the rest
+// is the staging's round trip and the bf16 stores, at two work-groups a CU.  Every output adds its tap pairs in the order of
+// conv2_kernel, so the bits are the same.
+template <bool OUTF>
+__global__ __launch_bounds__(kConvThreads, 4) void conv16_kernel(Conv2Args a) {
+    extern __shared__ u4v lds[];
+    constexpr int SP = 18, PL = SP * SP, ROWS = 8;
+    static_assert(kZS * 16 / ROWS == kConvThreads / 64, "a wave per 8 rows");
+    const int tile = blockIdx.x / a.slabs, z0 = (blockIdx.x - tile * a.slabs) * kZS;
+    stage_planes<16, SP>(a, lds, (int64_t)(a.idx ? a.idx[tile] : tile) * a.sin * a.sin * a.sin, z0, kZS);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    u4v wv[kTP];
+#pragma unroll
+    for (int tp = 0; tp < kTP; ++tp) wv[tp] = a.wb[tp * 64 + lane];
+    const int m = lane & 15, kb = lane >> 4, h = kb >> 1;
+    float bias[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) bias[j] = a.bias ? a.bias[4 * kb + j] : 0.0f;
+    const int zl = wave >> 1, y0 = (wave & 1) * ROWS;
+    const u4v *cell = lds + 2 * (zl * PL + y0 * SP + m) + (kb & 1);  // row y0, x = m of plane zl
+    const u4v *pair = cell + 2 * h * PL;                              // planes zl, zl + 1
+    const u4v *high = cell + 4 * PL;                                  // plane zl + 2
+    __syncthreads();
+    auto mma = [&](f4 &c, int tp, const u4v &v) {
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, wv[tp]), __builtin_bit_cast(bf8, v), c, 0, 0,
+                                                    0);
+    };
+    f4 acc[3];  // output rows r, r - 1, r - 2 at r, r - 1, r - 2 modulo 3
+    const int64_t o = ((int64_t)tile * 16 + z0 + zl) * 256 + y0 * 16 + m;
+    u4v v[3];
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx) v[dx] = pair[2 * dx];
+#pragma unroll
+    for (int r = 0; r < ROWS + 2; ++r) {
+        const int y = r - 2;  // the output that this step finishes
+        u4v next[3], top[5];
+        if (r + 1 < ROWS + 2)
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx) next[dx] = pair[2 * ((r + 1) * SP + dx)];
+        if (y >= 0) {
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx) top[dx] = high[2 * ((y + h) * SP + dx)];
+            top[3] = high[2 * ((y + 2) * SP + h)];
+            top[4] = high[2 * ((y + 2) * SP + 2)];
+        }
+        if (r < ROWS) acc[r % 3] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+            for (int dy = 0; dy < 3; ++dy)  // three outputs in turn; each one's dy, dx ascend
+                if (r - dy >= 0 && r - dy < ROWS) mma(acc[(r - dy) % 3], 3 * dy + dx, v[dx]);
+        if (y >= 0) {
+            f4 &c = acc[y % 3];
+#pragma unroll
+            for (int i = 0; i < 5; ++i) mma(c, 9 + i, top[i]);
+            put_cell<OUTF>(a, c, bias, o + 16 * y, kb);
+        }
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) v[dx] = next[dx];
+        // the next step's reads stay in the next step: all of them at once take 224 registers
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 // Output edge sout = SP - 2; input cell (off + x, off + y, off + z) of the
 // tile's sin^3 input sits at staged (x, y, z - z0).
 template <int CIN, int SP, bool OUTF>
@@ -105,31 +249,11 @@ __global__ __launch_bounds__(kConvThreads) void conv2_kernel(Conv2Args a) {
     extern __shared__ u4v lds[];
     constexpr int SOUT = SP - 2, S2 = SOUT * SOUT;
     constexpr int NTP = CIN == 16 ? kTP : 2;
-    constexpr int VPC = CIN == 16 ? 2 : 1;  // staged words per cell: 2 x 16 B, or one 4-byte pair
     const int tile = blockIdx.x / a.slabs, slab = blockIdx.x - tile * a.slabs;
     const int z0 = slab * kZS, zn = min(kZS, SOUT - z0);
-    const int sin = a.sin, off = a.off;
+    const int sin = a.sin;
     const int64_t tin = (int64_t)(a.idx ? a.idx[tile] : tile) * sin * sin * sin;
-    {
-        // stage planes z0 + off .. z0 + off + zn + 1, rows and columns off .. off + SP - 1
-        const int nst = (zn + 2) * SP * SP * VPC;
-        for (int i = threadIdx.x; i < nst; i += kConvThreads) {
-            const unsigned c = (unsigned)i / VPC, v = (unsigned)i - c * VPC;
-            const int p = (int)(c / (SP * SP)), r = (int)(c - p * (SP * SP)), y = r / SP, x = r - y * SP;
-            const int iz = z0 + off + p, iy = off + y, ix = off + x;
-            const bool in = (unsigned)iz < (unsigned)sin && (unsigned)iy < (unsigned)sin && (unsigned)ix < (unsigned)sin;
-            const int64_t g = ((int64_t)iz * sin + iy) * sin + ix;
-            if constexpr (CIN == 16) {
-                u4v w = {0u, 0u, 0u, 0u};
-                if (in) w = reinterpret_cast<const u4v *>(a.in)[(tin + g) * 2 + v];
-                lds[i] = w;
-            } else {
-                uint32_t w = 0u;
-                if (in) w = reinterpret_cast<const uint32_t *>(a.in)[tin + g];
-                reinterpret_cast<uint32_t *>(lds)[i] = w;
-            }
-        }
-    }
+    stage_planes<CIN, SP>(a, lds, tin, z0, zn);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     u4v wv[NTP];
 #pragma unroll
@@ -195,27 +319,7 @@ __global__ __launch_bounds__(kConvThreads) void conv2_kernel(Conv2Args a) {
             const int cl = grp * 16 + m;  // this lane's cell; channels 4 kb .. 4 kb + 3
             if (grp >= groups || cl >= ncell) continue;
             const int64_t o = ((int64_t)tile * SOUT + z0) * S2 + cl;
-            float v[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                v[j] = acc[g][j] + bias[j];
-                if (a.relu) v[j] = v[j] > 0.0f ? v[j] : 0.0f;
-            }
-            if (a.mask) {
-                const uint2 mk = *reinterpret_cast<const uint2 *>(a.mask + o * 16 + 4 * kb);
-                const uint16_t mh[4] = {(uint16_t)(mk.x & 0xffffu), (uint16_t)(mk.x >> 16), (uint16_t)(mk.y & 0xffffu),
-                                        (uint16_t)(mk.y >> 16)};
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (!(from_bf16(mh[j]) > 0.0f)) v[j] = 0.0f;
-            }
-            if (OUTF) {
-                if (kb == 0) ((float *)a.out)[o] = v[0];
-            } else {
-                const uint2 w = make_uint2((uint32_t)to_bf16(v[0]) | (uint32_t)to_bf16(v[1]) << 16,
-                                           (uint32_t)to_bf16(v[2]) | (uint32_t)to_bf16(v[3]) << 16);
-                *reinterpret_cast<uint2 *>((uint16_t *)a.out + o * 16 + 4 * kb) = w;
-            }
+            put_cell<OUTF>(a, acc[g], bias, o, kb);
         }
     }
 }
@@ -760,16 +864,20 @@ void conv(hipStream_t s, const uint16_t *in, const int32_t *idx, int sin, int of
     a.slabs = (SOUT + kZS - 1) / kZS;
     constexpr int SP = SOUT + 2;
     const size_t lds = (size_t)(kZS + 2) * SP * SP * CIN * 2;
-    conv2_kernel<CIN, SP, OUTF><<<n * a.slabs, kConvThreads, lds, s>>>(a);
+    if constexpr (CIN == 16 && SOUT == 16)
+        conv16_kernel<OUTF><<<n * a.slabs, kConvThreads, lds, s>>>(a);
+    else
+        conv2_kernel<CIN, SP, OUTF><<<n * a.slabs, kConvThreads, lds, s>>>(a);
 }
 
-void forward(msbg_learned *net, hipStream_t s, const uint16_t *x0, const int32_t *idx, int n) {
+// The network's output of n tiles into y (f32 [tile][16^3]).
+void forward(msbg_learned *net, hipStream_t s, const uint16_t *x0, const int32_t *idx, int n, float *y) {
     const u4v *W = net->d_wb;
     const float *P = net->d_params;
     conv<2, 18, false>(s, x0, idx, 20, 0, W, P + 0 * kLP + kTap, 1, nullptr, net->A1, n);
     conv<16, 16, false>(s, net->A1, nullptr, 18, 0, W + kWB, P + 1 * kLP + kTap, 1, nullptr, net->A2, n);
     conv<16, 16, false>(s, net->A2, nullptr, 16, -1, W + 2 * kWB, P + 2 * kLP + kTap, 1, nullptr, net->A3, n);
-    conv<16, 16, true>(s, net->A3, nullptr, 16, -1, W + 3 * kWB, P + 3 * kLP + kTap, 0, nullptr, net->Y, n);
+    conv<16, 16, true>(s, net->A3, nullptr, 16, -1, W + 3 * kWB, P + 3 * kLP + kTap, 0, nullptr, y, n);
 }
 
 // Partials of one layer's weight gradient in net->wpart: layers 1..3 one of
@@ -801,7 +909,7 @@ const float *wgrad(msbg_learned *net, hipStream_t s, int l, const uint16_t *X, c
 // Loss and gradients of n tiles into net->d_grad; loss into net->d_loss (and loss_f if given).
 void loss_grad(msbg_learned *net, hipStream_t s, const uint16_t *x0, const float *target, const int32_t *idx, int n,
                float *loss_f) {
-    forward(net, s, x0, idx, n);
+    forward(net, s, x0, idx, n, net->Y);
     const double inv = 1.0 / ((double)n * 4096.0);
     const int nb = n * 16;
     loss_kernel<<<nb, 256, 0, s>>>(net->Y, target, idx, n, (float)inv, net->G4, net->loss_part);
@@ -860,7 +968,7 @@ int correct(msbg_poisson *p, msbg_learned *net, const msbg_grid *phi, float *x, 
         net_input_kernel<<<blocks_for((int64_t)n * 8000), 256, 0, s>>>(
             p->d_blocks + k0, p->dom, (int)p->nx, (int)p->ny, p->d_b2s, p->d_listed, p->d_r, p->d_scale, 0.0f,
             phi->d_slab, phi->d_b2s, x0, n);
-        forward(net, s, x0, nullptr, n);
+        forward(net, s, x0, nullptr, n, net->Y);
         delta_kernel<<<blocks_for((int64_t)n * 4096), 256, 0, s>>>(p->d_blocks + k0, p->dom, net->Y, net->out_scale,
                                                                    p->d_scale, p->d_delta, n);
     }
@@ -969,8 +1077,7 @@ int msbg_learned_forward(msbg_learned *n, const uint16_t *d_x0, int64_t count, f
     if (rc) return rc;
     for (int64_t k0 = 0; k0 < count; k0 += chunk) {
         const int c = (int)std::min<int64_t>(chunk, count - k0);
-        forward(n, stream(), d_x0 + k0 * 16000, nullptr, c);
-        MSBG_HIP(hipMemcpyAsync(d_y + k0 * 4096, n->Y, (size_t)c * 4096 * 4, hipMemcpyDeviceToDevice, stream()));
+        forward(n, stream(), d_x0 + k0 * 16000, nullptr, c, d_y + k0 * 4096);
     }
     MSBG_HIP(hipGetLastError());
     return MSBG_OK;

@@ -186,3 +186,21 @@ def test_gradient_of_a_repeated_batch(pkg, hip, n):
     for l in range(4):
         a, b = g1[l * 6928:(l + 1) * 6928], g2[l * 6928:(l + 1) * 6928]
         assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(a), (l, np.linalg.norm(a - b) / np.linalg.norm(a))
+
+
+@pytest.mark.parametrize("n", [513, 1030])
+def test_forward_in_chunks(pkg, hip, n):
+    """More tiles than one pass takes: every tile has the bits of a call of its
+    own, wherever in the batch it lies, with +-inf and NaN inputs in their tiles only."""
+    rng = np.random.default_rng(n)
+    p = random_params(rng)
+    five = bf16_bits(rng.normal(size=(5, 20, 20, 20, 2)))
+    five[3, 10, 10, 10, 0] = 0x7F80  # +inf
+    five[4, 3, 17, 9, 1] = 0x7FC0    # NaN
+    net = net_for(pkg, hip, p)
+    alone = np.concatenate([net.forward(hip.to_device(np.ascontiguousarray(t[None])), 1).get().reshape(1, 4096)
+                            for t in five])
+    which = rng.integers(0, 5, n)
+    got = net.forward(hip.to_device(np.ascontiguousarray(five[which])), n).get().reshape(n, 4096)
+    assert np.all(np.isfinite(alone[:3]))  # (the hidden layers' ReLU takes a NaN to 0)
+    assert np.array_equal(got.view(np.uint32), alone[which].view(np.uint32))
