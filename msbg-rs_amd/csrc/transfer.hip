@@ -190,20 +190,151 @@ __global__ void blend_kernel(const float *__restrict__ u_old, const float *__res
 struct MacViews {
     GridView v[3];
 };
+__device__ __forceinline__ float flip_blend(float u_old, float su, float st, float alpha) {
+    const float delta = su - st;  // g2p.rs:43-44
+    return (u_old + delta) * alpha + su * (1.0f - alpha);
+}
+
+template <int IP>
+__device__ __forceinline__ void g2p_flip_one(const MacViews &u, const MacViews &ut, const float *__restrict__ pos,
+                                             const float *__restrict__ u_old, int64_t i, int bc, float alpha,
+                                             float *__restrict__ out) {
+    const float p[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
+#pragma unroll 1
+    for (int a = 0; a < 3; ++a) {  // one axis at a time keeps the live registers of one sample pair
+        const float q[3] = {a == 0 ? p[0] - 0.5f : p[0], a == 1 ? p[1] - 0.5f : p[1], a == 2 ? p[2] - 0.5f : p[2]};
+        const float su = sample_ip<IP>(u.v[a], q[0], q[1], q[2], 1, bc);
+        const float st = sample_ip<IP>(ut.v[a], q[0], q[1], q[2], 1, bc);
+        out[3 * i + a] = flip_blend(u_old[3 * i + a], su, st, alpha);
+    }
+}
+
 template <int IP>
 __global__ void g2p_flip_kernel(MacViews u, MacViews ut, const float *__restrict__ pos,
                                 const float *__restrict__ u_old, int64_t n, int bc, float alpha,
                                 float *__restrict__ out) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const float p[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
-#pragma unroll 1
-        for (int a = 0; a < 3; ++a) {  // one axis at a time keeps the live registers of one sample pair
-            const float q[3] = {a == 0 ? p[0] - 0.5f : p[0], a == 1 ? p[1] - 0.5f : p[1], a == 2 ? p[2] - 0.5f : p[2]};
-            const float su = sample_ip<IP>(u.v[a], q[0], q[1], q[2], 1, bc);
-            const float st = sample_ip<IP>(ut.v[a], q[0], q[1], q[2], 1, bc);
-            const float delta = su - st;  // g2p.rs:43-44
-            out[3 * i + a] = (u_old[3 * i + a] + delta) * alpha + su * (1.0f - alpha);
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        g2p_flip_one<IP>(u, ut, pos, u_old, i, bc, alpha, out);
+}
+
+// The linear samples of 256 consecutive particles.  A sample waits for its
+// position, its blocks' slots and its values in turn, and those waits were the
+// kernel's time (87% of its waves', at a quarter of the memory rate).  So the
+// slots of the blocks around the work-group's particles go into LDS together,
+// and every particle then issues all of its 48 values, x pairs in one load
+// where a block holds both: three waits instead of nine.  A FLIP step's
+// particles come sorted along a Morton curve, so their blocks are few; a
+// work-group whose particles lie in more (any order is allowed), and particles
+// near the domain's bounds, go through sample_ip.  Both give its bits.
+// 67 M sorted particles: 5.35 ms through sample_ip, 3.96 so (in step, a
+// direction at a time, 4.9; from cells staged in LDS, whose boxes are twice the
+// particles' own cells, 5.35).
+constexpr int kFlipThreads = 256, kFlipBlocks = 64;
+__global__ __launch_bounds__(kFlipThreads) void g2p_flip_linear_kernel(MacViews u, MacViews ut,
+                                                                       const float *__restrict__ pos,
+                                                                       const float *__restrict__ u_old, int64_t n,
+                                                                       int bc, float alpha, float *__restrict__ out) {
+    __shared__ int s_box[6], s_slot[6][kFlipBlocks];
+    const int t = threadIdx.x;
+    const int64_t i = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * kFlipThreads + t;
+    const GridView &g = u.v[0];
+    if (t < 6) s_box[t] = t < 3 ? INT_MAX : INT_MIN;
+    float p[3] = {0.0f, 0.0f, 0.0f};
+    bool in = i < n;
+    if (in)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) p[d] = pos[3 * i + d];
+    // cells of all three directions: floor(p - 1) .. floor(p - 1/2) + 1, in
+    // sample_ip's roundings, all inside the domain (a NaN is not)
+    const float top[3] = {(float)(g.sx - 1), (float)(g.sy - 1), (float)(g.sz - 1)};
+    int lo[3] = {INT_MAX, INT_MAX, INT_MAX}, hi[3] = {INT_MIN, INT_MIN, INT_MIN};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) in = in && floorf((p[d] - 0.5f) - 0.5f) >= 0.0f && floorf(p[d] - 0.5f) + 1.0f <= top[d];
+    if (in)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            lo[d] = (int)floorf((p[d] - 0.5f) - 0.5f) >> 4;
+            hi[d] = ((int)floorf(p[d] - 0.5f) + 1) >> 4;
         }
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+        for (int o = 32; o > 0; o >>= 1) {
+            lo[d] = min(lo[d], __shfl_xor(lo[d], o));
+            hi[d] = max(hi[d], __shfl_xor(hi[d], o));
+        }
+    __syncthreads();
+    if ((t & 63) == 0 && lo[0] <= hi[0])
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            atomicMin(&s_box[d], lo[d]);
+            atomicMax(&s_box[3 + d], hi[d]);
+        }
+    __syncthreads();
+    const int bx0 = s_box[0], by0 = s_box[1], bz0 = s_box[2];
+    const bool any = s_box[3] >= bx0;
+    const int64_t nx = any ? s_box[3] - bx0 + 1 : 0, ny = any ? s_box[4] - by0 + 1 : 0, nz = any ? s_box[5] - bz0 + 1 : 0;
+    const bool few = any && nx * ny * nz <= kFlipBlocks;  // uniform over the work-group
+    const int nxy = (int)(nx * ny);
+    if (few)
+        for (int e = t; e < 6 * kFlipBlocks; e += kFlipThreads) {
+            const int a = e / kFlipBlocks, b = e % kFlipBlocks;
+            if (b >= nxy * (int)nz) continue;
+            const int64_t bid = (bx0 + b % (int)nx) + (int64_t)(by0 + (b % nxy) / (int)nx) * g.nx +
+                                (int64_t)(bz0 + b / nxy) * g.nx * g.ny;
+            s_slot[a][b] = a == 0   ? u.v[0].b2s[bid]
+                           : a == 1 ? u.v[1].b2s[bid]
+                           : a == 2 ? u.v[2].b2s[bid]
+                           : a == 3 ? ut.v[0].b2s[bid]
+                           : a == 4 ? ut.v[1].b2s[bid]
+                                    : ut.v[2].b2s[bid];
+        }
+    __syncthreads();
+    if (i >= n) return;
+    if (!few || !in) {
+        g2p_flip_one<0>(u, ut, pos, u_old, i, bc, alpha, out);
+        return;
+    }
+    float f[3][3];      // fractions of direction a
+    float2 e[3][2][4];  // the x pairs of direction a in u and u*
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        int c[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const float x = (d == a ? p[d] - 0.5f : p[d]) - 0.5f, b = floorf(x);
+            f[a][d] = x - b;
+            c[d] = (int)b;
+        }
+        const int vx = c[0] & 15, x0 = min(vx, 14);  // (a pair from 15 on would leave the row)
+        const bool X = vx == 15;
+        const int bx = (c[0] >> 4) - bx0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int y = c[1] + (k & 1), z = c[2] + (k >> 1);
+            const int b = bx + (int)nx * ((y >> 4) - by0) + nxy * ((z >> 4) - bz0), row = (y & 15) << 4 | (z & 15) << 8;
+#pragma unroll
+            for (int w = 0; w < 2; ++w) {
+                const float *slab = (w ? ut : u).v[a].slab;
+                float2 v;
+                __builtin_memcpy(&v, slab + ((int64_t)s_slot[a + 3 * w][b] << 12) + (row | x0), 8);
+                if (X) {
+                    v.x = v.y;
+                    v.y = slab[((int64_t)s_slot[a + 3 * w][b + 1] << 12) + row];
+                }
+                e[a][w][k] = v;
+            }
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        float r[2];
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const float c00 = lerp_f(e[a][w][0].x, e[a][w][0].y, f[a][0]), c10 = lerp_f(e[a][w][1].x, e[a][w][1].y, f[a][0]);
+            const float c01 = lerp_f(e[a][w][2].x, e[a][w][2].y, f[a][0]), c11 = lerp_f(e[a][w][3].x, e[a][w][3].y, f[a][0]);
+            r[w] = lerp_f(lerp_f(c00, c10, f[a][1]), lerp_f(c01, c11, f[a][1]), f[a][2]);
+        }
+        out[3 * i + a] = flip_blend(u_old[3 * i + a], r[0], r[1], alpha);
     }
 }
 
@@ -1107,7 +1238,11 @@ int msbg_g2p_flip(msbg_grid *const *vel, msbg_grid *const *vel_tilde, const floa
         u.v[a] = vel[a]->view();
         ut.v[a] = vel_tilde[a]->view();
     }
-    if (interp == 0)
+    const int64_t groups = (n + kFlipThreads - 1) / kFlipThreads;
+    if (interp == 0 && groups <= INT32_MAX)
+        hipLaunchKernelGGL(g2p_flip_linear_kernel, dim3((unsigned)groups), dim3(kFlipThreads), 0, stream(), u, ut, d_pos,
+                           d_u_old, n, bc, alpha, d_out);
+    else if (interp == 0)
         hipLaunchKernelGGL(g2p_flip_kernel<0>, dim3(grid_for(n, 256)), dim3(256), 0, stream(), u, ut, d_pos, d_u_old,
                            n, bc, alpha, d_out);
     else
