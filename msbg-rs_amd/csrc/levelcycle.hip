@@ -18,7 +18,10 @@
 // 71 (sweep), 63, 127 (prolongation and sweep) and 71 here.  A row of 8 cells
 // has 32 bytes and 30 instructions a cell, so it is bound by both.  On bands of
 // a few hundred blocks a pass takes its launch, 3 to 4 us, and a level has 5 of
-// them instead of 10.
+// them instead of 10; there the 2^3 level and the coarsest one are one launch.
+#include <algorithm>
+
+#include "coarse_cg.hpp"
 #include "poisson.hpp"
 
 namespace msbg {
@@ -431,6 +434,153 @@ __global__ __launch_bounds__(kWg) void level_restrict_kernel(LevelArgs A, float 
     bc[(i64)k * C3 + t] = 0.5f * ((s[0] + s[H]) + (s[B * H] + s[(B + 1) * H]));
 }
 
+// The 2^3 level and the coarsest one (a cell per block) in one work-group, on
+// bands of at most kCoarseMax blocks: nu sweeps from x = 0, the residual's sum,
+// the coarsest level's solution, its interpolation and nu sweeps back.  A lane
+// holds up to kTailRows rows of 2 cells (4 lanes to a block), one cell of each
+// colour, in registers with everything that it knows of them; other lanes see x
+// in LDS, so a half sweep is 5 LDS reads a row and one barrier.
+// What bounds it is latency, barriers and the iterations of the coarsest level's
+// solve, on one CU; seven launches (three sweeps of 4.3 us, 3.5, 2.9 and 4.6 us
+// for the first sweep, the restriction and the interpolation, 13 to 27 us for
+// the solve) took 37 us on 144 blocks, 41 on 450 and 51 on 704, it takes 20, 36
+// and 45.  As many lanes as there are rows: with a lane per block, 300 blocks
+// took 34 us instead of 31.
+constexpr int kTailRows = 4, kTailLanes = kCoarseMax;
+constexpr int kTailNone = 8 * kCoarseMax;  // two cells that hold 0
+
+__global__ __launch_bounds__(kTailLanes) void level_tail_kernel(LevelArgs A, CoarseArgs C, int nu) {
+    __shared__ float s_x[8 * kCoarseMax + 2];
+    __shared__ float s_c[kCoarseMax];
+    __shared__ int32_t s_nb[6 * kCoarseMax];  // the coarsest level's links, loaded with everything else
+    __shared__ float s_cf[6 * kCoarseMax];
+    __shared__ CoarseShared S;
+    const int t = threadIdx.x, lanes = blockDim.x, rows = 4 * A.n;
+    const int per = (rows + lanes - 1) / lanes;
+    float x[kTailRows][2], b[kTailRows][2], dg[kTailRows][2], inv[kTailRows][2];
+    int at[kTailRows], l[kTailRows], r[kTailRows], ym[kTailRows], yp[kTailRows], zm[kTailRows], zp[kTailRows];
+    bool live[kTailRows][2];
+    const int ry = t & 1, rz = (t >> 1) & 1, par = ry ^ rz;  // lanes is a multiple of 4
+    for (int i = t; i < 8 * A.n; i += lanes) s_x[i] = 0.0f;
+    if (t < 2) s_x[kTailNone + t] = 0.0f;
+    for (int i = t; i < 6 * C.n; i += lanes) {
+        s_nb[i] = C.nb[i];
+        s_cf[i] = C.cf[i];
+    }
+#pragma unroll
+    for (int j = 0; j < kTailRows; ++j) {
+        const int i = t + j * lanes, k = i >> 2;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            x[j][e] = b[j][e] = dg[j][e] = inv[j][e] = 0.0f;
+            live[j][e] = false;
+        }
+        at[j] = l[j] = r[j] = ym[j] = yp[j] = zm[j] = zp[j] = kTailNone;
+        if (i >= rows) continue;
+        const PBlock Bk = A.blocks[k];
+        LaneRow<2> R;
+        R.set(i & 3, k, Bk, A);
+        const int32_t *N = A.nb27 + (i64)k * 27;
+        const int vym = ry ? k : N[10], vyp = ry ? N[16] : k, vzm = rz ? k : N[4], vzp = rz ? N[22] : k;
+        const int row = 2 * ry + 4 * rz;
+        at[j] = 8 * k + row;
+        if (R.nbl >= 0) l[j] = 8 * R.nbl + row + 1;
+        if (R.nbr >= 0) r[j] = 8 * R.nbr + row;
+        if (vym >= 0) ym[j] = 8 * vym + (row ^ 2);
+        if (vyp >= 0) yp[j] = 8 * vyp + (row ^ 2);
+        if (vzm >= 0) zm[j] = 8 * vzm + (row ^ 4);
+        if (vzp >= 0) zp[j] = 8 * vzp + (row ^ 4);
+        if (!R.in) continue;
+        R.diagonals(k, Bk, A);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            b[j][e] = A.b[(i64)at[j] + e];
+            dg[j][e] = R.diag(e, inv[j][e]);
+            live[j][e] = e <= R.lim;
+        }
+    }
+    __syncthreads();
+    const auto neighbours = [&](int j, int e) {
+        const float xl = sel(e, x[j][0], s_x[l[j]]), xr = sel(e, s_x[r[j]], x[j][1]);
+        return ((((xl + xr) + s_x[ym[j] + e]) + s_x[yp[j] + e]) + s_x[zm[j] + e]) + s_x[zp[j] + e];
+    };
+    // the cells of one colour look at the other colour alone
+    const auto half = [&](int colour) {
+        const int e = par ^ colour;
+#pragma unroll
+        for (int j = 0; j < kTailRows; ++j) {
+            if (j >= per || t + j * lanes >= rows) continue;
+            const float v = relaxed(sel(e, x[j][1], x[j][0]), neighbours(j, e), sel(e, b[j][1], b[j][0]),
+                                    sel(e, dg[j][1], dg[j][0]), sel(e, inv[j][1], inv[j][0]), A.omega);
+            if (e ? live[j][1] : live[j][0]) {
+                x[j][0] = sel(e, x[j][0], v);
+                x[j][1] = sel(e, v, x[j][1]);
+                s_x[at[j] + e] = v;
+            }
+        }
+        __syncthreads();
+    };
+    for (int it = 0; it < nu; ++it) {
+        half(0);
+        half(1);
+    }
+#pragma unroll
+    for (int j = 0; j < kTailRows; ++j) {
+        const int i = t + j * lanes;
+        float p = 0.0f;
+        if (i < rows) {
+            float res[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                res[e] = live[j][e] ? b[j][e] + neighbours(j, e) - dg[j][e] * x[j][e] : 0.0f;
+            p = res[0] + res[1];
+        }
+        p += __shfl_xor(p, 1);
+        p += __shfl_xor(p, 2);
+        if (i < rows && (i & 3) == 0) s_c[i >> 2] = 0.5f * p;
+    }
+    __syncthreads();
+    const float xc = (float)coarse_cg(C, s_nb, s_cf, t < C.n ? s_c[t] : 0.0f, S);
+    __syncthreads();
+    if (t < C.n) s_c[t] = xc;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kTailRows; ++j) {
+        const int i = t + j * lanes, k = i >> 2;
+        if (i >= rows) continue;
+        const int32_t *N = A.nb27 + (i64)k * 27;
+        // towards the block on the cell's side; one beyond the domain is the cell itself
+        int dy = ry ? 3 : -3, dz = rz ? 9 : -9;
+        dy = N[13 + dy] == -2 ? 0 : dy;
+        dz = N[13 + dz] == -2 ? 0 : dz;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            if (!live[j][e]) continue;
+            const int dx = N[13 + (e ? 1 : -1)] == -2 ? 0 : (e ? 1 : -1);
+            float v = 0.0f;
+#pragma unroll
+            for (int kk = 0; kk < 8; ++kk) {
+                const int nb = N[13 + ((kk & 1) ? dx : 0) + ((kk & 2) ? dy : 0) + ((kk & 4) ? dz : 0)];
+                const float wt = ((kk & 1) ? 0.25f : 0.75f) * ((kk & 2) ? 0.25f : 0.75f) * ((kk & 4) ? 0.25f : 0.75f);
+                if (nb >= 0) v += wt * s_c[nb];
+            }
+            x[j][e] += v;
+            s_x[at[j] + e] = x[j][e];
+        }
+    }
+    __syncthreads();
+    for (int it = 0; it < nu; ++it) {
+        half(1);
+        half(0);
+    }
+#pragma unroll
+    for (int j = 0; j < kTailRows; ++j)
+        if (t + j * lanes < rows) {
+            A.dst[(i64)at[j]] = x[j][0];
+            A.dst[(i64)at[j] + 1] = x[j][1];
+        }
+}
+
 template <int B>
 void sweep(hipStream_t s, const LevelArgs &A, int from) {
     const int g = (A.n + Rows<B>::kBlocks - 1) / Rows<B>::kBlocks;
@@ -502,6 +652,15 @@ const float *level_after(const msbg_poisson *p, hipStream_t s, const int32_t *nb
         A.src = A.dst;
     }
     return A.src;
+}
+
+void level_tail(const msbg_poisson *p, hipStream_t s, const int32_t *nb27, float w, float omega, int nu,
+                const CoarseArgs &cg, const float *b, float *x) {
+    LevelArgs A = args_of(p, nb27, 2, w, omega, b);
+    A.dst = x;
+    // a row a lane up to 256 blocks, whole waves
+    const int lanes = std::min(kTailLanes, (4 * A.n + 63) / 64 * 64);
+    level_tail_kernel<<<1, lanes, 0, s>>>(A, cg, nu);
 }
 
 }  // namespace mg

@@ -10,6 +10,7 @@ using i64 = int64_t;
 
 namespace mg {
 struct Hierarchy;
+struct CoarseArgs;
 }
 
 // One listed value block: its slot, voxel origin and the slots of its six
@@ -172,6 +173,10 @@ void level_before(const msbg_poisson *p, hipStream_t s, const int32_t *nb27, int
                   float *x, float *y, const float *b, float *bc);
 const float *level_after(const msbg_poisson *p, hipStream_t s, const int32_t *nb27, int B, float w, float omega, int nu,
                          float *x, float *y, const float *b, const float *xc);
+// The 2^3 level before and after the coarsest level of one cell per block, and that level's solve, in one launch
+// (at most kCoarseMax blocks); the result in x.
+void level_tail(const msbg_poisson *p, hipStream_t s, const int32_t *nb27, float w, float omega, int nu,
+                const CoarseArgs &cg, const float *b, float *x);
 // The field that level_before leaves its result in.
 inline float *level_field(float *x, float *y, int nu) { return (nu & 1) ? x : y; }
 

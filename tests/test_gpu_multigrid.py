@@ -342,3 +342,13 @@ def test_one_cycle_equals_dense_arithmetic(pkg, orc, hip, s, seed, frac, storage
     assert st["sweeps"] == 2 * nu and st["levels"] == 5
     got = dense_from_slabs(g.b2s, dx.get().reshape(-1, 4096).astype(np.float64) - x, s)
     assert np.abs(got - e)[m].max() <= tol * np.abs(e).max() + 2.0 ** -23 * np.abs(x).max()
+
+
+@pytest.mark.parametrize("s,seed,frac,lo,hi", [((128, 122, 64), 6, 0.97, 193, 256), ((130, 128, 61), 7, 0.97, 257, 288),
+                                               ((127, 128, 250), 8, 0.97, 769, 1024)])
+def test_coarse_levels_of_one_to_four_rows_a_lane(pkg, orc, hip, s, seed, frac, lo, hi):
+    """The launch that holds the 2^3 level and the coarsest one, at one, two and
+    four rows a lane; the bound is FP32's of the test above."""
+    g, active, _, _ = band_problem(pkg, *s, seed, frac)
+    assert lo <= len(active) <= hi
+    test_one_cycle_equals_dense_arithmetic(pkg, orc, hip, s, seed, frac, 0, 1e-4, 2, False)
