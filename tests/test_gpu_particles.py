@@ -46,6 +46,28 @@ def test_radix_sort_is_stable_sort(hip, orc, n, bits):
     assert np.array_equal(dk.get(), keys[want])
 
 
+@pytest.mark.parametrize("tiles", [1, 15, 16, 17, 127, 128, 129])
+@pytest.mark.parametrize("odd", [0, 1])
+def test_radix_tables_about_the_short_scan(hip, orc, tiles, odd):
+    """Tables of 256 x tiles digit counts: less than, just and more than a round
+    of 4,096 entries, and about the 32,768 that one work-group scans."""
+    test_radix_sort_is_stable_sort(hip, orc, 4096 * tiles - odd, 8)
+
+
+@pytest.mark.parametrize("nb", [(1, 1, 1), (3, 1, 1), (5, 3, 7), (16, 16, 17), (32, 32, 32), (33, 31, 33)])
+def test_active_blocks_of_odd_grids(hip, orc, nb):
+    """Flags of 1 to 33,759 blocks, most of their counts no multiple of 4."""
+    rng = np.random.default_rng(nb[0] + 100 * nb[2])
+    s = [16 * k for k in nb]
+    pos = (rng.random((200, 3)) * s).astype(np.float32)
+    got = P.active_blocks(*s, pos, 4.0, lib=hip)
+    lo = np.clip(np.floor(pos / 16 - 0.25).astype(int), 0, None)  # both bounds are exact in float32
+    hi = np.minimum(np.trunc(pos / 16 + 0.25).astype(int), np.array(nb) - 1)
+    want = {x + nb[0] * (y + nb[1] * z) for l, h in zip(lo, hi) for x in range(l[0], h[0] + 1)
+            for y in range(l[1], h[1] + 1) for z in range(l[2], h[2] + 1)}
+    assert got.tolist() == sorted(want)
+
+
 def test_morton_sort_matches_oracle(hip, orc):
     rng = np.random.default_rng(3)
     pos = rng.uniform(0, 512, size=(300_000, 3)).astype(np.float32)
