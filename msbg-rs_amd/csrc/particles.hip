@@ -213,6 +213,22 @@ int noalloc_scratch(uint32_t **out) {
     return MSBG_OK;
 }
 
+int active_blocks_flagged(int64_t sx, int64_t sy, int64_t sz, const float *d_pos, int64_t n, float r_scan,
+                          int32_t *d_out, int64_t *n_out, const uint32_t **flags) {
+    MSBG_CHECK(n_out && d_out, MSBG_EINVAL, "active_blocks: null output");
+    MSBG_CHECK(sx > 0 && sy > 0 && sz > 0 && n >= 0 && (n == 0 || d_pos), MSBG_EINVAL, "active_blocks: bad argument");
+    const int32_t nx = (int32_t)((sx + 15) >> 4), ny = (int32_t)((sy + 15) >> 4), nz = (int32_t)((sz + 15) >> 4);
+    const int64_t nb = (int64_t)nx * ny * nz;
+    MSBG_CHECK(nb < ((int64_t)1 << 31), MSBG_EINVAL, "active_blocks: block grid too large for a dense flag array");
+    int rc;
+    uint32_t *marks = (uint32_t *)workspace(5, sizeof(uint32_t) * 2 * nb, &rc);
+    if (rc) return rc;
+    uint32_t *sums = (uint32_t *)workspace(0, sizeof(uint32_t) * scan_sums_words(nb), &rc);
+    if (rc) return rc;
+    *flags = marks;
+    return active_blocks_into(d_pos, n, r_scan, nx, ny, nz, marks, marks + nb, sums, d_out, n_out);
+}
+
 int morton_sort_async(const float *d_pos, int64_t n, uint32_t *d_keys, uint32_t *d_perm) {
     if (n == 0) return MSBG_OK;
     hipLaunchKernelGGL(morton_keys_kernel, dim3(grid_for(n)), dim3(256), 0, stream(), d_pos, n, d_keys, d_perm);
@@ -316,17 +332,8 @@ int msbg_bucket_indices(const int32_t *d_bids, int64_t n, int64_t n_blocks, int3
 
 int msbg_active_blocks(int64_t sx, int64_t sy, int64_t sz, const float *d_pos, int64_t n, float r_scan,
                        int32_t *d_out, int64_t *n_out) {
-    MSBG_CHECK(n_out && d_out, MSBG_EINVAL, "active_blocks: null output");
-    MSBG_CHECK(sx > 0 && sy > 0 && sz > 0 && n >= 0 && (n == 0 || d_pos), MSBG_EINVAL, "active_blocks: bad argument");
-    const int32_t nx = (int32_t)((sx + 15) >> 4), ny = (int32_t)((sy + 15) >> 4), nz = (int32_t)((sz + 15) >> 4);
-    const int64_t nb = (int64_t)nx * ny * nz;
-    MSBG_CHECK(nb < ((int64_t)1 << 31), MSBG_EINVAL, "active_blocks: block grid too large for a dense flag array");
-    int rc;
-    uint32_t *flags = (uint32_t *)workspace(5, sizeof(uint32_t) * 2 * nb, &rc);
-    if (rc) return rc;
-    uint32_t *sums = (uint32_t *)workspace(0, sizeof(uint32_t) * scan_sums_words(nb), &rc);
-    if (rc) return rc;
-    return active_blocks_into(d_pos, n, r_scan, nx, ny, nz, flags, flags + nb, sums, d_out, n_out);
+    const uint32_t *flags;
+    return active_blocks_flagged(sx, sy, sz, d_pos, n, r_scan, d_out, n_out, &flags);
 }
 
 int msbg_active_blocks_noalloc(int64_t sx, int64_t sy, int64_t sz, const float *d_pos, int64_t n, float r_scan,

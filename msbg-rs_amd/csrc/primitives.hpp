@@ -22,6 +22,11 @@ int64_t scan_sums_words(int64_t n);
 // Stable sort of (keys, vals) in place, keys below 2^key_bits.
 int radix_sort_pairs(uint32_t *keys, uint32_t *vals, int64_t n, int key_bits);
 
+// msbg_active_blocks, with a flag per block of the lattice (1: active), valid
+// until the next call for active blocks.
+int active_blocks_flagged(int64_t sx, int64_t sy, int64_t sz, const float *d_pos, int64_t n, float r_scan,
+                          int32_t *d_out, int64_t *n_out, const uint32_t **flags);
+
 // msbg_morton_sort without the final synchronization (stream-ordered).
 int morton_sort_async(const float *d_pos, int64_t n, uint32_t *d_keys, uint32_t *d_perm);
 // Some order along a Morton curve over the domain (keys and particle indices):

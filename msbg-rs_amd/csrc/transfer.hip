@@ -856,6 +856,7 @@ __device__ __forceinline__ void acc_add(Acc4 &a, float wxy, float pz, int cz, fl
 template <int ORDER, int SPAN>
 __global__ __launch_bounds__(256) void p2g_bspline_kernel(GridView mg, GridView v0, GridView v1, GridView v2,
                                                           const int32_t *__restrict__ active,
+                                                          const uint32_t *__restrict__ flags,
                                                           const uint2 *__restrict__ range,
                                                           const float4 *__restrict__ pm,
                                                           const float4 *__restrict__ pu) {
@@ -869,9 +870,16 @@ __global__ __launch_bounds__(256) void p2g_bspline_kernel(GridView mg, GridView 
     if (threadIdx.x < 27) {
         const int t = threadIdx.x;
         const int nx = bx + t % 3 - 1, ny = by + (t / 3) % 3 - 1, nz = bz + t / 9 - 1;
-        s_nb[t] = (nx >= 0 && nx < mg.nx && ny >= 0 && ny < mg.ny && nz >= 0 && nz < mg.nz)
-                      ? mg.b2s[nx + (int64_t)ny * mg.nx + (int64_t)nz * mg.nx * mg.ny]
-                      : 0;
+        // only blocks active in this call have ranges; a value block that is not
+        // (one of an earlier call, or the caller's own) holds no particle
+        int slot = 0;
+        if (nx >= 0 && nx < mg.nx && ny >= 0 && ny < mg.ny && nz >= 0 && nz < mg.nz) {
+            const int64_t nb = nx + (int64_t)ny * mg.nx + (int64_t)nz * mg.nx * mg.ny;
+            const uint32_t on = flags[nb];
+            slot = mg.b2s[nb];
+            if (!on) slot = 0;
+        }
+        s_nb[t] = slot;
     }
     __syncthreads();
     const int ms = s_nb[13];
@@ -1163,15 +1171,17 @@ int check_same_dims(msbg_grid *const *grids, int ng) {
     return MSBG_OK;
 }
 
-// Active blocks of the particles (device list), downloaded.
+// Active blocks of the particles (device list, and a flag per block), downloaded.
 int active_list(const msbg_grid *g, const float *d_pos, int64_t n, float r_scan, std::vector<int64_t> &out,
-                int32_t **d_list) {
+                int32_t **d_list, const uint32_t **d_flags = nullptr) {
     int rc;
     int32_t *d_act = (int32_t *)workspace(6, sizeof(int32_t) * std::max<int64_t>(g->n_blocks, 1), &rc);
     if (rc) return rc;
     int64_t k = 0;
-    rc = msbg_active_blocks(g->sx, g->sy, g->sz, d_pos, n, r_scan, d_act, &k);
+    const uint32_t *flags = nullptr;
+    rc = active_blocks_flagged(g->sx, g->sy, g->sz, d_pos, n, r_scan, d_act, &k, &flags);
     if (rc) return rc;
+    if (d_flags) *d_flags = flags;
     std::vector<int32_t> h((size_t)k);
     if (k) MSBG_HIP(hipMemcpy(h.data(), d_act, sizeof(int32_t) * k, hipMemcpyDeviceToHost));
     out.assign(h.begin(), h.end());
@@ -1414,7 +1424,8 @@ int msbg_p2g_bspline(int order, msbg_grid *mass, msbg_grid *const *vel, const fl
     // support cells floor(p)-1 .. floor(p)+1 lie in the footprint blocks of r_scan 2
     std::vector<int64_t> act;
     int32_t *d_act = nullptr;
-    rc = active_list(mass, d_pos, n, 2.0f, act, &d_act);
+    const uint32_t *d_flags = nullptr;
+    rc = active_list(mass, d_pos, n, 2.0f, act, &d_act, &d_flags);
     if (rc) return rc;
     rc = zero_blocks(all, 4, act);
     if (rc) return rc;
@@ -1436,8 +1447,8 @@ int msbg_p2g_bspline(int order, msbg_grid *mass, msbg_grid *const *vel, const fl
     if (rc) return rc;
     float4 *pm = pay, *pu = pay + n;
     hipLaunchKernelGGL(gather_records_kernel, dim3(grid_for(n, 256)), dim3(256), 0, stream(), rec, perm, n, pm, pu);
-    // per-voxel ranges of the sorted particles, indexed like the mass slab; the
-    // dummy slots' are never looked at
+    // per-voxel ranges of the sorted particles, indexed like the mass slab; those
+    // of blocks that are not active are neither written nor looked at
     uint2 *range = (uint2 *)workspace(8, sizeof(uint2) * mass->n_slots * 4096, &rc);
     if (rc) return rc;
     hipLaunchKernelGGL(voxel_ranges_kernel, dim3((unsigned)act.size()), dim3(256), 0, stream(), keys, (uint32_t)n, d_act,
@@ -1446,7 +1457,7 @@ int msbg_p2g_bspline(int order, msbg_grid *mass, msbg_grid *const *vel, const fl
     const unsigned na = (unsigned)act.size();
     const auto spread = [&](auto kernel, int span) {
         kernel<<<na * (16 / span), 256, 0, stream()>>>(mass->view(), vel[0]->view(), vel[1]->view(), vel[2]->view(),
-                                                       d_act, range, pm, pu);
+                                                       d_act, d_flags, range, pm, pu);
     };
     // Up to 8 columns of a work-group a CU fit at once, and fewer leave it idle
     // (1 M particles, 350 blocks: 375 us whole, 141 in spans of 4, 164 of 2; 16.8 M,

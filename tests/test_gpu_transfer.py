@@ -489,3 +489,32 @@ def test_p2g_bspline_rows_and_strays(pkg, orc, hip, order, s, spread):
     assert_bitexact(tg.mass.to_host().to_dense(), dense_from_slabs(b2s, slabs[0], s), "mass")
     for a in range(3):
         assert_bitexact(tg.velocity[a].to_host().to_dense(), dense_from_slabs(b2s, slabs[1 + a], s), "vel %d" % a)
+
+
+@pytest.mark.parametrize("order", [1, 2])
+@pytest.mark.parametrize("ensured", [False, True])
+def test_p2g_bspline_on_a_grid_used_before(pkg, orc, hip, order, ensured):
+    """One grid, four calls: a cloud, the cloud moved by 20 cells, a tenth of
+    it elsewhere, and the cloud again.  Blocks of an earlier call, and blocks
+    that the caller ensured, border the active ones and hold no particle: the
+    active blocks have the oracle's bits of each call alone."""
+    s = (96, 80, 112)
+    rng = np.random.default_rng(order)
+    cloud = rng.uniform(8.0, [60.0, 50.0, 70.0], (30000, 3)).astype(np.float32)
+    vel = rng.normal(size=cloud.shape).astype(np.float32)
+    mass = rng.uniform(0.5, 2.0, cloud.shape[0]).astype(np.float32)
+    tg = T.TransferGrid(*s, capacity_blocks=6 * 5 * 7 + 8, lib=hip)
+    grids = [tg.mass] + tg.velocity
+    if ensured:
+        every = np.arange(tg.mass.n_blocks, dtype=np.int64)
+        for g in grids:
+            hip.call("msbg_grid_ensure_blocks", g.h, every.ctypes.data, every.size)
+    tenth = slice(0, cloud.shape[0] // 10)
+    for pos, part in ((cloud, slice(None)), (cloud + np.float32(20.0), slice(None)),
+                      (cloud[tenth] * np.float32(0.3) + np.float32(40.0), tenth), (cloud, slice(None))):
+        u, m = np.ascontiguousarray(vel[part]), np.ascontiguousarray(mass[part])
+        active, b2s, slabs = oracle_p2g_bspline(orc, order, s, pos, u, m)
+        assert tg.p2g(order, pos, u, m) == active.size
+        for g, want in zip(grids, slabs):
+            h = g.to_host()
+            assert_bitexact(h.slab[h.b2s[active]], want[b2s[active]], "active blocks")
