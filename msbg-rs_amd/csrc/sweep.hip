@@ -1238,12 +1238,17 @@ int launch_flow(msbg_sweep_plan *p, hipStream_t s, TS *fslab, int stencil, float
     return launch_flow_st<MSBG_BILAPLACIAN, MULTI, TS>(p, s, fslab, dt, clamp01, sweeps);
 }
 
+// Work-groups of a one-launch sweep: a launch has fewer than 2^32 lanes along
+// an axis, and 2^20 groups are ~50 ms, beside which a launch costs nothing.
+constexpr int64_t kFlowGroups = (int64_t)1 << 20;
+static_assert(kFlowGroups * kFlowThreads < (int64_t)1 << 32 && kFlowMost <= kFlowGroups, "groups of one launch");
+
 // `iterations` sweeps as one launch (Density8: one a sweep, whose number keys
-// its rounding), or several when their blocks would exceed 2^24.
+// its rounding), or several when they take more than kFlowGroups groups.
 int launch_flow_sweeps(msbg_sweep_plan *p, hipStream_t s, int stencil, float dt, int iterations, int clamp01) {
-    const int most = p->slab8 ? 1 : (int)(((int64_t)1 << 24) / p->flow.n);
-    for (int it = 0; it < iterations; it += most) {
-        const unsigned sweeps = (unsigned)std::min(most, iterations - it);
+    const int64_t most = p->slab8 ? 1 : kFlowGroups / p->flow.n;
+    for (int64_t it = 0; it < iterations; it += most) {
+        const unsigned sweeps = (unsigned)std::min<int64_t>(most, iterations - it);
         int rc;
         if (p->coarse)
             rc = launch_flow<true, float>(p, s, p->g->d_slab, stencil, dt, clamp01, sweeps);

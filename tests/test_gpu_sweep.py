@@ -447,3 +447,17 @@ def test_one_launch_sweeps_of_many_iterations(pkg, hip):
         hip.call("msbg_sweep_plan_free", plan)
         out.append(d.get())
     assert np.array_equal(out[0], out[1])
+
+
+def test_one_launch_sweeps_past_a_launch(pkg, hip):
+    """4,100 sweeps of 1,024 blocks are 4.2 M blocks, more than the 2^32 lanes
+    of a launch hold: several launches in a row, with the bits of 4,100 rounds
+    of colour passes."""
+    g, active = shuffled_plan_problem(pkg, 1024, (208, 193, 181), 9)
+    ga, gb = pkg.DeviceGrid.from_host(g, lib=hip), pkg.DeviceGrid.from_host(g, lib=hip)
+    pa, pb = pkg.SweepPlan(ga, active), pkg.SweepPlan(gb, active)
+    pa.run_async(0, 0.1, 4100, True)
+    for _ in range(41):
+        pb.run_timed(0, 0.1, 100, True)
+    hip.synchronize()
+    assert_bitexact(ga.to_host().slab, gb.to_host().slab, "4100 sweeps")
