@@ -15,6 +15,7 @@
 #include <climits>
 #include <vector>
 
+#include "launch.hpp"
 #include "primitives.hpp"
 
 namespace msbg {
@@ -1249,7 +1250,7 @@ int msbg_g2p_flip(msbg_grid *const *vel, msbg_grid *const *vel_tilde, const floa
         ut.v[a] = vel_tilde[a]->view();
     }
     const int64_t groups = (n + kFlipThreads - 1) / kFlipThreads;
-    if (interp == 0 && groups <= INT32_MAX)
+    if (interp == 0 && groups <= max_groups(kFlipThreads))  // a lane a particle; past 2^32 lanes stride
         hipLaunchKernelGGL(g2p_flip_linear_kernel, dim3((unsigned)groups), dim3(kFlipThreads), 0, stream(), u, ut, d_pos,
                            d_u_old, n, bc, alpha, d_out);
     else if (interp == 0)

@@ -518,3 +518,25 @@ def test_p2g_bspline_on_a_grid_used_before(pkg, orc, hip, order, ensured):
         for g, want in zip(grids, slabs):
             h = g.to_host()
             assert_bitexact(h.slab[h.b2s[active]], want[b2s[active]], "active blocks")
+
+
+def test_g2p_flip_past_the_lanes_of_a_launch(pkg, hip):
+    """2^32 + 300 particles, more than a launch has lanes: all at one place,
+    and their first, middle and last results are those of a small call."""
+    s, n = (32, 32, 32), 2 ** 32 + 300
+    from test_gpu_flip import mac_from_channels
+    macs = [mac_from_channels(pkg, hip, mac_channels(pkg, s, lambda a, X, Y, Z: np.sin(0.21 * X + a + k) + 0.03 * Z))
+            for k in (0, 1)]
+    x = np.float32(13.37)
+    want = T.g2p_flip(*macs, np.full((256, 3), x, np.float32), np.full((256, 3), x, np.float32), 0.95).get()
+    pos = hip.empty((n, 3), np.float32)  # positions and old velocities at once
+    word, piece = int(x.view(np.uint32)), 2 ** 30
+    for at in range(0, 3 * n, piece):
+        hip.call("msbg_fill_u32", pos.ptr + 4 * at, min(piece, 3 * n - at), word)
+    out = T.g2p_flip(*macs, pos, pos, 0.95)
+    got = np.empty((256, 3), np.float32)
+    for first in (0, n // 2, n - 256):
+        hip.call("msbg_memcpy_dtoh", got.ctypes.data, out.ptr + 12 * first, got.nbytes)
+        assert_bitexact(got, want, "g2p flip")
+    pos.free()
+    out.free()
