@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "internal.hpp"
+#include "launch.hpp"
 #include "primitives.hpp"
 
 namespace msbg {
@@ -256,9 +257,11 @@ int msbg_density_splat(msbg_grid *g, uint16_t *d_slab16, int64_t slab_slots, con
     if (lds > 65536)
         MSBG_HIP(hipFuncSetAttribute((const void *)density_splat_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)lds));
-    if (!order.empty())
-        density_splat_kernel<<<(unsigned)order.size(), kSplatThreads, lds, s>>>(P, g->d_b2s, d_slab16, d_sorted,
-                                                                              d_blocks, d_items);
+    // (past 8.4 M items, which take a domain of 6 M occupied blocks, a second launch)
+    const int64_t n_items = (int64_t)order.size(), most = max_groups(kSplatThreads);
+    for (int64_t i = 0; i < n_items; i += most)
+        density_splat_kernel<<<(unsigned)std::min(most, n_items - i), kSplatThreads, lds, s>>>(
+            P, g->d_b2s, d_slab16, d_sorted, d_blocks, d_items + i);
     MSBG_HIP(hipGetLastError());
     MSBG_HIP(hipStreamSynchronize(s));
     return MSBG_OK;

@@ -7,6 +7,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
+# (256: FLIP G2P; 512: the density splat, whose split takes ~200 GB of grid to reach)
 @pytest.mark.parametrize("threads", [64, 256, 448, 512, 1024])
 def test_lanes_of_a_launch_stay_below_2_to_the_32(tmp_path, threads):
     src = tmp_path / "limit.cpp"
