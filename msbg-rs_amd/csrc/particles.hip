@@ -325,7 +325,8 @@ int msbg_bucket_indices(const int32_t *d_bids, int64_t n, int64_t n_blocks, int3
     MSBG_HIP(hipMemcpyAsync(keys, d_bids, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, stream()));
     hipLaunchKernelGGL(iota_kernel, dim3(grid_for(n)), dim3(256), 0, stream(), (uint32_t *)d_perm, n);
     MSBG_HIP(hipGetLastError());
-    rc = radix_sort_pairs(keys, (uint32_t *)d_perm, n, bits_for(n_blocks - 1));
+    // whole bytes: a particle on the domain's upper z bound has an id past the last block's
+    rc = radix_sort_pairs(keys, (uint32_t *)d_perm, n, (bits_for(n_blocks - 1) + 7) / 8 * 8);
     if (rc) return rc;
     return run_lengths(keys, n, d_particle_blocks, d_starts, n_occupied);
 }

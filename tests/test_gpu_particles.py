@@ -143,3 +143,23 @@ def test_gather_rows(hip):
     perm = rng.permutation(1000).astype(np.uint32)
     got = P.gather_rows(hip.to_device(src), hip.to_device(perm), lib=hip).get()
     assert np.array_equal(got, src[perm])
+
+
+@pytest.mark.parametrize("s", [(80, 80, 80), (64, 64, 128), (320, 320, 640)])
+def test_bucket_indices_of_the_upper_z_bound(hip, s):
+    """Particles on the upper z bound have ids past the last block, here with a
+    bit more than those of 125, 128 and 16,000 blocks: every id once, ascending,
+    its particles in input order."""
+    nb = [(k + 15) // 16 for k in s]
+    rng = np.random.default_rng(s[0])
+    pos = rng.uniform(0.0, np.array(s) - 1e-3, (5000, 3)).astype(np.float32)
+    pos[::3, 2] = s[2]
+    bids = P.particle_bids(*s, pos, lib=hip)
+    ids = bids.get()
+    n_blocks = nb[0] * nb[1] * nb[2]
+    assert int(ids.max()).bit_length() > (n_blocks - 1).bit_length()
+    plan = P.bucket_indices(bids, n_blocks, lib=hip)
+    blocks, counts = np.unique(ids, return_counts=True)
+    pb, starts, perm = plan.host()
+    assert np.array_equal(pb, blocks) and np.array_equal(starts, np.concatenate([[0], np.cumsum(counts)]))
+    assert np.array_equal(perm, np.argsort(ids, kind="stable"))
