@@ -56,6 +56,14 @@ __device__ __forceinline__ void atomic_min_2xu16(uint32_t *w, uint32_t lo, uint3
     }
 }
 
+// Lowers one 16-bit cell, by its aligned word (in a slab that starts between
+// words the pair of atomic_min_2xu16 is no aligned word).
+__device__ __forceinline__ void atomic_min_u16(uint16_t *p, uint32_t v) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(p);
+    const bool high = (a & 2) != 0;
+    atomic_min_2xu16(reinterpret_cast<uint32_t *>(a & ~(uintptr_t)3), high ? 0xffffu : v, high ? v : 0xffffu);
+}
+
 // LDS atomics bound it: ~270 cells a particle at r_scan = 4.
 __global__ __launch_bounds__(kSplatThreads) void density_splat_kernel(SplatParams P, const int32_t *__restrict__ b2s,
                                                                       uint16_t *slab, const float *__restrict__ pos,
@@ -137,6 +145,7 @@ __global__ __launch_bounds__(kSplatThreads) void density_splat_kernel(SplatParam
     // region; with an odd margin the first and last word's outer cell is not
     // the window's), dst = min(dst, code)
     const int odd = m & 1, words = (W + 2 * odd) / 2;
+    const bool words_apart = (reinterpret_cast<uintptr_t>(slab) & 2) != 0;
     auto code = [&](int cx, int row) -> uint32_t {
         if (cx < 0 || cx >= W) return 0xffffu;
         const uint32_t v = st[row + cx];
@@ -153,7 +162,12 @@ __global__ __launch_bounds__(kSplatThreads) void density_splat_kernel(SplatParam
         if (slot < 0) continue;
         const int gx = b0x + cx - m, gy = b0y + cy - m, gz = b0z + cz - m;
         uint16_t *d = slab + ((int64_t)slot << 12) + ((gx & 15) | ((gy & 15) << 4) | ((gz & 15) << 8));
-        atomic_min_2xu16(reinterpret_cast<uint32_t *>(d), lo, hi16);
+        if (words_apart) {
+            if (lo != 0xffffu) atomic_min_u16(d, lo);
+            if (hi16 != 0xffffu) atomic_min_u16(d + 1, hi16);
+        } else {
+            atomic_min_2xu16(reinterpret_cast<uint32_t *>(d), lo, hi16);
+        }
     }
 }
 

@@ -1,5 +1,7 @@
 """GPU parity of the transfers: the reference sampler, MAC P2G and the
 B-spline P2G / G2P against the oracle."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -540,3 +542,26 @@ def test_g2p_flip_past_the_lanes_of_a_launch(pkg, hip):
         assert_bitexact(got, want, "g2p flip")
     pos.free()
     out.free()
+
+
+@pytest.mark.parametrize("r_scan", [4.0, 4.5])
+def test_density_splat_into_a_slab_between_words(pkg, hip, r_scan):
+    """A u16 slab 2 bytes past a 4-byte boundary gets the cells of an aligned
+    one (split dense blocks among them), and the cells beside it stay."""
+    from msbg_rs_amd.particles import DensityGrid
+    s, n = (48, 40, 33), 6000
+    rng = np.random.default_rng(5)
+    pos = rng.uniform(0.0, np.array(s) - 1e-3, (n, 3)).astype(np.float32)
+    pos[:2500] = rng.uniform(17.0, 22.0, (2500, 3))
+    aligned, odd = (DensityGrid(*s, capacity_blocks=27 + 4, lib=hip) for _ in range(2))
+    aligned.splat(pos, r_scan)
+    b2s, want = aligned.to_host()
+    cells = odd.slots * 4096
+    buf = hip.to_device(np.full(cells + 2, 0x1234, np.uint16))
+    k, d = C.c_int64(), hip.to_device(pos)
+    hip.call("msbg_density_splat", odd.layout.h, buf.ptr + 2, odd.slots, d.ptr, n, r_scan, C.byref(k))
+    host = buf.get()
+    got = host[1 : 1 + want.size].reshape(want.shape)
+    assert np.array_equal(odd.layout.to_host().b2s, b2s)
+    assert np.array_equal(got, want)
+    assert host[0] == 0x1234 and np.all(host[1 + want.size :] == 0x1234)
