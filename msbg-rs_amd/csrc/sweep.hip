@@ -973,7 +973,7 @@ struct msbg_sweep_plan {
     uint32_t sr_seed = 0;        // Density8: stochastic-rounding seed
     uint32_t *d_sr_ctr = nullptr;  // Density8: sweeps done by this plan (device)
     // One-launch sweeps (sweep_flow_kernel): n = 0 when the plan has none
-    // (all-level plans, large bands, repeated block ids).
+    // (all-level plans, large bands, repeated block ids, misaligned u16 / u8 slabs).
     msbg::FlowArgs flow{nullptr, nullptr, nullptr, 0};
     // All-level plans (msbg_sweep_plan_new_levels): g / coarse are levels 0
     // and 1, d_bids / d_topo / counts the level-0 blocks; the coarse blocks
@@ -1514,7 +1514,8 @@ int msbg_sweep_plan_new(msbg_grid *g, const int64_t *active, int64_t n, msbg_swe
 int msbg_sweep_plan_new_density(msbg_grid *layout, uint16_t *d_slab16, const int64_t *active, int64_t n,
                                 msbg_sweep_plan **out) {
     MSBG_CHECK(d_slab16, MSBG_EINVAL, "density plan: null u16 slab");
-    int rc = plan_new(layout, nullptr, nullptr, active, n, out);
+    // the one-launch sweeps' accesses are atomic: they need the slab's quads aligned
+    int rc = plan_new(layout, nullptr, nullptr, active, n, out, ((uintptr_t)d_slab16 & 7) == 0);
     if (rc) return rc;
     (*out)->slab16 = d_slab16;
     return MSBG_OK;
@@ -1539,7 +1540,7 @@ int msbg_sweep_density(msbg_grid *layout, uint16_t *d_slab16, const int64_t *act
 int msbg_sweep_plan_new_density8(msbg_grid *layout, uint8_t *d_slab8, const int64_t *active, int64_t n,
                                  uint32_t seed, msbg_sweep_plan **out) {
     MSBG_CHECK(d_slab8, MSBG_EINVAL, "density8 plan: null u8 slab");
-    int rc = plan_new(layout, nullptr, nullptr, active, n, out);
+    int rc = plan_new(layout, nullptr, nullptr, active, n, out, ((uintptr_t)d_slab8 & 3) == 0);
     if (rc) return rc;
     msbg_sweep_plan *p = *out;
     p->slab8 = d_slab8;

@@ -461,3 +461,35 @@ def test_one_launch_sweeps_past_a_launch(pkg, hip):
         pb.run_timed(0, 0.1, 100, True)
     hip.synchronize()
     assert_bitexact(ga.to_host().slab, gb.to_host().slab, "4100 sweeps")
+
+
+def density_at_offset(pkg, orc, hip, stencil, dt, dtype, offset):
+    """Two sweeps of a density slab `offset` bytes past an aligned address:
+    (device cells, oracle's)."""
+    import ctypes as C
+    from test_oracle_density import density_of, sweep16
+    g = random_grid(pkg, 64, 48, 80, seed=31 + stencil, lo=0.0, hi=1.0, empty=0.0, full=1.0)
+    active = np.nonzero(g.b2s >= 2)[0].astype(np.int64)
+    q = density_of(g)
+    if dtype == np.uint8:
+        q = (q >> 8).astype(np.uint8)
+        want = q.copy()
+        orc.orc_sweep_density8(g.sx, g.sy, g.sz, want, g.n_slots, g.b2s, active, active.size, stencil, dt, 2, 1, 5, 0)
+    else:
+        q[0], q[1] = 0, 65535
+        want = sweep16(orc, g, q, active, stencil, dt, it=2)
+    layout = pkg.DeviceGrid.from_host(g, lib=hip)
+    buf = hip.to_device(np.concatenate([np.zeros(offset, np.uint8), q.reshape(-1).view(np.uint8)]))
+    if dtype == np.uint8:
+        hip.call("msbg_sweep_density8", layout.h, buf.ptr + offset, active.ctypes.data, active.size, stencil, dt, 2, 1, 5)
+    else:
+        hip.call("msbg_sweep_density", layout.h, buf.ptr + offset, active.ctypes.data, active.size, stencil, dt, 2, 1)
+    return np.ascontiguousarray(buf.get()[offset:]).view(dtype).reshape(want.shape), want
+
+
+@pytest.mark.parametrize("stencil,dt", [(0, 0.1), (1, 0.02), (2, 0.005)])
+@pytest.mark.parametrize("offset", [2, 4, 8])
+def test_density_sweep_of_a_slab_between_quads(pkg, orc, hip, stencil, dt, offset):
+    """u16 slabs on any cell boundary."""
+    got, want = density_at_offset(pkg, orc, hip, stencil, dt, np.uint16, offset)
+    assert np.array_equal(got, want)
