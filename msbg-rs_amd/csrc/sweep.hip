@@ -425,7 +425,7 @@ __device__ __forceinline__ void fill_tile_rows(float *tile, const TS *fs, const 
     for (int k = 0; k < QI; ++k) {
         qv[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (!qe[k]) continue;
-        const TS *p = reinterpret_cast<const TS *>(qe[k] & ~1ull);
+        const TS *p = reinterpret_cast<const TS *>(MULTI ? qe[k] & ~1ull : qe[k]);  // (a u8 row's address may be odd)
         qv[k] = ld_quad<COH>(p + (MULTI && (qe[k] & 1) ? 4 * (q >> 1) : 4 * q));
     }
 #pragma unroll

@@ -493,3 +493,11 @@ def test_density_sweep_of_a_slab_between_quads(pkg, orc, hip, stencil, dt, offse
     """u16 slabs on any cell boundary."""
     got, want = density_at_offset(pkg, orc, hip, stencil, dt, np.uint16, offset)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("stencil,dt", [(0, 0.1), (1, 0.02), (2, 0.005)])
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_density8_sweep_of_a_slab_between_quads(pkg, orc, hip, stencil, dt, offset):
+    """u8 slabs at any address, odd ones among them."""
+    got, want = density_at_offset(pkg, orc, hip, stencil, dt, np.uint8, offset)
+    assert np.array_equal(got, want)
