@@ -351,9 +351,11 @@ __global__ void fill_i32_kernel(int32_t *p, int64_t n, int32_t v) {
 
 // Block ids as keys, at most `most` (particles far outside the domain), and
 // *ungrouped set to 1 when some particle's block precedes the previous
-// particle's in Morton order or lies past 1,023 on an axis: otherwise
-// (Morton-sorted input) each block's particles already form one run in input
-// order, which is the order the stable bucket sort gives within a block.
+// particle's in Morton order, or lies past 1,023 on an axis or past the last
+// block along x or y (its id is then that of a block of the next row, which has
+// a run of its own): otherwise (Morton-sorted input) each block's particles
+// already form one run in input order, which is the order the stable bucket sort
+// gives within a block.
 __global__ void bucket_keys_grouped_kernel(const float *__restrict__ pos, int64_t n, int32_t nx, int32_t ny,
                                            uint32_t most, uint32_t *__restrict__ keys, uint32_t *__restrict__ idx,
                                            int32_t *__restrict__ ungrouped) {
@@ -362,9 +364,10 @@ __global__ void bucket_keys_grouped_kernel(const float *__restrict__ pos, int64_
     };
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         const uint32_t x = trunc_index(pos[3 * i]), y = trunc_index(pos[3 * i + 1]), z = trunc_index(pos[3 * i + 2]);
-        keys[i] = min((x >> 4) + (y >> 4) * (uint32_t)nx + (z >> 4) * (uint32_t)nx * (uint32_t)ny, most);
+        const uint64_t id = (x >> 4) + (uint64_t)nx * ((y >> 4) + (uint64_t)ny * (z >> 4));
+        keys[i] = (uint32_t)min(id, (uint64_t)most);
         idx[i] = (uint32_t)i;
-        bool down = ((x | y | z) >> 14) != 0;
+        bool down = ((x | y | z) >> 14) != 0 || (x >> 4) >= (uint32_t)nx || (y >> 4) >= (uint32_t)ny;
         if (i > 0) {
             const uint32_t px = trunc_index(pos[3 * i - 3]), py = trunc_index(pos[3 * i - 2]),
                            pz = trunc_index(pos[3 * i - 1]);

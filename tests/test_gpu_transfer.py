@@ -565,3 +565,31 @@ def test_density_splat_into_a_slab_between_words(pkg, hip, r_scan):
     assert np.array_equal(odd.layout.to_host().b2s, b2s)
     assert np.array_equal(got, want)
     assert host[0] == 0x1234 and np.all(host[1 + want.size :] == 0x1234)
+
+
+@pytest.mark.parametrize("s", [(48, 32, 48), (64, 64, 32)])
+def test_particles_to_grid_mac_sorted_with_strays(pkg, hip, s):
+    """Morton-sorted particles, some on or past the upper x and y bounds, whose
+    block ids are those of other blocks: these keep the values of a call without
+    the strays (no cell is in a stray's reach) up to roundings of partial sums
+    of one sign."""
+    rng = np.random.default_rng(s[1])
+    pos = rng.uniform(0.0, np.array(s) - 3.0, (3000, 3)).astype(np.float32)
+    stray = rng.uniform(0.0, np.array(s) - 3.0, (40, 3)).astype(np.float32)
+    stray[:20, 0] = s[0] + np.float32([2.5, 7.0, 40.0, 900.0])[np.arange(20) % 4]
+    stray[20:, 1] = s[1] + np.float32([2.5, 7.0, 40.0, 900.0])[np.arange(20) % 4]
+    both = np.concatenate([pos, stray])
+    vel = rng.uniform(1.0, 2.0, both.shape).astype(np.float32)
+    mass = rng.uniform(0.5, 2.0, both.shape[0]).astype(np.float32)
+    order = morton_order(both)
+    macs = []
+    for rows in (order, order[order < pos.shape[0]]):
+        mac = T.MacGrid(*s, capacity_blocks=64, lib=hip)
+        T.particles_to_grid(mac, both[rows], vel[rows], mass[rows], 2.0)
+        macs.append(mac)
+    for a in range(3):
+        for gs, gp in zip(macs[0].mass[a : a + 1] + macs[0].velocity[a : a + 1],
+                          macs[1].mass[a : a + 1] + macs[1].velocity[a : a + 1]):
+            got, want = gs.to_host().to_dense(), gp.to_host().to_dense()
+            np.testing.assert_allclose(got, want, rtol=16 * 2.0 ** -24, atol=0)
+            assert (want > 0).any()
