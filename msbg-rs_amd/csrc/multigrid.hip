@@ -45,7 +45,6 @@
 
 #include "coarse_cg.hpp"
 #include "poisson.hpp"
-#include "primitives.hpp"
 
 namespace msbg {
 namespace mg {
@@ -73,7 +72,7 @@ struct Level {
 struct Hierarchy {
     std::vector<Level> lv;    // lv[k] is level k + 1
     int32_t *nb27 = nullptr;  // [n_active][27]: listed index of block k's neighbour (dx, dy, dz), -1 / -2
-    int32_t *slot27 = nullptr;  // its slot, -1 where not listed
+    int32_t *slot27 = nullptr;  // its slot, -1 where not listed (then scratch of the set-up)
 };
 
 namespace {
@@ -533,16 +532,12 @@ int ensure(msbg_poisson *p) {
     const i64 na = p->n_active;
     Hierarchy *H = new Hierarchy();
     p->mg = H;
-    // each listed block's 27 neighbours
-    int rc;
-    int32_t *index = (int32_t *)workspace(21, sizeof(int32_t) * (size_t)p->n_blocks, &rc);
-    if (rc) {
-        release(p);
-        return rc;
-    }
+    // each listed block's 27 neighbours, by way of every block's listed index
+    // (behind the slots: hierarchies share no scratch, so several can be built at once)
     const size_t n27 = (size_t)na * 27;
     hipError_t e = hipMalloc(&H->nb27, sizeof(int32_t) * n27);
-    if (e == hipSuccess) e = hipMalloc(&H->slot27, sizeof(int32_t) * n27);
+    if (e == hipSuccess) e = hipMalloc(&H->slot27, sizeof(int32_t) * (n27 + (size_t)p->n_blocks));
+    int32_t *index = H->slot27 + n27;
     if (e == hipSuccess) {
         const int nx = (int)p->nx, ny = (int)p->ny, nz = (int)p->nz;
         unlisted_kernel<<<grid_of(p->n_blocks), kT, 0, stream()>>>(index, p->n_blocks);

@@ -1079,16 +1079,12 @@ int build_flow(msbg_sweep_plan *p, const std::vector<int64_t> &order) {
             if (order[(size_t)(off + i)] == order[(size_t)(off + i - 1)]) return MSBG_OK;
         off += p->counts[c];
     }
-    // one allocation: ticket, done, dep; the plan index of each block id is scratch
+    // one allocation: ticket, done, dep, and the plan index of each block id, which
+    // is scratch (of the plan's own: several plans can be made at once)
     const size_t at_done = sizeof(unsigned long long), at_dep = at_done + sizeof(uint32_t) * (size_t)n;
     char *mem = nullptr;
-    MSBG_HIP(hipMalloc(&mem, at_dep + sizeof(int32_t) * 27 * (size_t)n));
-    int rc = MSBG_OK;
-    int32_t *index = (int32_t *)workspace(21, sizeof(int32_t) * (size_t)g->n_blocks, &rc);
-    if (rc) {
-        (void)hipFree(mem);
-        return rc;
-    }
+    MSBG_HIP(hipMalloc(&mem, at_dep + sizeof(int32_t) * (27 * (size_t)n + (size_t)g->n_blocks)));
+    int32_t *index = (int32_t *)(mem + at_dep) + 27 * n;
     hipError_t e = hipMemsetAsync(mem, 0, at_dep, stream());
     if (e == hipSuccess) e = hipMemsetAsync(index, 0xff, sizeof(int32_t) * (size_t)g->n_blocks, stream());
     if (e == hipSuccess) {

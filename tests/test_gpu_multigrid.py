@@ -352,3 +352,38 @@ def test_coarse_levels_of_one_to_four_rows_a_lane(pkg, orc, hip, s, seed, frac, 
     g, active, _, _ = band_problem(pkg, *s, seed, frac)
     assert lo <= len(active) <= hi
     test_one_cycle_equals_dense_arithmetic(pkg, orc, hip, s, seed, frac, 0, 1e-4, 2, False)
+
+
+def test_bands_and_plans_made_by_several_threads(pkg, hip):
+    """Multigrid hierarchies and sweep plans set up and run by four threads at
+    once (the C calls release the interpreter's lock) have the bits of those made
+    one after the other: none shares scratch with another.  (Direct launches: one
+    thread's graph capture does not stand another's set-up calls.)"""
+    import threading
+    shapes = [(48 + 32 * k, 40 + 16 * k, 64 + 48 * k) for k in range(4)]
+    problems = [band_problem(pkg, *s, 20 + k, 0.7) for k, s in enumerate(shapes)]
+
+    def run(k, out):
+        g, active, x, b = problems[k]
+        for _ in range(5):
+            layout, pb = setup(pkg, hip, g, active)
+            dx = pb.field(0, host=x.reshape(-1))
+            pb.solve(dx, hip.to_device(np.ascontiguousarray(b)), storage=1, multigrid=True, omega=1.0,
+                     sweeps_per_check=2, max_sweeps=12, tol=0.0, direct=True)
+            pkg.SweepPlan(layout, active).run_async(0, 0.1, 2, True)
+            hip.synchronize()
+            out[k].append((dx.get(), layout.to_host().slab.copy()))
+
+    alone, together = [[] for _ in shapes], [[] for _ in shapes]
+    for k in range(4):
+        run(k, alone)
+    threads = [threading.Thread(target=run, args=(k, together)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for a, t in zip(alone, together):
+        assert len(t) == 5
+        for (xa, sa), (xt, st) in zip(a, t):
+            assert np.array_equal(xa.view(np.uint32), xt.view(np.uint32))
+            assert np.array_equal(sa.view(np.uint32), st.view(np.uint32))
