@@ -64,6 +64,8 @@ struct msbg_grid {
     std::vector<int32_t> b2s_host;
     float *d_slab = nullptr;
     int32_t *d_b2s = nullptr;
+    void *d_windows = nullptr;  // splat windows of msbg_particles_to_grid_mac, where they are large
+    size_t window_bytes = 0;
 
     msbg::GridView view() const {
         msbg::GridView v;

@@ -217,6 +217,7 @@ int msbg_grid_free(msbg_grid *g) {
     if (!g) return MSBG_OK;
     if (g->d_slab) (void)hipFree(g->d_slab);
     if (g->d_b2s) (void)hipFree(g->d_b2s);
+    if (g->d_windows) (void)hipFree(g->d_windows);
     delete g;
     return MSBG_OK;
 }

@@ -403,6 +403,7 @@ constexpr int kSplatThreads = 1024;  // one group per CU holds the 128 KB window
 // blocks: 20 + 14 us a direction for splat and commit, 25 + 23 with two items
 // per CU).
 constexpr int kSplatMost = 16384, kSplatLeast = 256, kSplatItems = 256;
+constexpr size_t kSplatShared = (size_t)64 << 20;  // bytes of windows in the shared workspace
 constexpr int kSplatMaxCells = 8192;  // window cells of the two-channel kernels (m <= 2: 20^3)
 
 // One face direction of the MAC splat (p2g.rs:261-333): work-group i adds up
@@ -1193,6 +1194,37 @@ int active_list(const msbg_grid *g, const float *d_pos, int64_t n, float r_scan,
     return MSBG_OK;
 }
 
+// `bytes` of splat windows for `g`: small ones in the shared workspace, large
+// ones g's own, kept until it is freed.  (Given back and taken anew by every FLIP
+// step of 67 M particles, 53% of the steps waited 10 ms to 2 s for the driver to
+// hand out memory that was freed just before; kept, 32%, as in its other buffers.)
+int splat_windows(msbg_grid *g, size_t bytes, float2 **win) {
+    int rc = MSBG_OK;
+    if (bytes <= kSplatShared) {
+        *win = (float2 *)workspace(24, bytes, &rc);
+        return rc;
+    }
+    if (bytes > g->window_bytes) {
+        constexpr size_t kStep = (size_t)256 << 20;  // (a growing set takes new ones seldom)
+        bytes = (bytes + kStep - 1) / kStep * kStep;
+        if (g->d_windows) {
+            MSBG_HIP(hipStreamSynchronize(stream()));
+            (void)hipFree(g->d_windows);
+            g->d_windows = nullptr;
+            g->window_bytes = 0;
+        }
+        const hipError_t e = hipMalloc(&g->d_windows, bytes);
+        if (e != hipSuccess) {
+            g->d_windows = nullptr;
+            return e == hipErrorOutOfMemory ? fail(MSBG_ENOMEM, "particles_to_grid: out of device memory")
+                                            : hip_fail(e, "particles_to_grid windows");
+        }
+        g->window_bytes = bytes;
+    }
+    *win = (float2 *)g->d_windows;
+    return MSBG_OK;
+}
+
 }  // namespace msbg
 
 using namespace msbg;
@@ -1350,7 +1382,7 @@ int msbg_particles_to_grid_mac(msbg_grid *const *vel, msbg_grid *const *mass, co
     int chunk = std::max(1, std::min(n_items, (int)(((int64_t)1 << 31) / ((int64_t)sizeof(float2) * ns))));
     float2 *win = nullptr;
     for (;; chunk = (chunk + 1) / 2) {
-        win = (float2 *)workspace(24, sizeof(float2) * ns * (size_t)chunk, &rc);
+        rc = splat_windows(mass[0], sizeof(float2) * ns * (size_t)chunk, &win);
         if (!rc) break;
         if (rc != MSBG_ENOMEM || chunk <= 16) return rc;
         (void)hipGetLastError();

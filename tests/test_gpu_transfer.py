@@ -1,6 +1,7 @@
 """GPU parity of the transfers: the reference sampler, MAC P2G and the
 B-spline P2G / G2P against the oracle."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -593,3 +594,28 @@ def test_particles_to_grid_mac_sorted_with_strays(pkg, hip, s):
             got, want = gs.to_host().to_dense(), gp.to_host().to_dense()
             np.testing.assert_allclose(got, want, rtol=16 * 2.0 ** -24, atol=0)
             assert (want > 0).any()
+
+
+def test_particles_to_grid_mac_gives_its_windows_back(pkg, hip):
+    """A call whose windows take 2 GiB (as many as one pass holds): they go with
+    the grid that they were made for."""
+    def free_bytes():
+        hip.synchronize()
+        free, total = C.c_size_t(), C.c_size_t()
+        assert C.CDLL("libamdhip64.so").hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    nb, s = 33, (528, 528, 528)
+    b = np.arange(nb ** 3)
+    pos = (16.0 * np.stack([b % nb, (b // nb) % nb, b // nb ** 2], 1) + 8.0).astype(np.float32)
+    d = [hip.to_device(x) for x in (pos, np.ones(pos.shape, np.float32), np.ones(b.size, np.float32))]
+    before = free_bytes()
+    mac = T.MacGrid(*s, capacity_blocks=nb ** 3 + 8, lib=hip)
+    for _ in range(2):
+        T.particles_to_grid(mac, *d, 2.0)
+    del mac
+    for _ in range(100):  # the driver counts freed memory as free a while later
+        if before - free_bytes() < 2 ** 28:
+            break
+        time.sleep(0.05)
+    assert before - free_bytes() < 2 ** 28
