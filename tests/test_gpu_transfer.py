@@ -619,3 +619,19 @@ def test_particles_to_grid_mac_gives_its_windows_back(pkg, hip):
             break
         time.sleep(0.05)
     assert before - free_bytes() < 2 ** 28
+
+
+def test_particles_to_grid_mac_commits_nothing_of_a_cut_margin(pkg, hip):
+    """A domain of 40 cells in z: particles whose footprints lie in its last
+    block, which the bound cuts, and past the bound leave every mass and velocity
+    cell of all three directions at exactly 0."""
+    s, n = (32, 48, 40), 60
+    rng = np.random.default_rng(8)
+    pos = rng.uniform(3.0, 28.0, (n, 3)).astype(np.float32)
+    pos[:, 2] = np.float32([35.0, 38.5, 40.0, 40.5, 41.25, 42.0])[np.arange(n) % 6]
+    mac = T.MacGrid(*s, capacity_blocks=64, lib=hip)
+    assert T.particles_to_grid(mac, pos, np.ones((n, 3), np.float32), np.ones(n, np.float32), 2.0) > 0
+    for g in mac.mass + mac.velocity:
+        h = g.to_host()
+        active = np.nonzero(h.b2s >= 2)[0]
+        assert active.size and np.all(h.slab[h.b2s[active]] == 0.0)
