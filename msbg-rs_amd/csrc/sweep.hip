@@ -631,7 +631,7 @@ __global__ void sr_advance_kernel(uint32_t *ctr) {
 }
 
 // ---------------------------------------------------------------------------
-// Whole sweeps of a small band in one launch.  A colour pass over few blocks
+// Whole sweeps of a small band, one a launch.  A colour pass over few blocks
 // is a chain of latencies (launch, topology row, tile loads, update), and the
 // next colour's launch waits for its last work-group: 6.1 us a colour on a
 // 128^3 shell (8 x 35 blocks).  Here a work-group takes the next block of the
@@ -973,8 +973,9 @@ struct msbg_sweep_plan {
     uint32_t sr_seed = 0;        // Density8: stochastic-rounding seed
     uint32_t *d_sr_ctr = nullptr;  // Density8: sweeps done by this plan (device)
     // One-launch sweeps (sweep_flow_kernel): n = 0 when the plan has none
-    // (all-level plans, large bands, repeated block ids, misaligned u16 / u8 slabs).
+    // (all-level plans, bands past kFlowPairs, repeated block ids, misaligned u16 / u8 slabs).
     msbg::FlowArgs flow{nullptr, nullptr, nullptr, 0};
+    int64_t flow_pairs = 0;  // ordered pairs of neighbours among the blocks
     // All-level plans (msbg_sweep_plan_new_levels): g / coarse are levels 0
     // and 1, d_bids / d_topo / counts the level-0 blocks; the coarse blocks
     // are d_cbids (colour-major, then level, then Morton order) with 27-entry
@@ -1060,12 +1061,56 @@ int build_topology(const msbg_grid *g, const msbg_grid *coarse, const uint8_t *d
     return MSBG_OK;
 }
 
-// Bands of at most this many blocks sweep in one launch: a curvature and a
-// bi-Laplacian sweep of 280 / 608 / 1,112 / 1,976 / 4,688 blocks take 69 / 93 /
-// 104 / 125 / 199 us that way and 98 / 104 / 107 / 119 / 182 us as colour passes,
-// where each colour has enough blocks to fill the chip and a waiting group
-// would only hold a CU's lanes.
-constexpr int64_t kFlowMost = 1024;
+// Where one-launch sweeps pay: a group that waits holds a CU's lanes, and the
+// more neighbours the blocks have the more groups wait, so the line lies at a
+// number of ordered neighbour pairs.  us a sweep, mean curvature, one launch
+// against colour passes (a sweep a call; in brackets, in graphs of 5, which are
+// at 48 in graphs of 2):
+//   FP32 160^3 shell, 248 blocks, 2,160 pairs:      37 against 47 (41)
+//   FP32 192^3 shell, 360 blocks, 3,144 pairs:      42 against 47 (41)
+//   FP32 box of 320 blocks, 5,972 pairs:            45 against 49 (41)
+//   FP32 256^3 shell, 704 blocks, 6,672 pairs:      48 against 47 (42)
+//   FP32 box of 1,000 blocks, 20,952 pairs:         57 against 48 (43)
+//   cross-level, 290 blocks, 5,460 pairs:           43 against 48 (44)
+//   cross-level, 444 blocks, 8,322 pairs:           48 against 48 (45)
+//   cross-level, 984 blocks, 18,698 pairs:          57 against 50 (46)
+//   u16 box of 294 blocks, 5,482 pairs:             47 against 52 (47)
+//   u16, 603 of 1,000 blocks, 7,672 pairs:          51 against 53 (49)
+// Blocks of fewer colours make fewer passes and wait less often, both of which
+// the square of their number stands for (plate of 256 blocks, 4 colours, 1,860
+// pairs: 22 against 23 (20); of 1,024, 7,812 pairs: 39 against 25 (24)).
+constexpr int64_t kFlowPairs[2][3] = {{6500, 5000, 3000}, {8500, 8000, 5500}};  // [cross-level or 16- / 8-bit][1, 2 - 3, more sweeps]
+constexpr int64_t kFlowMost = 1024;  // blocks
+
+// Ordered pairs of neighbours among the plan's blocks.
+int64_t neighbour_pairs(const msbg_grid *g, const std::vector<int64_t> &order, int64_t n) {
+    std::vector<uint64_t> on((size_t)(g->n_blocks + 63) / 64, 0);
+    for (int64_t i = 0; i < n; ++i) on[(size_t)order[i] >> 6] |= (uint64_t)1 << (order[i] & 63);
+    int64_t pairs = 0;
+    for (int64_t i = 0; i < n; ++i) {
+        const int64_t b = order[i], x = b % g->nx, y = (b / g->nx) % g->ny, z = b / g->nxy;
+        for (int t = 14; t < 27; ++t) {  // the neighbours after it; the others count it
+            const int64_t qx = x + t % 3 - 1, qy = y + (t / 3) % 3 - 1, qz = z + t / 9 - 1;
+            if (qx < 0 || qx >= g->nx || qy < 0 || qy >= g->ny || qz >= g->nz) continue;
+            const int64_t q = qx + g->nx * (qy + g->ny * qz);
+            pairs += 2 * (int64_t)((on[(size_t)q >> 6] >> (q & 63)) & 1);
+        }
+    }
+    return pairs;
+}
+
+int64_t colours_of(const msbg_sweep_plan *p) {
+    return std::count_if(p->counts, p->counts + 8, [](int64_t c) { return c > 0; });
+}
+
+// Whether a call of `sweeps` sweeps of this plan goes by launches of whole sweeps.
+bool flow_pays(const msbg_sweep_plan *p, int sweeps) {
+    if (!p->flow.n) return false;
+    const int64_t colours = colours_of(p);
+    if (colours == 1) return p->n <= 32;  // one pass a sweep has nothing to wait for
+    const bool wide = p->coarse || p->slab16 || p->slab8;
+    return p->flow_pairs * 64 <= kFlowPairs[wide][sweeps > 3 ? 2 : sweeps > 1] * colours * colours;
+}
 
 // The neighbour table and counters of a plan's one-launch sweeps (`order`:
 // its blocks, colour-major).
@@ -1079,6 +1124,8 @@ int build_flow(msbg_sweep_plan *p, const std::vector<int64_t> &order) {
             if (order[(size_t)(off + i)] == order[(size_t)(off + i - 1)]) return MSBG_OK;
         off += p->counts[c];
     }
+    p->flow_pairs = neighbour_pairs(g, order, n);
+    if (p->flow_pairs > kFlowPairs[1][0]) return MSBG_OK;
     // one allocation: ticket, done, dep, and the plan index of each block id, which
     // is scratch (of the plan's own: several plans can be made at once)
     const size_t at_done = sizeof(unsigned long long), at_dep = at_done + sizeof(uint32_t) * (size_t)n;
@@ -1234,15 +1281,13 @@ int launch_flow(msbg_sweep_plan *p, hipStream_t s, TS *fslab, int stencil, float
     return launch_flow_st<MSBG_BILAPLACIAN, MULTI, TS>(p, s, fslab, dt, clamp01, sweeps);
 }
 
-// Work-groups of a one-launch sweep: a launch has fewer than 2^32 lanes along
-// an axis, and 2^20 groups are ~50 ms, beside which a launch costs nothing.
-constexpr int64_t kFlowGroups = (int64_t)1 << 20;
-static_assert(kFlowGroups * kFlowThreads < (int64_t)1 << 32 && kFlowMost <= kFlowGroups, "groups of one launch");
-
-// `iterations` sweeps as one launch (Density8: one a sweep, whose number keys
-// its rounding), or several when they take more than kFlowGroups groups.
+// `iterations` sweeps, one a launch, or several while all their groups are on the
+// chip at once, a group a CU.  (In longer launches the groups of later sweeps take
+// the lanes that earlier ones wait for: 125 blocks 36 us a sweep so, 43 in launches
+// of 20 sweeps; 956 scattered ones 42 and 63; 8 blocks 31 a sweep by itself, 27 in
+// launches of 20.  Density8: one a launch, whose number keys its rounding.)
 int launch_flow_sweeps(msbg_sweep_plan *p, hipStream_t s, int stencil, float dt, int iterations, int clamp01) {
-    const int64_t most = p->slab8 ? 1 : kFlowGroups / p->flow.n;
+    const int64_t most = p->slab8 ? 1 : std::max<int64_t>(1, 256 / p->flow.n);
     for (int64_t it = 0; it < iterations; it += most) {
         const unsigned sweeps = (unsigned)std::min<int64_t>(most, iterations - it);
         int rc;
@@ -1321,7 +1366,7 @@ int launch_iterations(msbg_sweep_plan *p, hipStream_t s, int stencil, float dt, 
     MSBG_CHECK(!(p->has_edge1 && stencil == MSBG_BILAPLACIAN), MSBG_EINVAL,
                "the radius-2 bi-Laplacian needs blocks of edge >= 2 (a level-4 halo would reach past its "
                "neighbour blocks)");
-    if (p->flow.n && !ev) return launch_flow_sweeps(p, s, stencil, dt, iterations, clamp01);
+    if (!ev && flow_pays(p, iterations)) return launch_flow_sweeps(p, s, stencil, dt, iterations, clamp01);
     for (int it = 0; it < iterations; ++it) {
         int rc = p->n_levels ? launch_sweep_levels(p, s, stencil, dt, clamp01, ev)
                  : p->coarse ? launch_sweep<true>(p, s, stencil, dt, clamp01, ev)
@@ -1604,8 +1649,11 @@ int msbg_sweep_plan_run_graph_async(msbg_sweep_plan *p, int stencil, float dt, i
     if (rc) return rc;
     MSBG_CHECK(iterations >= 0, MSBG_EINVAL, "negative iterations");
     if (iterations == 0 || p->n == 0) return MSBG_OK;
-    // one launch needs no graph
-    if (p->flow.n && !p->slab8) return launch_iterations(p, stream(), stencil, dt, iterations, clamp01);
+    // launches of whole sweeps need no graph, nor do up to 8 passes of a small band
+    // (a graph of them takes 50 us, 46 by themselves; one of one pass 19, 6 by itself)
+    if (!p->slab8 && !p->n_levels &&
+        (flow_pays(p, iterations) || (p->n <= kFlowMost && iterations * colours_of(p) <= 8)))
+        return launch_iterations(p, stream(), stencil, dt, iterations, clamp01);
     // a hit, else an empty entry, else the least recently used one
     msbg_sweep_plan::GraphEntry *hit = nullptr, *lru = nullptr;
     for (auto &e : p->graphs) {

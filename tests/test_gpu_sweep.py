@@ -449,18 +449,19 @@ def test_one_launch_sweeps_of_many_iterations(pkg, hip):
     assert np.array_equal(out[0], out[1])
 
 
-def test_one_launch_sweeps_past_a_launch(pkg, hip):
-    """4,100 sweeps of 1,024 blocks are 4.2 M blocks, more than the 2^32 lanes
-    of a launch hold: several launches in a row, with the bits of 4,100 rounds
-    of colour passes."""
-    g, active = shuffled_plan_problem(pkg, 1024, (208, 193, 181), 9)
+@pytest.mark.parametrize("n,sweeps", [(1024, 4100), (290, 4100), (32, 9), (33, 17), (255, 3), (256, 3)])
+def test_many_sweeps_in_one_call(pkg, hip, n, sweeps):
+    """Calls of many sweeps (4,100 of 1,024 blocks are more than the 2^32 lanes
+    that one launch holds), and of more than the sweeps that a launch of whole
+    sweeps takes (256 blocks in all), against single rounds of colour passes."""
+    g, active = shuffled_plan_problem(pkg, n, (208, 193, 181), 9)
     ga, gb = pkg.DeviceGrid.from_host(g, lib=hip), pkg.DeviceGrid.from_host(g, lib=hip)
     pa, pb = pkg.SweepPlan(ga, active), pkg.SweepPlan(gb, active)
-    pa.run_async(0, 0.1, 4100, True)
-    for _ in range(41):
-        pb.run_timed(0, 0.1, 100, True)
+    pa.run_async(0, 0.1, sweeps, True)
+    for at in range(0, sweeps, 100):
+        pb.run_timed(0, 0.1, min(100, sweeps - at), True)
     hip.synchronize()
-    assert_bitexact(ga.to_host().slab, gb.to_host().slab, "4100 sweeps")
+    assert_bitexact(ga.to_host().slab, gb.to_host().slab, "%d sweeps" % sweeps)
 
 
 def density_at_offset(pkg, orc, hip, stencil, dt, dtype, offset):
