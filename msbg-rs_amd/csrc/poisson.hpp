@@ -111,7 +111,7 @@ struct msbg_poisson {
     float *d_r = nullptr;       // FP32 residual, n_slots * 4096
     void *d_e = nullptr, *d_rt = nullptr;  // inner fields (2 or 4 B elements)
     int inner_bytes = 0;
-    bool e_zeroed = false;
+    int zeroed_for = 0;              // element bytes that the inner fields were last cleared for
     // learned correction scratch
     float *d_delta = nullptr, *d_xtry = nullptr;
     double *d_dots = nullptr;  // [2]: r . A delta, |A delta|^2

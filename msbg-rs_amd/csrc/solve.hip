@@ -783,14 +783,14 @@ int ensure_inner(msbg_poisson *p, int storage) {
         MSBG_HIP(hipMalloc(&p->d_e, n * eb));
         MSBG_HIP(hipMalloc(&p->d_rt, n * eb));
         p->inner_bytes = eb;
-        p->e_zeroed = false;
+        p->zeroed_for = 0;
     }
-    if (!p->e_zeroed) {
+    if (p->zeroed_for != eb) {  // fields of another width leave values in the slots that this one's must find zero
         const i64 words = (i64)(n * p->inner_bytes / 4);
         zero_u32_kernel<<<1024, 256, 0, stream()>>>((uint32_t *)p->d_e, words);
         zero_u32_kernel<<<1024, 256, 0, stream()>>>((uint32_t *)p->d_rt, words);
         MSBG_HIP(hipGetLastError());
-        p->e_zeroed = true;
+        p->zeroed_for = eb;
     }
     return MSBG_OK;
 }

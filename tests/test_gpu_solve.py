@@ -162,3 +162,22 @@ def test_shell_solve_to_1e6_vs_fp64(pkg, orc, hip, storage, refine):
     ref = dense_from_slabs(g.b2s, xd, s)[m]
     err = np.abs(dense_from_slabs(g.b2s, xg, s)[m] - ref).max() / np.abs(ref).max()
     assert err < 1e-5, err
+
+
+@pytest.mark.parametrize("order", [(0, 1, 2, 0), (0, 2, 1), (1, 0, 2)])
+@pytest.mark.parametrize("multigrid", [False, True])
+def test_refinement_in_several_storages_on_one_band(pkg, orc, hip, order, multigrid):
+    """Solves of one band with the inner fields in FP32, FP16 and BF16 in turn
+    have the bits of solves on bands of their own: the fields' unlisted slots are
+    zero whatever width the fields had before."""
+    g, active, x, b = band_problem(pkg, 64, 48, 80, 3, frac=0.7)
+    _, shared = setup(pkg, hip, g, active)
+    db = hip.to_device(np.ascontiguousarray(b))
+    kw = dict(omega=1.0, sweeps_per_check=2, max_sweeps=12, tol=0.0)
+    for storage in order:
+        _, alone = setup(pkg, hip, g, active)
+        got, want = shared.field(0, host=x.reshape(-1)), alone.field(0, host=x.reshape(-1))
+        a = shared.solve(got, db, storage=storage, refine=not multigrid, multigrid=multigrid, **kw)
+        w = alone.solve(want, db, storage=storage, refine=not multigrid, multigrid=multigrid, **kw)
+        assert a["sweeps"] == w["sweeps"] == 12
+        assert_bitexact(got.get(), want.get(), "storage %d" % storage)
