@@ -225,16 +225,26 @@ __global__ void g2p_flip_kernel(MacViews u, MacViews ut, const float *__restrict
 // and every particle then issues all of its 48 values, x pairs in one load
 // where a block holds both: three waits instead of nine.  A FLIP step's
 // particles come sorted along a Morton curve, so their blocks are few; a
-// work-group whose particles lie in more (any order is allowed), and particles
-// near the domain's bounds, go through sample_ip.  Both give its bits.
+// work-group whose particles lie in more than `most` (any order is allowed), and
+// particles near the domain's bounds, go through sample_ip.  Both give its bits.
 // 67 M sorted particles: 5.35 ms through sample_ip, 3.96 so (in step, a
 // direction at a time, 4.9; from cells staged in LDS, whose boxes are twice the
 // particles' own cells, 5.35).
-constexpr int kFlipThreads = 256, kFlipBlocks = 64;
+// Scattered particles share no lines, and then 48 loads at once only crowd the
+// caches, so the line lies at a mean number of particles a value block (all
+// sorted; sample_ip against this): 61 a block, 0.18 ms against 0.21 (1 M), 244,
+// 1.25 against 1.50 (8 M), 488, 1.85 against 1.97 (16 M), 977, 0.41 against
+// 0.39 (4 M), 1,950, 1.00 against 0.85 (8 M), 12,000, 1.40 against 0.99 (16 M).
+// 1 M unsorted ones in 64 blocks: 0.19 against 0.22, hence 27 blocks at most. A
+// few thousand are a chain of latencies, which this shortens when they lie close
+// (33 us against 25 in 8 blocks).
+constexpr int kFlipThreads = 256, kFlipBlocks = 27, kFlipBlocksFew = 8;
+constexpr int64_t kFlipPerBlock = 750, kFlipFew = 4096;
 __global__ __launch_bounds__(kFlipThreads) void g2p_flip_linear_kernel(MacViews u, MacViews ut,
                                                                        const float *__restrict__ pos,
                                                                        const float *__restrict__ u_old, int64_t n,
-                                                                       int bc, float alpha, float *__restrict__ out) {
+                                                                       int bc, float alpha, int most,
+                                                                       float *__restrict__ out) {
     __shared__ int s_box[6], s_slot[6][kFlipBlocks];
     const int t = threadIdx.x;
     const int64_t i = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * kFlipThreads + t;
@@ -274,7 +284,7 @@ __global__ __launch_bounds__(kFlipThreads) void g2p_flip_linear_kernel(MacViews 
     const int bx0 = s_box[0], by0 = s_box[1], bz0 = s_box[2];
     const bool any = s_box[3] >= bx0;
     const int64_t nx = any ? s_box[3] - bx0 + 1 : 0, ny = any ? s_box[4] - by0 + 1 : 0, nz = any ? s_box[5] - bz0 + 1 : 0;
-    const bool few = any && nx * ny * nz <= kFlipBlocks;  // uniform over the work-group
+    const bool few = any && nx * ny * nz <= most;  // uniform over the work-group
     const int nxy = (int)(nx * ny);
     if (few)
         for (int e = t; e < 6 * kFlipBlocks; e += kFlipThreads) {
@@ -1285,9 +1295,11 @@ int msbg_g2p_flip(msbg_grid *const *vel, msbg_grid *const *vel_tilde, const floa
         ut.v[a] = vel_tilde[a]->view();
     }
     const int64_t groups = (n + kFlipThreads - 1) / kFlipThreads;
-    if (interp == 0 && groups <= max_groups(kFlipThreads))  // a lane a particle; past 2^32 lanes stride
+    const bool dense = n >= kFlipPerBlock * (vel[0]->n_slots - 2);
+    // a lane a particle; past 2^32 lanes stride
+    if (interp == 0 && (dense || n <= kFlipFew) && groups <= max_groups(kFlipThreads))
         hipLaunchKernelGGL(g2p_flip_linear_kernel, dim3((unsigned)groups), dim3(kFlipThreads), 0, stream(), u, ut, d_pos,
-                           d_u_old, n, bc, alpha, d_out);
+                           d_u_old, n, bc, alpha, dense ? kFlipBlocks : kFlipBlocksFew, d_out);
     else if (interp == 0)
         hipLaunchKernelGGL(g2p_flip_kernel<0>, dim3(grid_for(n, 256)), dim3(256), 0, stream(), u, ut, d_pos, d_u_old,
                            n, bc, alpha, d_out);

@@ -635,3 +635,10 @@ def test_particles_to_grid_mac_commits_nothing_of_a_cut_margin(pkg, hip):
         h = g.to_host()
         active = np.nonzero(h.b2s >= 2)[0]
         assert active.size and np.all(h.slab[h.b2s[active]] == 0.0)
+
+
+@pytest.mark.parametrize("n,sort", [(255, True), (4096, True), (4096, False), (4097, True), (20249, True), (20250, True)])
+def test_g2p_flip_about_the_lines_of_its_kernels(pkg, orc, hip, n, sort):
+    """Up to 4,096 particles, and from 750 a block (27 blocks here) on, blocks'
+    slots are shared by a work-group; between them every sample is on its own."""
+    test_g2p_flip_matches_sample_twice_and_blend(pkg, orc, hip, 0, 0, n, sort)
