@@ -815,6 +815,11 @@ __global__ __launch_bounds__(256) void voxel_ranges_kernel(const uint32_t *__res
     for (int v = t; v < 4096; v += 256) s_cnt[v] = 0;
     __syncthreads();
     const uint32_t b0 = s_run[0], b1 = s_run[1];
+    uint4 *out = reinterpret_cast<uint4 *>(range + ((int64_t)slot << 12));
+    if (b0 == b1) {  // most active blocks of a sparse set: the footprints' margins
+        for (int v = t; v < 2048; v += 256) out[v] = make_uint4(b0, b0, b0, b0);
+        return;
+    }
     for (uint32_t i = b0 + t; i < b1; i += 256) atomicAdd(&s_cnt[keys[i] & 4095u], 1u);
     __syncthreads();
     uint32_t c[16], sum = 0;
@@ -832,11 +837,10 @@ __global__ __launch_bounds__(256) void voxel_ranges_kernel(const uint32_t *__res
     __syncthreads();
     uint32_t at = b0 + x - sum;
     for (int w = 0; w < t >> 6; ++w) at += s_sum[w];
-    uint4 *out = reinterpret_cast<uint4 *>(range + ((int64_t)slot << 12) + 16 * t);
 #pragma unroll
     for (int v = 0; v < 16; v += 2) {
         const uint32_t m = at + c[v], e = m + c[v + 1];
-        out[v / 2] = make_uint4(at, m, m, e);
+        out[8 * t + v / 2] = make_uint4(at, m, m, e);
         at = e;
     }
 }
