@@ -786,10 +786,11 @@ __global__ void block_keys_pack_kernel(const float *__restrict__ pos, const floa
 // The sorted particles [beg, end) of every voxel of the active blocks, indexed
 // by slot * 4096 + vid; an empty voxel's range is empty where its particles
 // would be, so neighbouring voxels' ranges join.  A work-group per block: its
-// run by search, a count per voxel in LDS, their scan.
+// run by search, a count per voxel in LDS, their scan.  *widest: the particles of
+// the fullest block.
 __global__ __launch_bounds__(256) void voxel_ranges_kernel(const uint32_t *__restrict__ keys, uint32_t n,
                                                            const int32_t *__restrict__ active, GridView g,
-                                                           uint2 *__restrict__ range) {
+                                                           uint2 *__restrict__ range, uint32_t *widest) {
     __shared__ uint32_t s_cnt[4096];
     __shared__ uint32_t s_run[2], s_sum[4];
     const uint32_t bid = (uint32_t)active[blockIdx.x];
@@ -820,6 +821,7 @@ __global__ __launch_bounds__(256) void voxel_ranges_kernel(const uint32_t *__res
         for (int v = t; v < 2048; v += 256) out[v] = make_uint4(b0, b0, b0, b0);
         return;
     }
+    if (widest && t == 0) atomicMax(widest, b1 - b0);
     for (uint32_t i = b0 + t; i < b1; i += 256) atomicAdd(&s_cnt[keys[i] & 4095u], 1u);
     __syncthreads();
     uint32_t c[16], sum = 0;
@@ -865,26 +867,34 @@ __device__ __forceinline__ void acc_add(Acc4 &a, float wxy, float pz, int cz, fl
 // dz = -1 plane), v (dz = 0) and v-1 (dz = +1), so each particle is read once
 // per column and every cell still receives its planes in increasing z.
 //
-// SPAN: cells of the column that a work-group takes.  The whole column (16) has
-// the least to read (18 planes for 16 cells); on few blocks, where a column's
-// chain of dependent reads is all the time, spans of 4 (6 planes).
+// A work-group takes the whole column, which has the least to read (18 planes
+// for 16 cells), or (split = 4) on few blocks, where a column's chain of dependent
+// reads is all the time, a span of 4 (6 planes); there too a quarter of the
+// work-groups take whole columns where no block holds more than `even` particles
+// (*widest), so that the columns are a full and even load.
 // Bound by its arithmetic and by lanes that wait for the fullest of their wave
 // (16.8 M particles in 9,000 blocks, quadratic: 1,240 us with 9 voxels a plane
 // to step through, most of them empty, 1,025 with joined rows; 1 M in 350
 // blocks, linear: 375 and 120).
-template <int ORDER, int SPAN>
+template <int ORDER>
 __global__ __launch_bounds__(256) void p2g_bspline_kernel(GridView mg, GridView v0, GridView v1, GridView v2,
                                                           const int32_t *__restrict__ active,
                                                           const uint32_t *__restrict__ flags,
                                                           const uint2 *__restrict__ range,
                                                           const float4 *__restrict__ pm,
-                                                          const float4 *__restrict__ pu) {
+                                                          const float4 *__restrict__ pu, int split,
+                                                          const uint32_t *__restrict__ widest, uint32_t even) {
     __shared__ int s_nb[27];
     // voxel ranges of the block's 18 x 18 plane window (the block's columns
     // and a 1-voxel ring), double-buffered: plane v + 1 loads during plane v
     __shared__ uint2 s_pl[2][18 * 18];
-    const int64_t bid = active[blockIdx.x / (16 / SPAN)];
-    const int lz0 = (int)(blockIdx.x % (16 / SPAN)) * SPAN;  // first cell of the span
+    // (the first quarter of the work-groups then: every fourth of them would all
+    // fall on two of the 8 XCDs)
+    const bool joined = even && *widest <= even;
+    if (joined && blockIdx.x >= gridDim.x / split) return;
+    const int64_t bid = active[joined ? blockIdx.x : blockIdx.x / split];
+    const int part = joined ? 0 : (int)(blockIdx.x % split);
+    const int span = joined ? 16 : 16 / split, lz0 = part * span;  // cells of the span, the first of them
     const int bx = (int)(bid % mg.nx), by = (int)((bid / mg.nx) % mg.ny), bz = (int)(bid / ((int64_t)mg.nx * mg.ny));
     if (threadIdx.x < 27) {
         const int t = threadIdx.x;
@@ -940,9 +950,9 @@ __global__ __launch_bounds__(256) void p2g_bspline_kernel(GridView mg, GridView 
     plane_ranges(cz0 - 1, nxt);
     put_plane(0, nxt);
     __syncthreads();
-    for (int lv = -1; lv <= SPAN; ++lv) {
+    for (int lv = -1; lv <= span; ++lv) {
         const int vz = cz0 + lv, cur = (lv + 1) & 1;
-        if (lv < SPAN) plane_ranges(vz + 1, nxt);  // in flight while this plane's particles are added
+        if (lv < span) plane_ranges(vz + 1, nxt);  // in flight while this plane's particles are added
         if (vz >= 0 && vz < mg.sz) {
             // This lane's 9 voxels are window voxels (ly + dy + 1, lx + dx + 1).
             // The three of a row are one run of the sorted particles, or two
@@ -987,11 +997,11 @@ __global__ __launch_bounds__(256) void p2g_bspline_kernel(GridView mg, GridView 
                 }
                 const float wxy = bspline_w<ORDER>(p.x, cx) * bspline_w<ORDER>(p.y, cy);
                 if (lv >= 1) acc_add<ORDER>(lo, wxy, p.z, cz0 + lv - 1, p.w, u);
-                if (lv >= 0 && lv <= SPAN - 1) acc_add<ORDER>(mid, wxy, p.z, cz0 + lv, p.w, u);
-                if (lv <= SPAN - 2) acc_add<ORDER>(hi, wxy, p.z, cz0 + lv + 1, p.w, u);
+                if (lv >= 0 && lv <= span - 1) acc_add<ORDER>(mid, wxy, p.z, cz0 + lv, p.w, u);
+                if (lv <= span - 2) acc_add<ORDER>(hi, wxy, p.z, cz0 + lv + 1, p.w, u);
             }
         }
-        if (lv < SPAN) put_plane(cur ^ 1, nxt);  // buffer cur ^ 1 was last read before the previous barrier
+        if (lv < span) put_plane(cur ^ 1, nxt);  // buffer cur ^ 1 was last read before the previous barrier
         __syncthreads();
         if (lv >= 1) store(lv - 1, lo);  // cell lv-1 has its planes lv-2, lv-1, lv
         lo = mid;
@@ -1501,28 +1511,31 @@ int msbg_p2g_bspline(int order, msbg_grid *mass, msbg_grid *const *vel, const fl
     hipLaunchKernelGGL(gather_records_kernel, dim3(grid_for(n, 256)), dim3(256), 0, stream(), rec, perm, n, pm, pu);
     // per-voxel ranges of the sorted particles, indexed like the mass slab; those
     // of blocks that are not active are neither written nor looked at
-    uint2 *range = (uint2 *)workspace(8, sizeof(uint2) * mass->n_slots * 4096, &rc);
+    const size_t n_range = (size_t)mass->n_slots * 4096;
+    uint2 *range = (uint2 *)workspace(8, sizeof(uint2) * n_range + sizeof(uint32_t), &rc);
     if (rc) return rc;
-    hipLaunchKernelGGL(voxel_ranges_kernel, dim3((unsigned)act.size()), dim3(256), 0, stream(), keys, (uint32_t)n, d_act,
-                       mass->view(), range);
-    MSBG_HIP(hipGetLastError());
     const unsigned na = (unsigned)act.size();
-    const auto spread = [&](auto kernel, int span) {
-        kernel<<<na * (16 / span), 256, 0, stream()>>>(mass->view(), vel[0]->view(), vel[1]->view(), vel[2]->view(),
-                                                       d_act, d_flags, range, pm, pu);
-    };
     // Up to 8 columns of a work-group a CU fit at once, and fewer leave it idle
     // (1 M particles, 350 blocks: 375 us whole, 141 in spans of 4, 164 of 2; 16.8 M,
     // 9,000 blocks: 1,265 whole, 1,334 in spans of 4; all before the rows joined).
-    const bool whole = na >= 2048;
-    if (order == 1 && whole)
-        spread(p2g_bspline_kernel<1, 16>, 16);
-    else if (order == 1)
-        spread(p2g_bspline_kernel<1, 4>, 4);
-    else if (whole)
-        spread(p2g_bspline_kernel<2, 16>, 16);
+    // Two columns a CU are load enough where the blocks are alike and full (calls
+    // of 4 M / 8 M particles in a box of 512 blocks: 726 / 1,190 us whole, 692 /
+    // 1,480 in spans; of 8 M in 768 uneven ones 8,750 and 4,660).
+    const unsigned split = na >= 2048 ? 1 : 4;
+    const uint32_t even = split > 1 && na >= 512 && n >= 10000 * (int64_t)na ? (uint32_t)(2 * n / na) : 0;
+    uint32_t *widest = even ? (uint32_t *)(range + n_range) : nullptr;
+    if (widest) hipLaunchKernelGGL(set_flag_kernel, dim3(1), dim3(1), 0, stream(), (int32_t *)widest, 0);
+    hipLaunchKernelGGL(voxel_ranges_kernel, dim3(na), dim3(256), 0, stream(), keys, (uint32_t)n, d_act, mass->view(),
+                       range, widest);
+    MSBG_HIP(hipGetLastError());
+    const auto spread = [&](auto kernel) {
+        kernel<<<na * split, 256, 0, stream()>>>(mass->view(), vel[0]->view(), vel[1]->view(), vel[2]->view(), d_act,
+                                                 d_flags, range, pm, pu, (int)split, widest, even);
+    };
+    if (order == 1)
+        spread(p2g_bspline_kernel<1>);
     else
-        spread(p2g_bspline_kernel<2, 4>, 4);
+        spread(p2g_bspline_kernel<2>);
     MSBG_HIP(hipGetLastError());
     MSBG_HIP(hipStreamSynchronize(stream()));
     return MSBG_OK;

@@ -642,3 +642,27 @@ def test_g2p_flip_about_the_lines_of_its_kernels(pkg, orc, hip, n, sort):
     """Up to 4,096 particles, and from 750 a block (27 blocks here) on, blocks'
     slots are shared by a work-group; between them every sample is on its own."""
     test_g2p_flip_matches_sample_twice_and_blend(pkg, orc, hip, 0, 0, n, sort)
+
+
+@pytest.mark.parametrize("order", [1, 2])
+def test_p2g_bspline_full_even_blocks(pkg, hip, order):
+    """512 blocks of some 10,900 particles each are taken by whole columns; with
+    one block of 30,000 far from them (more than twice the mean) by spans: the
+    512 have the same bits."""
+    s, n = (128, 128, 192), 5_600_000
+    rng = np.random.default_rng(order)
+    pos = rng.random((n, 3), np.float32) * np.float32(125.0) + np.float32(0.5)
+    vel, mass = rng.random((n, 3), np.float32), rng.random(n, np.float32)
+    far = np.float32([60.0, 60.0, 167.0]) + rng.random((30_000, 3), np.float32) * np.float32(8.0)
+    got = []
+    for extra in (False, True):
+        p = np.concatenate([pos, far]) if extra else pos
+        u = np.concatenate([vel, vel[: len(far)]]) if extra else vel
+        m = np.concatenate([mass, mass[: len(far)]]) if extra else mass
+        tg = T.TransferGrid(*s, capacity_blocks=8 * 8 * 12, lib=hip)
+        k = tg.p2g(order, p, u, m)
+        assert k >= 512 and (k == 512) == (not extra) and len(p) >= 10_000 * k
+        hosts = [g.to_host() for g in [tg.mass] + tg.velocity]
+        got.append([h.slab[h.b2s[:512]] for h in hosts])
+    for a, b in zip(*got):
+        assert_bitexact(a, b, "even blocks")
