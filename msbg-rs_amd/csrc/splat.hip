@@ -32,7 +32,10 @@ struct SplatParams {
 };
 
 constexpr int kMaxMargin = 6;   // window edge W <= 28: 88 KB of LDS
-constexpr int kSplatThreads = 512;
+// Lanes per item: windows of up to 26^3 cells (70 KB) lie two to a CU, a larger one
+// has it to itself (1 M particles in 512^3, r_scan = 6: 5.6 ms with 512 lanes, 3.9
+// with 1,024).
+constexpr int kSplatThreads = 512, kSplatThreadsWide = 1024, kSplatWide = 27;
 constexpr int kChunk = 256;     // particles staged per pass
 
 // A work item: particles p0 .. p1 - 1 (bucketed order) of occupied block blocks[k].
@@ -65,7 +68,8 @@ __device__ __forceinline__ void atomic_min_u16(uint16_t *p, uint32_t v) {
 }
 
 // LDS atomics bound it: ~270 cells a particle at r_scan = 4.
-__global__ __launch_bounds__(kSplatThreads) void density_splat_kernel(SplatParams P, const int32_t *__restrict__ b2s,
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void density_splat_kernel(SplatParams P, const int32_t *__restrict__ b2s,
                                                                       uint16_t *slab, const float *__restrict__ pos,
                                                                       const int32_t *__restrict__ blocks,
                                                                       const DItem *__restrict__ items) {
@@ -80,7 +84,7 @@ __global__ __launch_bounds__(kSplatThreads) void density_splat_kernel(SplatParam
     const int W = P.W, m = P.m;
     const int cells = W * W * W;
     constexpr uint32_t kFar = 0x7f800000u;  // +inf
-    for (int i = threadIdx.x; i < cells; i += kSplatThreads) st[i] = kFar;
+    for (int i = threadIdx.x; i < cells; i += THREADS) st[i] = kFar;
     const int b0x = bx * 16, b0y = by * 16, b0z = bz * 16, hi = 16 + m - 1;
     if (threadIdx.x < 27) {
         // region (rx, ry, rz): skipped when any voxel lies outside the domain
@@ -121,7 +125,7 @@ __global__ __launch_bounds__(kSplatThreads) void density_splat_kernel(SplatParam
         }
         __syncthreads();
         const int n = min(kChunk, item.p1 - c0), ey = s_ext[0], rows = ey * s_ext[1];
-        for (int i = threadIdx.x; i < n * rows; i += kSplatThreads) {
+        for (int i = threadIdx.x; i < n * rows; i += THREADS) {
             const int p = i / rows, rr = i - p * rows;
             const int cz = s_r[p][4] + rr / ey, cy = s_r[p][2] + rr % ey;
             if (cz > s_r[p][5] || cy > s_r[p][3]) continue;
@@ -151,7 +155,7 @@ __global__ __launch_bounds__(kSplatThreads) void density_splat_kernel(SplatParam
         const uint32_t v = st[row + cx];
         return v == kFar ? 0xffffu : (uint32_t)(int)roundf((__uint_as_float(v) * P.inv) * 65535.0f);
     };
-    for (int i = threadIdx.x; i < W * W * words; i += kSplatThreads) {
+    for (int i = threadIdx.x; i < W * W * words; i += THREADS) {
         const int wd = i % words, r = i / words, cy = r % W, cz = r / W, cx = 2 * wd - odd;
         const uint32_t lo = code(cx, r * W), hi16 = code(cx + 1, r * W);
         if ((lo & hi16) == 0xffffu) continue;
@@ -268,14 +272,16 @@ int msbg_density_splat(msbg_grid *g, uint16_t *d_slab16, int64_t slab_slots, con
     if (rc) return rc;
     MSBG_HIP(hipMemcpyAsync(d_items, order.data(), sizeof(DItem) * order.size(), hipMemcpyHostToDevice, s));
     const size_t lds = sizeof(uint32_t) * P.W * P.W * P.W;
+    const bool wide = P.W >= kSplatWide;
+    const auto kernel = wide ? density_splat_kernel<kSplatThreadsWide> : density_splat_kernel<kSplatThreads>;
+    const int threads = wide ? kSplatThreadsWide : kSplatThreads;
     if (lds > 65536)
-        MSBG_HIP(hipFuncSetAttribute((const void *)density_splat_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)lds));
+        MSBG_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     // (past 8.4 M items, which take a domain of 6 M occupied blocks, a second launch)
-    const int64_t n_items = (int64_t)order.size(), most = max_groups(kSplatThreads);
+    const int64_t n_items = (int64_t)order.size(), most = max_groups(threads);
     for (int64_t i = 0; i < n_items; i += most)
-        density_splat_kernel<<<(unsigned)std::min(most, n_items - i), kSplatThreads, lds, s>>>(
-            P, g->d_b2s, d_slab16, d_sorted, d_blocks, d_items + i);
+        kernel<<<(unsigned)std::min(most, n_items - i), threads, lds, s>>>(P, g->d_b2s, d_slab16, d_sorted, d_blocks,
+                                                                          d_items + i);
     MSBG_HIP(hipGetLastError());
     MSBG_HIP(hipStreamSynchronize(s));
     return MSBG_OK;
