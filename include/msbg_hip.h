@@ -126,8 +126,10 @@ typedef struct msbg_sweep_plan msbg_sweep_plan;
 int msbg_sweep_plan_new(msbg_grid *g, const int64_t *active, int64_t n, msbg_sweep_plan **out);
 int msbg_sweep_plan_free(msbg_sweep_plan *p);
 int msbg_sweep_plan_run_async(msbg_sweep_plan *p, int stencil, float dt, int iterations, int clamp01);
-/* The same passes replayed as one HIP graph, captured on first use of a
- * stencil / dt / iterations / clamp01 combination.  The plan caches the
+/* The same passes with as few launches from the host as they need: replayed
+ * as one HIP graph, captured on first use of a stencil / dt / iterations /
+ * clamp01 combination, or, on bands of up to 1,024 blocks where a launch holds
+ * whole sweeps or the passes are few, launched directly.  The plan caches the
  * graphs of its 4 most recently used combinations, so alternating stencils
  * replay without re-capture; an evicted graph is destroyed only after its
  * last launch has completed. */
@@ -250,8 +252,9 @@ int msbg_block_topology(const uint8_t *d_levels, int64_t nx, int64_t ny, int64_t
 /* morton3 -- multires/sort.rs:20-22 -- of each particle's voxel (truncated
  * position, as p2g.rs:153), low 30 bits: exact for voxel coordinates < 1024. */
 int msbg_morton_keys(const float *d_pos, int64_t n, uint32_t *d_keys);
-/* Stable LSD radix sort of (key, value) pairs by the low key_bits bits, in
- * place (8-bit digits; wave ballot ranking, no global atomics).  The
+/* Stable LSD radix sort of (key, value) pairs by the low key_bits bits,
+ * rounded up to whole bytes, in place (wave ballot ranking, no global
+ * atomics).  The
  * reference has no radix sort: it is the permutation std::stable_sort gives. */
 int msbg_radix_sort_pairs(uint32_t *d_keys, uint32_t *d_vals, int64_t n, int key_bits);
 /* Morton sort of particles: d_keys = sorted 30-bit keys, d_perm[i] = original
@@ -325,14 +328,15 @@ int msbg_g2p_flip(msbg_grid *const *vel, msbg_grid *const *vel_tilde, const floa
  * channels x, y, z over one domain; 0 < r_p <= 3.  The commit adds each margin
  * region over its own width (the semantics of the reference's naive oracle,
  * p2g.rs:445-502).  Sums within a staging cell are order-dependent in the last
- * bits, as in the reference (particles/sort.rs:234-237). */
+ * bits, as in the reference (particles/sort.rs:234-237).  Staging windows of
+ * more than 64 MiB (2 GiB at most) are kept by mass[0] until it is freed. */
 int msbg_particles_to_grid_mac(msbg_grid *const *vel, msbg_grid *const *mass, const float *d_pos, const float *d_vel,
                                const float *d_mass, int64_t n, float r_p, int64_t *n_active);
 /* Trilinear (order 1) or quadratic B-spline (order 2) P2G onto a cell-centred
  * grid (no reference counterpart): blocks under the particles' r_scan = 2
- * footprint are ensured and zeroed on all four grids; particles are Morton
- * sorted and every cell gathers its 27 neighbour voxels in a fixed order, so
- * the result is deterministic.  mass[cell] = sum w m, vel[a][cell] =
+ * footprint are ensured and zeroed on all four grids; particles are sorted by
+ * block and voxel and every cell gathers its 27 neighbour voxels in a fixed
+ * order, so the result is deterministic.  mass[cell] = sum w m, vel[a][cell] =
  * sum w m u_a / mass (0 where mass is 0).  d_mass may be NULL (m = 1).
  * Particles lie in [0, s) per axis, s <= 1024. */
 int msbg_p2g_bspline(int order, msbg_grid *mass, msbg_grid *const *vel, const float *d_pos, const float *d_vel,

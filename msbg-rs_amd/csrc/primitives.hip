@@ -235,7 +235,7 @@ int scan_exclusive_u32_with(const uint32_t *in, uint32_t *out, int64_t n, uint32
 // Pass = histogram (LDS atomics per tile, bin-major table), one exclusive scan
 // of the table (so entry (d, tile) is the first output slot of digit d from
 // that tile), then a stable scatter: inside a chunk a key's rank among equal
-// digits comes from 8 ballots (peer mask), across chunks and waves from LDS
+// digits comes from a ballot per bit (peer mask), across chunks and waves from LDS
 // counters, so equal keys keep their input order.
 // ---------------------------------------------------------------------------
 constexpr int kRsThreads = 256, kRsChunks = 16, kRsTile = kRsThreads * kRsChunks;

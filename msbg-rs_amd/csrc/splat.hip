@@ -13,7 +13,7 @@
 // nor the order of the items changes the result, and all of them run in one
 // launch: the 8 colour passes (block parity) that kept windows apart before
 // left ~120 work-groups a pass (512^3, 64 instances of 8,171 points: 8 x 165
-// us; one launch: see density_splat_kernel).
+// us, 226 in one launch).
 #include <algorithm>
 #include <cmath>
 #include <vector>

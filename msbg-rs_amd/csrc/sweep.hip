@@ -9,7 +9,8 @@
 // slab slot of each of its (2H+1)^3 neighbours (halo.rs:59-80), or the coarse
 // slot of a coarser neighbour (halo.rs:234-251).  A workgroup then reads one
 // table row instead of chasing bid -> slot -> level pointers, and the colour
-// passes of a sweep replay as one HIP graph.
+// passes of a sweep replay as one HIP graph.  Small bands sweep in one launch
+// (sweep_flow_kernel).
 //
 // The arithmetic repeats the reference's operation order exactly (fma where
 // it writes mul_add, no contraction elsewhere; the file is built with
@@ -1064,8 +1065,8 @@ int build_topology(const msbg_grid *g, const msbg_grid *coarse, const uint8_t *d
 // Where one-launch sweeps pay: a group that waits holds a CU's lanes, and the
 // more neighbours the blocks have the more groups wait, so the line lies at a
 // number of ordered neighbour pairs.  us a sweep, mean curvature, one launch
-// against colour passes (a sweep a call; in brackets, in graphs of 5, which are
-// at 48 in graphs of 2):
+// against colour passes in a call of one sweep and (in brackets) in a graph of
+// 5; a graph of 2 lies near the former:
 //   FP32 160^3 shell, 248 blocks, 2,160 pairs:      37 against 47 (41)
 //   FP32 192^3 shell, 360 blocks, 3,144 pairs:      42 against 47 (41)
 //   FP32 box of 320 blocks, 5,972 pairs:            45 against 49 (41)

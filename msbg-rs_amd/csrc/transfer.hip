@@ -8,9 +8,10 @@
 //    its (16+2m)^3 window in LDS (mass + momentum) and writes the window out,
 //    then every cell adds the windows that cover it, in a fixed order, and
 //    divides, u = P/M (mac.rs:106-132).
-//  * B-spline P2G / G2P (trilinear, quadratic): particles Morton-sorted by
-//    voxel; every cell gathers its 27 neighbour voxels in a fixed order, so
-//    the result is deterministic and needs neither atomics nor colouring.
+//  * B-spline P2G / G2P (trilinear, quadratic): particles sorted by block and
+//    voxel for the P2G, where every cell gathers its 27 neighbour voxels in a
+//    fixed order, so the result is deterministic and needs neither atomics nor
+//    colouring, and visited along a Morton curve for the G2P.
 #include <algorithm>
 #include <climits>
 #include <vector>
@@ -1482,7 +1483,7 @@ int msbg_p2g_bspline(int order, msbg_grid *mass, msbg_grid *const *vel, const fl
     MSBG_CHECK(n >= 0 && n < ((int64_t)1 << 31) && (n == 0 || (d_pos && d_vel)), MSBG_EINVAL,
                "p2g_bspline: bad particle arrays");
     MSBG_CHECK(mass->sx <= 1024 && mass->sy <= 1024 && mass->sz <= 1024, MSBG_EINVAL,
-               "p2g_bspline: the 30-bit Morton key needs a domain of at most 1024^3");
+               "p2g_bspline: the 30-bit block and voxel key needs a domain of at most 1024^3");
     // support cells floor(p)-1 .. floor(p)+1 lie in the footprint blocks of r_scan 2
     std::vector<int64_t> act;
     int32_t *d_act = nullptr;

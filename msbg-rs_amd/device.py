@@ -214,7 +214,8 @@ class SweepPlan:
         self.grid.lib.call("msbg_sweep_plan_run_async", self.h, int(stencil), dt, iterations, int(clamp01))
 
     def run_graph_async(self, stencil, dt, iterations, clamp01=False):
-        """The same passes replayed as one cached HIP graph."""
+        """The same passes replayed as one cached HIP graph (small bands: launched
+        directly, where that takes less)."""
         self.grid.lib.call("msbg_sweep_plan_run_graph_async", self.h, int(stencil), dt, iterations, int(clamp01))
 
     def run_timed(self, stencil, dt, iterations, clamp01=False):
